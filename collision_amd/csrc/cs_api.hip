@@ -219,6 +219,7 @@ void free_dev(DevState& S) {
   dfree(S.lvl_ptr); dfree(S.plog); dfree(S.counters); dfree(S.spread); dfree(S.scn); dfree(S.vscene);
   dfree(S.sslot); dfree(S.spre); dfree(S.slast);
   dfree(S.lvl_active);
+  dfree(S.bands.rec); dfree(S.bands.blob);
   S = DevState();
 }
 
@@ -701,6 +702,160 @@ int check_ready(cs_solver* h) {
   return CS_OK;
 }
 
+// The banded strain-limit plan, with more bands (smaller vertex windows) as
+// long as a window does not fit; false when none does (elements in random
+// order over a large mesh: every band then meets most vertices at once).
+bool strain_plan_for(int nv, int ne, const std::vector<int4>& ev, const std::vector<uint8_t>& ef,
+                     const std::vector<dvec4>& l0, int nsched, StrainPlan& plan) {
+  std::vector<uint8_t> rigid((size_t)ne);
+  for (int e = 0; e < ne; ++e) rigid[e] = (ef[e] & EF_RIGID) ? 1 : 0;
+  std::vector<int> lev;
+  const int* e4 = reinterpret_cast<const int*>(ev.data());
+  const int nl = strain_levels(nv, ne, e4, rigid.data(), lev);
+  for (int nb = strain_band_count(nsched, nl);; nb = std::min(2 * nb, STRAIN_MAX_BANDS)) {
+    if (strain_build_plan(nv, ne, e4, rigid.data(), reinterpret_cast<const double*>(l0.data()), lev,
+                          nl, nb, plan))
+      return true;
+    if (nb >= STRAIN_MAX_BANDS || nb >= nsched) break;
+  }
+  plan = StrainPlan();
+  return false;
+}
+
+// level schedule and slot records of k_strain_pipe
+struct PipeSchedule {
+  int n_levels = 0, delta = 1;
+  std::vector<int> lptr;
+  std::vector<StrainSlot> sslot;
+  std::vector<int> slast;
+};
+
+// levels (cs_schedule.hip), then slots in level order, element order within a
+// level (the elements of one level share no vertex, so any order is exact there)
+int build_pipe_schedule(cs_solver* h, int nv, int ne, const std::vector<int4>& ev,
+                        const std::vector<uint8_t>& ef, const std::vector<dvec4>& l0,
+                        PipeSchedule& Q) {
+  std::vector<int> level;
+  int nlev = 0;
+  build_strain_schedule(nv, ne, ev.data(), ef.data(), level, nlev, Q.delta);
+  Q.n_levels = nlev;
+  int nsched = 0;
+  for (int e = 0; e < ne; ++e)
+    if (level[e] >= 0) ++nsched;
+  std::vector<int>& lptr = Q.lptr;
+  lptr.assign((size_t)nlev + 1, 0);
+  std::vector<int> slot_of((size_t)std::max(ne, 1), -1);
+  const size_t nslot = (size_t)std::max(nsched, 1);
+  for (int e = 0; e < ne; ++e)
+    if (level[e] >= 0) lptr[level[e] + 1]++;
+  if (nlev >= (1 << 21)) return fail(h, CS_ERR_UNSUPPORTED, "strain schedule above 2^21 levels");
+  for (int l = 0; l < nlev; ++l) {
+    if (lptr[l + 1] > STRAIN_LEVEL_CAP)
+      return fail(h, CS_ERR_INTERNAL, "strain schedule level above its size cap");
+    lptr[l + 1] += lptr[l];
+  }
+  {
+    std::vector<int> fill(lptr.begin(), lptr.end() - 1);
+    for (int e = 0; e < ne; ++e)
+      if (level[e] >= 0) slot_of[e] = fill[level[e]]++;
+  }
+  std::vector<StrainSlot>& sslot = Q.sslot;
+  sslot.resize(nslot);
+  std::memset(sslot.data(), 0, sizeof(StrainSlot) * nslot);
+  {
+    // links: each visit of a vertex to its next visit, the last to the
+    // first (element order and level order agree on the elements of one
+    // vertex)
+    std::vector<int> first((size_t)nv, -1), last((size_t)nv, -1);
+    for (size_t s = 0; s < nslot; ++s)
+      for (int i = 0; i < 3; ++i) {
+        sslot[s].v[i] = -1;
+        sslot[s].ns[i] = -1;
+        sslot[s].nl[i] = -1;
+      }
+    for (int e = 0; e < ne; ++e) {
+      if (level[e] < 0) continue;
+      const int np = (ef[e] & EF_TRI) ? 3 : 2;
+      const int vv[3] = {ev[e].x, ev[e].y, ev[e].z};
+      const int s = slot_of[e];
+      StrainSlot& r = sslot[s];
+      r.level = level[e];
+      r.L0[0] = l0[e].x; r.L0[1] = l0[e].y; r.L0[2] = l0[e].z;
+      for (int i = 0; i < np; ++i) {
+        const int v = vv[i];
+        r.v[i] = v;
+        if (last[v] >= 0) {
+          StrainSlot& p = sslot[last[v] >> 2];
+          p.ns[last[v] & 3] = 4 * s + i;
+          p.nl[last[v] & 3] = (level[e] << 10) | (s - lptr[level[e]]);
+        } else {
+          first[v] = 4 * s + i;
+        }
+        last[v] = 4 * s + i;
+      }
+    }
+    Q.slast = last;
+    for (int v = 0; v < nv; ++v) {
+      if (last[v] < 0) continue;
+      StrainSlot& p = sslot[last[v] >> 2];
+      p.ns[last[v] & 3] = first[v];
+      const int fs = first[v] >> 2, fl = sslot[fs].level;
+      p.nl[last[v] & 3] = (fl << 10) | (fs - lptr[fl]);
+    }
+  }
+  return CS_OK;
+}
+
+template <typename T>
+hipError_t upload(T** p, const std::vector<T>& v) {
+  CS_HIP_RET(dalloc(p, v.size()));
+  if (v.empty()) return hipSuccess;
+  return hipMemcpy(*p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
+}
+
+// the plan's tables in one allocation and one copy (the records, most of it,
+// in another), followed by the tasks' own words
+hipError_t upload_plan(DevState& S, const StrainPlan& P) {
+  StrainBands& B = S.bands;
+  B.nband = P.nband;
+  B.n_levels = P.n_levels;
+  B.cap = P.cap;
+  std::vector<uint8_t> host;
+  std::vector<std::pair<void**, size_t>> at;
+  auto put = [&](auto** dst, const auto& v) {
+    const size_t off = (host.size() + 255) & ~(size_t)255, n = v.size() * sizeof(v[0]);
+    host.resize(off + n);
+    if (n) std::memcpy(host.data() + off, v.data(), n);
+    at.push_back({(void**)dst, off});
+  };
+  put(&B.step_ptr, P.step_ptr);
+  put(&B.step_level, P.step_level);
+  put(&B.grp_ptr, P.grp_ptr);
+  put(&B.grp, P.grp);
+  put(&B.imp, P.imp);
+  put(&B.exp_ptr, P.exp_ptr);
+  put(&B.exp, P.exp);
+  put(&B.lo_ptr, P.lo_ptr);
+  put(&B.lo, P.lo);
+  put(&B.up_ptr, P.up_ptr);
+  put(&B.up, P.up);
+  put(&B.slot, P.slot);
+  size_t total = host.size();
+  auto reserve = [&](auto** dst, size_t bytes) {
+    const size_t off = (total + 255) & ~(size_t)255;
+    total = off + bytes;
+    at.push_back({(void**)dst, off});
+  };
+  reserve(&B.pre, P.rec.size());
+  reserve(&B.prog, sizeof(int) * (size_t)SB_MAX_SWEEPS * P.nband * SB_PROG_STRIDE);
+  reserve(&B.stat, sizeof(int) * SB_STAT_INTS);
+  CS_HIP_RET(dalloc(&B.blob, total));
+  for (auto& a : at) *a.first = B.blob + a.second;
+  CS_HIP_RET(hipMemcpy(B.blob, host.data(), host.size(), hipMemcpyHostToDevice));
+  CS_HIP_RET(upload(&B.rec, P.rec));
+  return strain_bands_setup(S);
+}
+
 }  // namespace
 
 // checkpoint file: header, the parameters, then the arrays
@@ -949,72 +1104,19 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   for (int v = 0; v < nv; ++v)
     if (!used[v])
       return fail(h, CS_ERR_ARG, "every vertex must belong to a triangle or bond");
-  // strain-limit schedule: levels (cs_schedule.hip), then slots in level
-  // order, element order within a level (the elements of one level share no
-  // vertex, so any order is exact there)
-  std::vector<int> level;
-  int nlev = 0, sdelta = 1;
-  build_strain_schedule(nv, ne, ev.data(), ef.data(), level, nlev, sdelta);
+  // strain limiting: the banded plan, or the level schedule of the one-work-group
+  // sweep where no number of bands has vertex windows that fit LDS
+  StrainPlan plan;
+  PipeSchedule pipe;
   int nsched = 0;
-  for (int e = 0; e < ne; ++e)
-    if (level[e] >= 0) ++nsched;
-  std::vector<int> lptr((size_t)nlev + 1, 0), slot_of((size_t)std::max(ne, 1), -1);
-  const size_t nslot = (size_t)std::max(nsched, 1);
-  for (int e = 0; e < ne; ++e)
-    if (level[e] >= 0) lptr[level[e] + 1]++;
-  if (nlev >= (1 << 21)) return fail(h, CS_ERR_UNSUPPORTED, "strain schedule above 2^21 levels");
-  for (int l = 0; l < nlev; ++l) {
-    if (lptr[l + 1] > STRAIN_LEVEL_CAP)
-      return fail(h, CS_ERR_INTERNAL, "strain schedule level above its size cap");
-    lptr[l + 1] += lptr[l];
-  }
-  {
-    std::vector<int> fill(lptr.begin(), lptr.end() - 1);
-    for (int e = 0; e < ne; ++e)
-      if (level[e] >= 0) slot_of[e] = fill[level[e]]++;
-  }
-  std::vector<StrainSlot> sslot(nslot);
-  std::vector<int> slast;
-  std::memset(sslot.data(), 0, sizeof(StrainSlot) * nslot);
-  {
-    // links: each visit of a vertex to its next visit, the last to the
-    // first (element order and level order agree on the elements of one
-    // vertex)
-    std::vector<int> first((size_t)nv, -1), last((size_t)nv, -1);
-    for (size_t s = 0; s < nslot; ++s)
-      for (int i = 0; i < 3; ++i) {
-        sslot[s].v[i] = -1;
-        sslot[s].ns[i] = -1;
-        sslot[s].nl[i] = -1;
-      }
-    for (int e = 0; e < ne; ++e) {
-      if (level[e] < 0) continue;
-      const int np = (ef[e] & EF_TRI) ? 3 : 2;
-      const int vv[3] = {ev[e].x, ev[e].y, ev[e].z};
-      const int s = slot_of[e];
-      StrainSlot& r = sslot[s];
-      r.level = level[e];
-      r.L0[0] = l0[e].x; r.L0[1] = l0[e].y; r.L0[2] = l0[e].z;
-      for (int i = 0; i < np; ++i) {
-        const int v = vv[i];
-        r.v[i] = v;
-        if (last[v] >= 0) {
-          StrainSlot& p = sslot[last[v] >> 2];
-          p.ns[last[v] & 3] = 4 * s + i;
-          p.nl[last[v] & 3] = (level[e] << 10) | (s - lptr[level[e]]);
-        } else {
-          first[v] = 4 * s + i;
-        }
-        last[v] = 4 * s + i;
-      }
-    }
-    slast = last;
-    for (int v = 0; v < nv; ++v) {
-      if (last[v] < 0) continue;
-      StrainSlot& p = sslot[last[v] >> 2];
-      p.ns[last[v] & 3] = first[v];
-      const int fs = first[v] >> 2, fl = sslot[fs].level;
-      p.nl[last[v] & 3] = (fl << 10) | (fs - lptr[fl]);
+  for (int e = 0; e < ne; ++e) nsched += !(ef[e] & EF_RIGID);
+  if (nsched > 0) {
+    if (strain_plan_for(nv, ne, ev, ef, l0, nsched, plan)) {
+      if (plan.n_levels >= (1 << 21))
+        return fail(h, CS_ERR_UNSUPPORTED, "strain schedule above 2^21 levels");
+    } else {
+      const int rc = build_pipe_schedule(h, nv, ne, ev, ef, l0, pipe);
+      if (rc) return rc;
     }
   }
 
@@ -1095,12 +1197,19 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   HIPCHK(h, dalloc(&S.zkey, nv));
   HIPCHK(h, dalloc(&S.zval, nv)); HIPCHK(h, dalloc(&S.zval_tmp, nv));
   HIPCHK(h, dalloc(&S.zhead, nv)); HIPCHK(h, dalloc(&S.zend, nv));
-  S.n_levels = nlev;
   S.n_sched = nsched;
-  HIPCHK(h, dalloc(&S.lvl_ptr, nlev + 1));
-  S.strain_delta = sdelta;
-  HIPCHK(h, dalloc(&S.sslot, nslot));
-  HIPCHK(h, dalloc(&S.spre, nslot)); HIPCHK(h, dalloc(&S.slast, nv)); HIPCHK(h, dalloc(&S.lvl_active, std::max(nlev, 1)));
+  if (plan.nband > 0) {
+    HIPCHK(h, upload_plan(S, plan));
+  } else if (nsched > 0) {
+    S.n_levels = pipe.n_levels;
+    S.strain_delta = pipe.delta;
+    HIPCHK(h, upload(&S.lvl_ptr, pipe.lptr));
+    HIPCHK(h, upload(&S.sslot, pipe.sslot));
+    HIPCHK(h, upload(&S.slast, pipe.slast));
+    HIPCHK(h, dalloc(&S.spre, pipe.sslot.size()));
+    HIPCHK(h, hipMemset(S.spre, 0, sizeof(uint32_t) * pipe.sslot.size()));
+    HIPCHK(h, dalloc(&S.lvl_active, std::max(pipe.n_levels, 1)));
+  }
   S.plog_cap = 1 << 20;
   HIPCHK(h, dalloc(&S.plog, S.plog_cap));
   HIPCHK(h, dalloc(&S.counters, COUNTER_INTS));
@@ -1117,10 +1226,6 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   HIPCHK(h, hipMemcpy(S.eflags, ef.data(), ne, hipMemcpyHostToDevice));
   HIPCHK(h, hipMemcpy(S.len0, l0.data(), sizeof(dvec4) * ne, hipMemcpyHostToDevice));
   HIPCHK(h, hipMemcpy(S.fixed, fixed.data(), nv, hipMemcpyHostToDevice));
-  HIPCHK(h, hipMemcpy(S.lvl_ptr, lptr.data(), sizeof(int) * (nlev + 1), hipMemcpyHostToDevice));
-  HIPCHK(h, hipMemcpy(S.sslot, sslot.data(), sizeof(StrainSlot) * nslot, hipMemcpyHostToDevice));
-  HIPCHK(h, hipMemset(S.spre, 0, sizeof(uint32_t) * nslot));
-  HIPCHK(h, hipMemcpy(S.slast, slast.data(), sizeof(int32_t) * nv, hipMemcpyHostToDevice));
   HIPCHK(h, hipMemset(S.counters, 0, sizeof(int) * COUNTER_INTS));
   HIPCHK(h, hipMemset(S.has, 0, nv));
   HIPCHK(h, hipMemset(S.dirty_e, 0, ((size_t)ne + 3) & ~(size_t)3));

@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "cs_device.h"
+#include "cs_strain_plan.h"
 
 #define CS_HIP_RET(expr)                    \
   do {                                      \
@@ -129,6 +130,28 @@ constexpr int STRAIN_LEVEL_CAP = 1024;  // most slots in one level
 constexpr int TRAV_QCAP = 65536;        // split walks per round of the full traversal
 constexpr size_t TRAV_ITEM_BYTES = 48;
 
+// Device copy of the strain-limit plan (cs_strain_plan.h) and the state of its
+// tasks; nband == 0: the mesh has none (k_strain_pipe sweeps it).
+constexpr int SB_MAX_SWEEPS = 10;   // sweeps of one launch
+constexpr int SB_PROG_STRIDE = 16;  // ints between two tasks' progress words (64 B)
+constexpr int SB_STAT_INTS = 32;
+struct StrainBands {
+  int nband = 0, n_levels = 0, cap = 0;
+  uint8_t* blob = nullptr;  // the allocation of everything below but the records
+  StrainRec* rec = nullptr;
+  int32_t *step_ptr = nullptr, *step_level = nullptr;
+  int32_t* grp_ptr = nullptr;
+  StrainGroup* grp = nullptr;
+  StrainImport* imp = nullptr;
+  int32_t* exp_ptr = nullptr;
+  StrainExport* exp = nullptr;
+  int32_t *lo_ptr = nullptr, *lo = nullptr, *up_ptr = nullptr, *up = nullptr;
+  int32_t* slot = nullptr;  // element -> record (-1: rigid)
+  uint8_t* pre = nullptr;   // per record: the pre-check found an edge over the limit
+  int* prog = nullptr;      // per task: levels up to this one are done and exported
+  int* stat = nullptr;
+};
+
 // All device memory of one solver handle.
 struct DevState {
   int nv = 0, nt = 0, nb = 0, ne = 0;
@@ -235,6 +258,7 @@ struct DevState {
   uint8_t* lvl_active = nullptr;   // level holds an active element (pre-check)
   int n_levels = 0, n_sched = 0;
   int strain_delta = 1;            // 1 + widest level span of a vertex's visits
+  StrainBands bands;               // (the fields above stay empty when it has bands)
   // logs
   int4* plog = nullptr;
   int plog_cap = 0;
@@ -381,6 +405,10 @@ void launch_final_position(hipStream_t st, DevState& S, double dt);
 // appended (the caller reads and destroys them)
 hipError_t strain_limit(hipStream_t st, DevState& S, double dt, int max_sweeps,
                         std::vector<hipEvent_t>* marks);
+// cs_strain.hip: the same by bands (S.bands.nband > 0)
+hipError_t strain_bands_setup(const DevState& S);
+hipError_t strain_limit_bands(hipStream_t st, DevState& S, double dt, int max_sweeps,
+                              std::vector<hipEvent_t>* marks);
 // cs_schedule.hip (host)
 void build_strain_schedule(int nv, int ne, const int4* ev, const uint8_t* ef,
                            std::vector<int>& level, int& n_levels, int& delta);

@@ -1196,6 +1196,7 @@ hipError_t strain_limit(hipStream_t st, DevState& S, double dt, int max_sweeps,
                         std::vector<hipEvent_t>* marks) {
   const int n = S.n_sched;
   if (S.ne == 0 || n == 0 || max_sweeps <= 0) return hipSuccess;
+  if (S.bands.nband > 0) return strain_limit_bands(st, S, dt, max_sweeps, marks);
   // sweeps in flight: marks pending at one time cover K * delta - 1 levels
   const int kfit = std::max(1, SP_RING / std::max(1, S.strain_delta));
   for (int k0 = 0; k0 < max_sweeps;) {

@@ -53,63 +53,14 @@ void build_strain_schedule(int nv, int ne, const int4* ev, const uint8_t* ef,
   auto np_of = [&](int e) { return (ef[e] & EF_TRI) ? 3 : 2; };
   auto vtx = [&](int e, int k) { return k == 0 ? ev[e].x : (k == 1 ? ev[e].y : ev[e].z); };
   int nsched = 0;
-  std::vector<int> valence((size_t)nv, 0);
-  for (int e = 0; e < ne; ++e) {
-    if (ef[e] & EF_RIGID) continue;
-    ++nsched;
-    for (int k = 0; k < np_of(e); ++k) valence[vtx(e, k)]++;
-  }
-  if (nsched == 0) return;
-  const int maxval = *std::max_element(valence.begin(), valence.end());
-
-  // 1 + 2: earliest levels, relaxed so that each vertex's visits stay within W levels
-  std::vector<int> lv((size_t)nv), last((size_t)nv), lev((size_t)ne, 0);
-  std::vector<uint8_t> seen((size_t)nv);
-  bool converged = false;
-  for (int W = std::max(1, maxval - 1); W <= 64 && !converged; W *= 2) {
-    std::fill(lev.begin(), lev.end(), 0);
-    std::fill(last.begin(), last.end(), -1);
-    for (int pass = 0; pass < 16; ++pass) {
-      bool changed = false;
-      std::fill(lv.begin(), lv.end(), -1);
-      std::fill(seen.begin(), seen.end(), 0);
-      for (int e = 0; e < ne; ++e) {
-        if (ef[e] & EF_RIGID) continue;
-        int l = lev[e];
-        for (int k = 0; k < np_of(e); ++k) {
-          const int v = vtx(e, k);
-          l = std::max(l, lv[v] + 1);
-          if (!seen[v]) l = std::max(l, last[v] - W);
-        }
-        if (l != lev[e]) {
-          lev[e] = l;
-          changed = true;
-        }
-        for (int k = 0; k < np_of(e); ++k) {
-          lv[vtx(e, k)] = l;
-          seen[vtx(e, k)] = 1;
-        }
-      }
-      last = lv;
-      if (!changed) {
-        converged = true;
-        break;
-      }
-    }
-  }
-  if (!converged) {  // earliest levels
-    std::fill(lv.begin(), lv.end(), -1);
-    for (int e = 0; e < ne; ++e) {
-      if (ef[e] & EF_RIGID) continue;
-      int l = 0;
-      for (int k = 0; k < np_of(e); ++k) l = std::max(l, lv[vtx(e, k)] + 1);
-      lev[e] = l;
-      for (int k = 0; k < np_of(e); ++k) lv[vtx(e, k)] = l;
-    }
-  }
-  int L = 0;
   for (int e = 0; e < ne; ++e)
-    if (!(ef[e] & EF_RIGID)) L = std::max(L, lev[e] + 1);
+    if (!(ef[e] & EF_RIGID)) ++nsched;
+  if (nsched == 0) return;
+  // 1 + 2: earliest levels, relaxed so that each vertex's visits stay within W levels
+  std::vector<int> lev;
+  std::vector<uint8_t> rigid((size_t)std::max(ne, 1));
+  for (int e = 0; e < ne; ++e) rigid[e] = (ef[e] & EF_RIGID) ? 1 : 0;
+  const int L = strain_levels(nv, ne, reinterpret_cast<const int*>(ev), rigid.data(), lev);
 
   // 3: shift short components to the least loaded levels
   std::vector<int> uf((size_t)nv);
