@@ -64,6 +64,7 @@ struct NarrowParams {
   int ccd;        // 0 proximity, 1 CCD
   int mixed;      // FP32 screen of proximity sub-tests
   int mixed_stats;
+  int screen;     // CCD: run the certified coplanarity screen before isCoplanar
   int zone_mode;  // merge impact zones (s_detImpZone)
   int log_pairs;
   int pass_id;

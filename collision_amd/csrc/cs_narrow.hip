@@ -542,7 +542,7 @@ __device__ bool d_subtest(const Sub& S, bool is_pt, const NarrowParams& P, Contr
   // known: 1 = the certified screen already proved isCoplanar false, 0 = it
   // could not, -1 = not screened yet
   if (known == 1) return false;
-  if (known < 0 && P.mixed && d_coplanar_certainly_false(S, P.dt)) return false;
+  if (known < 0 && P.screen && d_coplanar_certainly_false(S, P.dt)) return false;
   if (!d_is_coplanar(S, P.dt, roots)) return false;
   *coplanar = true;
   for (int r = 0; r < 4; ++r) {
