@@ -219,7 +219,8 @@ void free_dev(DevState& S) {
   dfree(S.lvl_ptr); dfree(S.plog); dfree(S.counters); dfree(S.spread); dfree(S.scn); dfree(S.vscene);
   dfree(S.sslot); dfree(S.spre); dfree(S.slast);
   dfree(S.lvl_active);
-  dfree(S.bands.rec); dfree(S.bands.blob);
+  dfree(S.bands.rec); dfree(S.bands.blob); dfree(S.stage);
+  if (S.stage_host) (void)hipHostFree(S.stage_host);
   S = DevState();
 }
 
@@ -267,9 +268,18 @@ hipError_t alloc_sort_hist(DevState& S) {
   return dalloc(&S.sort_hist, words);
 }
 
-void to_dvec4(const double* src, int n, std::vector<dvec4>& out) {
-  out.resize((size_t)n);
-  for (int i = 0; i < n; ++i) out[i] = dvec4{src[3 * i], src[3 * i + 1], src[3 * i + 2], 0.0};
+// The staging memory of cs_set_state / cs_get_state, kept with the handle.
+// Small states go through pinned host memory that the kernels address
+// themselves (one launch, no copy commands); large ones through device memory
+// and one copy per array.
+hipError_t ensure_stage(DevState& S) {
+  if (S.stage || S.stage_host) return hipSuccess;
+  const size_t bytes = 97 * (size_t)S.nv;
+  if (bytes <= STAGE_HOST_MAX) return hipHostMalloc((void**)&S.stage_host, bytes);
+  uint8_t* p = nullptr;
+  CS_HIP_RET(dalloc(&p, bytes));
+  S.stage = reinterpret_cast<double*>(p);
+  return hipSuccess;
 }
 
 void from_dvec4(const std::vector<dvec4>& in, double* dst) {
@@ -1326,15 +1336,24 @@ int cs_set_state(cs_solver* h, const double* x, const double* vel, const uint8_t
   if (!h->assembled) return fail(h, CS_ERR_ARG, "cs_assemble has not been called");
   HIPCHK(h, hipSetDevice(h->P.device));
   DevState& S = h->S;
-  std::vector<dvec4> buf;
-  to_dvec4(x, S.nv, buf);
-  HIPCHK(h, hipMemcpy(S.x, buf.data(), sizeof(dvec4) * S.nv, hipMemcpyHostToDevice));
-  HIPCHK(h, hipMemcpy(S.x_old, buf.data(), sizeof(dvec4) * S.nv, hipMemcpyHostToDevice));
-  to_dvec4(vel, S.nv, buf);
-  HIPCHK(h, hipMemcpy(S.vel, buf.data(), sizeof(dvec4) * S.nv, hipMemcpyHostToDevice));
-  HIPCHK(h, hipMemset(S.av, 0, sizeof(dvec4) * S.nv));
-  if (has_collsn) HIPCHK(h, hipMemcpy(S.has, has_collsn, S.nv, hipMemcpyHostToDevice));
-  else HIPCHK(h, hipMemset(S.has, 0, S.nv));
+  HIPCHK(h, ensure_stage(S));
+  const size_t n3 = 3 * (size_t)S.nv;
+  if (S.stage_host) {  // read by the kernel from pinned host memory
+    HIPCHK(h, hipStreamSynchronize(h->st));
+    uint8_t* hc = reinterpret_cast<uint8_t*>(S.stage_host + 4 * n3);
+    std::memcpy(S.stage_host, x, sizeof(double) * n3);
+    std::memcpy(S.stage_host + n3, vel, sizeof(double) * n3);
+    if (has_collsn) std::memcpy(hc, has_collsn, (size_t)S.nv);
+    launch_unpack_state(h->st, S, S.stage_host, S.stage_host + n3, has_collsn ? hc : nullptr);
+  } else {
+    uint8_t* hc = reinterpret_cast<uint8_t*>(S.stage + 4 * n3);
+    HIPCHK(h, hipMemcpyAsync(S.stage, x, sizeof(double) * n3, hipMemcpyHostToDevice, h->st));
+    HIPCHK(h, hipMemcpyAsync(S.stage + n3, vel, sizeof(double) * n3, hipMemcpyHostToDevice, h->st));
+    if (has_collsn) HIPCHK(h, hipMemcpyAsync(hc, has_collsn, S.nv, hipMemcpyHostToDevice, h->st));
+    launch_unpack_state(h->st, S, S.stage, S.stage + n3, has_collsn ? hc : nullptr);
+    HIPCHK(h, hipStreamSynchronize(h->st));  // the caller may reuse its arrays
+  }
+  HIPCHK(h, hipGetLastError());
   if (S.nbody > 0) {  // initSurfaceState clears the RG accumulators (cdinit.cpp:192-197)
     HIPCHK(h, hipMemset(S.rg_imp, 0, sizeof(dvec4) * S.nbody));
     HIPCHK(h, hipMemset(S.rg_num, 0, sizeof(int32_t) * S.nbody));
@@ -1348,19 +1367,27 @@ int cs_get_state(cs_solver* h, double* x, double* vel, double* avg_vel, double* 
   if (!h) return CS_ERR_ARG;
   if (!h->assembled) return fail(h, CS_ERR_ARG, "cs_assemble has not been called");
   HIPCHK(h, hipSetDevice(h->P.device));
-  HIPCHK(h, hipStreamSynchronize(h->st));
   DevState& S = h->S;
-  std::vector<dvec4> buf((size_t)S.nv);
-  struct {
-    double* dst;
-    dvec4* src;
-  } items[4] = {{x, S.x}, {vel, S.vel}, {avg_vel, S.av}, {x_old, S.x_old}};
-  for (auto& it : items) {
-    if (!it.dst) continue;
-    HIPCHK(h, hipMemcpy(buf.data(), it.src, sizeof(dvec4) * S.nv, hipMemcpyDeviceToHost));
-    from_dvec4(buf, it.dst);
+  HIPCHK(h, ensure_stage(S));
+  const size_t n3 = 3 * (size_t)S.nv;
+  double* dst[4] = {x, vel, avg_vel, x_old};
+  const bool want[4] = {x != nullptr, vel != nullptr, avg_vel != nullptr, x_old != nullptr};
+  double* out = S.stage_host ? S.stage_host : S.stage;  // (the kernel writes pinned memory directly)
+  uint8_t* hc = reinterpret_cast<uint8_t*>(out + 4 * n3);
+  launch_pack_state(h->st, S, want, out, has_collsn ? hc : nullptr);
+  HIPCHK(h, hipGetLastError());
+  if (S.stage_host) HIPCHK(h, hipStreamSynchronize(h->st));
+  for (int k = 0; k < 4; ++k) {
+    if (!want[k]) continue;
+    if (S.stage_host) std::memcpy(dst[k], out, sizeof(double) * n3);
+    else HIPCHK(h, hipMemcpyAsync(dst[k], out, sizeof(double) * n3, hipMemcpyDeviceToHost, h->st));
+    out += n3;
   }
-  if (has_collsn) HIPCHK(h, hipMemcpy(has_collsn, S.has, S.nv, hipMemcpyDeviceToHost));
+  if (has_collsn) {
+    if (S.stage_host) std::memcpy(has_collsn, hc, (size_t)S.nv);
+    else HIPCHK(h, hipMemcpyAsync(has_collsn, hc, S.nv, hipMemcpyDeviceToHost, h->st));
+  }
+  if (!S.stage_host) HIPCHK(h, hipStreamSynchronize(h->st));
   return CS_OK;
 }
 

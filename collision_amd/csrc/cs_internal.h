@@ -128,6 +128,7 @@ struct alignas(16) StrainSlot {
 };
 static_assert(sizeof(StrainSlot) == 256, "StrainSlot layout");
 constexpr int STRAIN_LEVEL_CAP = 1024;  // most slots in one level
+constexpr size_t STAGE_HOST_MAX = 4u << 20;
 constexpr int TRAV_QCAP = 65536;        // split walks per round of the full traversal
 constexpr size_t TRAV_ITEM_BYTES = 48;
 
@@ -260,6 +261,10 @@ struct DevState {
   int n_levels = 0, n_sched = 0;
   int strain_delta = 1;            // 1 + widest level span of a vertex's visits
   StrainBands bands;               // (the fields above stay empty when it has bands)
+  // cs_set_state / cs_get_state: four [nv][3] arrays and nv bytes on their way
+  // in or out; the pinned copy only below STAGE_HOST_MAX
+  double* stage = nullptr;
+  double* stage_host = nullptr;
   // logs
   int4* plog = nullptr;
   int plog_cap = 0;
@@ -414,6 +419,11 @@ hipError_t strain_limit_bands(hipStream_t st, DevState& S, double dt, int max_sw
 void build_strain_schedule(int nv, int ne, const int4* ev, const uint8_t* ef,
                            std::vector<int>& level, int& n_levels, int& delta);
 void launch_final_velocity(hipStream_t st, DevState& S);
+// cs_set_state / cs_get_state: [n][3] arrays (device or pinned host memory) to
+// and from the state; want: x, vel, avgVel, x_old
+void launch_unpack_state(hipStream_t st, DevState& S, const double* x, const double* vel,
+                         const uint8_t* has);
+void launch_pack_state(hipStream_t st, DevState& S, const bool want[4], double* out, uint8_t* has);
 void launch_zone_labels(hipStream_t st, DevState& S, int32_t* out);
 
 // Work-group aggregated append: every lane of the block calls it; lanes with
