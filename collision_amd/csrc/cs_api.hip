@@ -200,12 +200,12 @@ void free_dev(DevState& S) {
   dfree(S.sort_hist); dfree(S.nodes); dfree(S.parent); dfree(S.nright); dfree(S.split_right);
   dfree(S.lpre); dfree(S.kleft); dfree(S.kright); dfree(S.kparent); dfree(S.krmin);
   dfree(S.krmax); dfree(S.pre);
-  dfree(S.rmin); dfree(S.rmax); dfree(S.arrive); dfree(S.pairs); dfree(S.hits);
-  dfree(S.top_start); dfree(S.scan_part); dfree(S.leaf_of);
+  dfree(S.tbox); dfree(S.top); dfree(S.pairs); dfree(S.hits);
+  dfree(S.scan_part); dfree(S.leaf_of);
   dfree(S.pairs_prev); dfree(S.qpairs); dfree(S.hits_prev); dfree(S.hp); dfree(S.hp_prev);
   dfree(S.dirty_e); dfree(S.dlist); dfree(S.pbox); dfree(S.pairs_seed);
   dfree(S.vlist); dfree(S.vadj_ptr); dfree(S.vadj);
-  dfree(S.dpre); dfree(S.rflag); dfree(S.rlist); dfree(S.tnext);
+  dfree(S.dpre); dfree(S.rflag); dfree(S.rlist);
   {
     uint8_t* tq = static_cast<uint8_t*>(S.tq);
     dfree(tq);
@@ -437,7 +437,8 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
   const int* vcount_prev = S.counters + CNT_VLIST + ((pass_id & 1) ^ 1);
   launch_zero_counters(h->st, S,
                        (1u << CNT_PAIRS) | (1u << CNT_HITS) | (1u << CNT_HIT_PAIRS) |
-                           (1u << CNT_HIT_SUB) | (1u << CNT_QPAIRS) | (1u << CNT_DIRTY) |
+                           (1u << CNT_HIT_SUB) | (1u << CNT_TMP) | (1u << CNT_QPAIRS) |
+                           (1u << CNT_DIRTY) | (3u << CNT_TSPLIT) |
                            (0x3fu << CNT_CAND64) | (1u << CNT_DRANGES) |
                            (1u << (CNT_VLIST + (pass_id & 1))));
   NarrowParams NP{};
@@ -474,12 +475,8 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
   int nhits = 0, nhp = 0;
   int narrow_n = 0;
   if (!incremental && !seeded) {
-    if (dual) {  // static boxes for this pass, swept boxes for the first CCD pass
-      launch_element_boxes(h->st, S, 0, P.dt, S.pbox);
-      launch_element_boxes(h->st, S, 1, P.dt, S.ebox);
-    } else {
-      launch_element_boxes(h->st, S, ccd, P.dt, S.ebox);
-    }
+    if (dual) launch_element_boxes(h->st, S, P.dt, S.pbox, S.ebox);  // swept: the first CCD pass's
+    else launch_element_boxes(h->st, S, P.dt, ccd ? nullptr : S.ebox, ccd ? S.ebox : nullptr);
     if (kind == CS_PASS_PROXIMITY) HIPCHK(h, build_bvh(h->st, S));
     HIPCHK(h, refit_bvh(h->st, S));
     for (;;) {  // traversal; re-run with a larger stream if it overflowed
@@ -499,6 +496,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
       HIPCHK(h, hipMemsetAsync(S.counters + CNT_PAIRS, 0, sizeof(int), h->st));
       HIPCHK(h, hipMemsetAsync(S.counters + CNT_CAND64, 0, 2 * sizeof(int), h->st));
       HIPCHK(h, hipMemsetAsync(S.counters + CNT_PCAND64, 0, 2 * sizeof(int), h->st));
+      HIPCHK(h, hipMemsetAsync(S.counters + CNT_TSPLIT, 0, 2 * sizeof(int), h->st));
     }
     cand = c64(h, CNT_CAND64);
     const int2* stream = S.pairs;
@@ -1148,7 +1146,7 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   HIPCHK(h, dalloc(&S.fixed, nv)); HIPCHK(h, dalloc(&S.has, nv)); HIPCHK(h, dalloc(&S.uf, nv));
   HIPCHK(h, dalloc(&S.ev, ne)); HIPCHK(h, dalloc(&S.eflags, ne)); HIPCHK(h, dalloc(&S.len0, ne));
   HIPCHK(h, dalloc(&S.ebox, ne));
-  HIPCHK(h, dalloc(&S.bounds, 6));
+  HIPCHK(h, dalloc(&S.bounds, BOUNDS_FLOATS));
   HIPCHK(h, dalloc(&S.mcode, ne)); HIPCHK(h, dalloc(&S.mid, ne));
   HIPCHK(h, dalloc(&S.mcode_tmp, ne)); HIPCHK(h, dalloc(&S.mid_tmp, ne));
   HIPCHK(h, dalloc(&S.nodes, 2 * ne - 1));
@@ -1159,8 +1157,7 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   HIPCHK(h, dalloc(&S.kparent, 2 * ne - 1)); HIPCHK(h, dalloc(&S.pre, 2 * ne - 1));
   HIPCHK(h, dalloc(&S.krmin, std::max(ne - 1, 1))); HIPCHK(h, dalloc(&S.krmax, std::max(ne - 1, 1)));
   HIPCHK(h, dalloc(&S.split_right, std::max(ne - 1, 1)));
-  HIPCHK(h, dalloc(&S.rmin, 2 * ne - 1)); HIPCHK(h, dalloc(&S.rmax, 2 * ne - 1));
-  HIPCHK(h, dalloc(&S.arrive, 2 * ne - 1)); HIPCHK(h, dalloc(&S.top_start, std::max(ne - 1, 1)));
+  HIPCHK(h, dalloc(&S.tbox, 6 * refit_tile_count(ne))); HIPCHK(h, dalloc(&S.top, std::max(ne - 1, 1)));
   S.pair_cap = (int)std::min<int64_t>(3ll * ne + 4096, INT32_MAX / 2);
   HIPCHK(h, dalloc(&S.pairs, S.pair_cap));
   HIPCHK(h, dalloc(&S.pairs_prev, S.pair_cap));
@@ -1196,7 +1193,6 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   HIPCHK(h, dalloc(&S.vadj_ptr, (size_t)nv + 1));
   HIPCHK(h, dalloc(&S.vadj, vadj.size()));
   HIPCHK(h, dalloc(&S.dpre, 2 * ne - 1));
-  HIPCHK(h, dalloc(&S.tnext, kNumXcd + 2));
   {
     uint8_t* tq = nullptr;
     HIPCHK(h, dalloc(&tq, 2 * TRAV_QCAP * TRAV_ITEM_BYTES));

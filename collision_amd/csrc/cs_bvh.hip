@@ -12,7 +12,7 @@
 //   * k_karras        : radix tree over the sorted codes (index tie-break);
 //     k_preorder / k_permute : the tree laid out in depth-first pre-order
 //     with escape links (ropes) for stackless traversal.
-//   * k_refit_tiles / k_refit_top : bottom-up FP32 boxes rounded outward,
+//   * k_refit_tiles / k_refit_top : FP32 boxes of all nodes, rounded outward,
 //     so every FP64 overlap is also an FP32 overlap.
 //   * k_traverse      : one lane per leaf in Morton order; it starts at its
 //     own leaf's rope, so it visits exactly the subtrees after itself in
@@ -27,86 +27,103 @@
 
 namespace cs {
 
-__global__ void k_element_boxes(const int4* __restrict__ ev, const dvec4* __restrict__ x,
-                                const dvec4* __restrict__ x_old, const dvec4* __restrict__ av,
-                                double dt, int moving, int ne, dbox* __restrict__ ebox) {
+// Element boxes (the reference's min/max_{static,moving}_coord,
+// dcollid.cpp:852-932), inflated by 1e-6: static boxes into sbox, swept boxes
+// into mbox, either may be null.
+__global__ void __launch_bounds__(256) k_element_boxes(const int4* __restrict__ ev,
+                                                       const dvec4* __restrict__ x,
+                                                       const dvec4* __restrict__ x_old,
+                                                       const dvec4* __restrict__ av, double dt, int ne,
+                                                       dbox* __restrict__ sbox,
+                                                       dbox* __restrict__ mbox) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= ne) return;
   const int4 t = ev[e];
   const int np = (t.z >= 0) ? 3 : 2;
   const int vid[3] = {t.x, t.y, t.z};
-  double lo[3] = {HUGE_VAL, HUGE_VAL, HUGE_VAL};
-  double hi[3] = {-HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
+  double lo[2][3], hi[2][3];  // static, swept
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      lo[k][d] = HUGE_VAL;
+      hi[k][d] = -HUGE_VAL;
+    }
   for (int i = 0; i < np; ++i) {
     const int v = vid[i];
-    if (moving) {
-      const dvec4 xo = x_old[v];
+    const dvec4 xo = x_old[v];
+    if (mbox) {
       const dvec4 a = av[v];
       const double o[3] = {xo.x, xo.y, xo.z};
       const double n[3] = {xo.x + a.x * dt, xo.y + a.y * dt, xo.z + a.z * dt};
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        hi[d] = smax(hi[d], o[d]);
-        hi[d] = smax(hi[d], n[d]);
-        lo[d] = smin(lo[d], o[d]);
-        lo[d] = smin(lo[d], n[d]);
+        hi[1][d] = smax(hi[1][d], o[d]);
+        hi[1][d] = smax(hi[1][d], n[d]);
+        lo[1][d] = smin(lo[1][d], o[d]);
+        lo[1][d] = smin(lo[1][d], n[d]);
       }
-    } else {
+    }
+    if (sbox) {
       // triangles use x_old, bonds use Coords (equal to x_old in the
       // proximity pass; dcollid.cpp:852-860, 892-910)
-      const dvec4 p = (np == 3) ? x_old[v] : x[v];
+      dvec4 p = xo;
+      if (np != 3) p = x[v];
       const double o[3] = {p.x, p.y, p.z};
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        hi[d] = smax(o[d], hi[d]);
-        lo[d] = smin(o[d], lo[d]);
+        hi[0][d] = smax(o[d], hi[0][d]);
+        lo[0][d] = smin(o[d], lo[0][d]);
       }
     }
   }
-  dbox b;
+  dbox* out[2] = {sbox, mbox};
 #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    b.lo[d] = lo[d] - CS_BOX_EPS;
-    b.hi[d] = hi[d] + CS_BOX_EPS;
+  for (int k = 0; k < 2; ++k) {
+    if (!out[k]) continue;
+    dbox b;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      b.lo[d] = lo[k][d] - CS_BOX_EPS;
+      b.hi[d] = hi[k][d] + CS_BOX_EPS;
+    }
+    out[k][e] = b;
   }
-  ebox[e] = b;
 }
 
-// min/max of box centres (FP32) -> bounds[0..5]; one atomic per block
-__global__ void k_bounds(const dbox* __restrict__ ebox, int ne, float* __restrict__ bounds) {
-  __shared__ float s[6][256];
-  float mn[3] = {3.4e38f, 3.4e38f, 3.4e38f}, mx[3] = {-3.4e38f, -3.4e38f, -3.4e38f};
-  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += gridDim.x * blockDim.x) {
+// min/max of the box centres (FP32): one row of six per work-group, reduced by
+// every work-group of k_morton (no atomics: 6,144 of them on six addresses
+// took 50-110 us)
+constexpr int BOUNDS_BLOCKS = 128, BOUNDS_THREADS = 512;
+__global__ void __launch_bounds__(BOUNDS_THREADS) k_bounds(const dbox* __restrict__ ebox, int ne,
+                                                           float* __restrict__ bounds) {
+  __shared__ float s[6][BOUNDS_THREADS / 64];
+  float m[6] = {3.4e38f, 3.4e38f, 3.4e38f, -3.4e38f, -3.4e38f, -3.4e38f};
+  for (int e = blockIdx.x * BOUNDS_THREADS + threadIdx.x; e < ne; e += gridDim.x * BOUNDS_THREADS) {
     const dbox b = ebox[e];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      float c = (float)(0.5 * (b.lo[d] + b.hi[d]));
-      mn[d] = fminf(mn[d], c);
-      mx[d] = fmaxf(mx[d], c);
+      const float c = (float)(0.5 * (b.lo[d] + b.hi[d]));
+      m[d] = fminf(m[d], c);
+      m[3 + d] = fmaxf(m[3 + d], c);
     }
   }
 #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    s[d][threadIdx.x] = mn[d];
-    s[3 + d][threadIdx.x] = mx[d];
-  }
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) {
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        s[d][threadIdx.x] = fminf(s[d][threadIdx.x], s[d][threadIdx.x + off]);
-        s[3 + d][threadIdx.x] = fmaxf(s[3 + d][threadIdx.x], s[3 + d][threadIdx.x + off]);
-      }
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
+  for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      atomicMin_float(&bounds[d], s[d][0]);
-      atomicMax_float(&bounds[3 + d], s[3 + d][0]);
+      m[d] = fminf(m[d], __shfl_xor(m[d], o));
+      m[3 + d] = fmaxf(m[3 + d], __shfl_xor(m[3 + d], o));
     }
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int d = 0; d < 6; ++d) s[d][threadIdx.x >> 6] = m[d];
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    const int d = threadIdx.x;
+    float r = s[d][0];
+    for (int w = 1; w < BOUNDS_THREADS / 64; ++w) r = d < 3 ? fminf(r, s[d][w]) : fmaxf(r, s[d][w]);
+    bounds[6 * blockIdx.x + d] = r;
   }
 }
 
@@ -118,23 +135,45 @@ __device__ inline uint32_t expand_bits10(uint32_t v) {
   return v;
 }
 
-__global__ void k_morton(const dbox* __restrict__ ebox, int ne, const float* __restrict__ bounds,
-                         uint32_t* __restrict__ codes, uint32_t* __restrict__ ids) {
+__global__ void __launch_bounds__(256) k_morton(const dbox* __restrict__ ebox, int ne,
+                                                const float* __restrict__ bounds, int nbounds,
+                                                uint32_t* __restrict__ codes,
+                                                uint32_t* __restrict__ ids) {
+  __shared__ float s[6][2];
+  if (threadIdx.x < BOUNDS_BLOCKS) {  // two wavefronts: the rows of k_bounds
+    const int r = min((int)threadIdx.x, nbounds - 1);
+    float m[6];
+#pragma unroll
+    for (int d = 0; d < 6; ++d) m[d] = bounds[6 * r + d];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        m[d] = fminf(m[d], __shfl_xor(m[d], o));
+        m[3 + d] = fmaxf(m[3 + d], __shfl_xor(m[3 + d], o));
+      }
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+      for (int d = 0; d < 6; ++d) s[d][threadIdx.x >> 6] = m[d];
+  }
+  __syncthreads();
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= ne) return;
   const dbox b = ebox[e];
   uint32_t q[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
+    const float lo = fminf(s[d][0], s[d][1]), hi = fmaxf(s[3 + d][0], s[3 + d][1]);
     float c = (float)(0.5 * (b.lo[d] + b.hi[d]));
-    float ext = bounds[3 + d] - bounds[d];
-    float u = ext > 0.f ? (c - bounds[d]) / ext : 0.5f;
+    float ext = hi - lo;
+    float u = ext > 0.f ? (c - lo) / ext : 0.5f;
     u = fminf(fmaxf(u, 0.f), 1.f);
     q[d] = (uint32_t)fminf(u * 1024.f, 1023.f);
   }
   codes[e] = (expand_bits10(q[0]) << 2) | (expand_bits10(q[1]) << 1) | expand_bits10(q[2]);
   ids[e] = (uint32_t)e;
 }
+static_assert(BOUNDS_BLOCKS == 128, "two wavefronts of k_morton");
 
 __device__ inline int lcp_delta(const uint32_t* __restrict__ codes, int n, int i, int j) {
   if (j < 0 || j >= n) return -1;
@@ -204,10 +243,9 @@ __global__ void k_preorder(int n, const int32_t* __restrict__ kleft,
 // scatter the construction tree into the pre-order arrays
 __global__ void k_permute(int n, const int32_t* __restrict__ pre, const int32_t* __restrict__ kright,
                           const int32_t* __restrict__ kparent, const int32_t* __restrict__ split_right,
-                          const int32_t* __restrict__ krmin, const int32_t* __restrict__ krmax,
+                          const int32_t* __restrict__ krmax,
                           const uint32_t* __restrict__ sorted_ids, bvh_node* __restrict__ nodes,
                           int32_t* __restrict__ parent, int32_t* __restrict__ nright,
-                          int32_t* __restrict__ rmin, int32_t* __restrict__ rmax,
                           int32_t* __restrict__ lpre, int32_t* __restrict__ enode) {
   const int x = blockIdx.x * blockDim.x + threadIdx.x;
   if (x >= 2 * n - 1) return;
@@ -220,116 +258,130 @@ __global__ void k_permute(int n, const int32_t* __restrict__ pre, const int32_t*
   if (internal) {
     nodes[p].left = -1;
     nright[p] = pre[kright[x]];
-    rmin[p] = krmin[x];
-    rmax[p] = krmax[x];
   } else {
     const int j = x - (n - 1);
     const int e = (int)sorted_ids[j];
     nodes[p].left = e;
     nright[p] = -1;
-    rmin[p] = j;
-    rmax[p] = j;
     lpre[j] = p;
     enode[e] = p;
   }
 }
 
-// Refit.  Every internal node covers a contiguous range [rmin, rmax] of
-// Morton-sorted leaves.  Nodes whose range lies inside one tile of
-// REFIT_TILE leaves are refit by that tile's work-group, bottom-up: the
-// second lane to arrive at a node (work-group-scope atomic counter) merges
-// both children.  The remaining "top" nodes are refit the same way by a
-// single work-group, starting from the top nodes whose children are all
-// tile-local.  No agent-scope fence is needed: every counter is touched by
-// one work-group only, and data crosses work-groups only at kernel
-// boundaries.  Leaf boxes are the FP64 boxes rounded outward to FP32.
-constexpr int REFIT_THREADS = 1024;
-constexpr int REFIT_TILE = 8192;
+// Refit.  Internal node i of the construction order covers the Morton-sorted
+// leaves [krmin, krmax], one end of which is i, so its box is a range minimum /
+// maximum over leaf boxes and needs no bottom-up chain (the atomic climb it
+// replaces took 150 us from 8,000 leaves on, all of it latency).  A work-group
+// holds REFIT_TILE leaf boxes (FP64 boxes rounded outward to FP32) and their
+// sparse table (level l: boxes of 2^l leaves) in LDS and answers every node
+// inside its tile with two reads; nodes that span tiles are listed and then
+// reduced by one wavefront each, over the leaves at both ends and the tile
+// boxes between.  Both kernels: 7,938 leaves 153 -> 18 us, 484,530 190 -> 50 us,
+// 2.2e6 400 -> under 110 us.
+constexpr int REFIT_SHIFT = 8, REFIT_TILE = 1 << REFIT_SHIFT;
 
-
-__device__ inline bool is_top(const int32_t* rmin, const int32_t* rmax, int node) {
-  return (rmin[node] / REFIT_TILE) != (rmax[node] / REFIT_TILE);
-}
-
-// the first child of an internal node is the next record (pre-order)
-__device__ inline void merge_children(bvh_node* nodes, const int32_t* __restrict__ nright,
-                                      int node) {
-  const bvh_node A = nodes[node + 1];
-  const bvh_node B = nodes[nright[node]];
+struct Box6 {
+  float v[6];  // lo, hi
+};
+__device__ inline Box6 box_empty() { return Box6{{3.4e38f, 3.4e38f, 3.4e38f, -3.4e38f, -3.4e38f, -3.4e38f}}; }
+__device__ inline void box_merge(Box6& a, const Box6& b) {
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    nodes[node].lo[d] = fminf(A.lo[d], B.lo[d]);
-    nodes[node].hi[d] = fmaxf(A.hi[d], B.hi[d]);
+    a.v[d] = fminf(a.v[d], b.v[d]);
+    a.v[3 + d] = fmaxf(a.v[3 + d], b.v[3 + d]);
   }
 }
-
-__device__ inline uint32_t wg_arrive(uint32_t* p) {
-  return __hip_atomic_fetch_add(p, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
-__global__ void __launch_bounds__(REFIT_THREADS)
-    k_refit_tiles(const dbox* __restrict__ ebox, const uint32_t* __restrict__ sorted_ids, int n,
-                  bvh_node* nodes, const int32_t* __restrict__ parent,
-                  const int32_t* __restrict__ nright, const int32_t* __restrict__ lpre,
-                  const int32_t* __restrict__ rmin, const int32_t* __restrict__ rmax,
-                  uint32_t* arrive) {
-  const int first = blockIdx.x * REFIT_TILE;
-  const int last = min(n, first + REFIT_TILE);
-  for (int j = first + threadIdx.x; j < last; j += REFIT_THREADS) {
-    const int e = (int)sorted_ids[j];
-    const dbox b = ebox[e];
-    const int leaf = lpre[j];
+__device__ inline void box_store(bvh_node* __restrict__ n, const Box6& b) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      nodes[leaf].lo[d] = f32_down(b.lo[d]);
-      nodes[leaf].hi[d] = f32_up(b.hi[d]);
-    }
-    if (n == 1) continue;
-    int node = parent[leaf];
-    while (node >= 0 && !is_top(rmin, rmax, node)) {
-      if (wg_arrive(&arrive[node]) == 0u) break;  // first arrival: sibling not done
-      merge_children(nodes, nright, node);
-      node = parent[node];
-    }
+  for (int d = 0; d < 3; ++d) {
+    n->lo[d] = b.v[d];
+    n->hi[d] = b.v[3 + d];
   }
 }
 
-// top nodes with no top child: start points of the single-work-group refit
-__global__ void k_mark_top(const bvh_node* __restrict__ nodes, const int32_t* __restrict__ nright,
-                           const int32_t* __restrict__ rmin, const int32_t* __restrict__ rmax,
-                           int n, int32_t* __restrict__ out, int* __restrict__ count) {
+__global__ void __launch_bounds__(REFIT_TILE)
+    k_refit_tiles(const dbox* __restrict__ ebox, const uint32_t* __restrict__ sorted_ids, int n,
+                  bvh_node* __restrict__ nodes, const int32_t* __restrict__ lpre,
+                  const int32_t* __restrict__ krmin, const int32_t* __restrict__ krmax,
+                  const int32_t* __restrict__ pre, float* __restrict__ tbox,
+                  int32_t* __restrict__ top, int* __restrict__ ntop) {
+  __shared__ float s[REFIT_SHIFT + 1][6][REFIT_TILE];
   __shared__ int s_cnt, s_base;
-  if (threadIdx.x == 0) s_cnt = 0;
+  const int t = threadIdx.x, first = blockIdx.x * REFIT_TILE, j = first + t;
+  Box6 b = box_empty();
+  if (j < n) {
+    const dbox d = ebox[sorted_ids[j]];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      b.v[c] = f32_down(d.lo[c]);
+      b.v[3 + c] = f32_up(d.hi[c]);
+    }
+    box_store(nodes + lpre[j], b);
+  }
+#pragma unroll
+  for (int c = 0; c < 6; ++c) s[0][c][t] = b.v[c];
+#pragma unroll
+  for (int l = 0; l < REFIT_SHIFT; ++l) {  // (past the tile's end: the boxes there are)
+    __syncthreads();
+    const int u = min(t + (1 << l), REFIT_TILE - 1);
+    Box6 o;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) o.v[c] = s[l][c][u];
+    box_merge(b, o);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) s[l + 1][c][t] = b.v[c];
+  }
   __syncthreads();
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  bool start = false;
-  if (i < 2 * n - 1 && nodes[i].left < 0 && is_top(rmin, rmax, i))
-    start = !is_top(rmin, rmax, i + 1) && !is_top(rmin, rmax, nright[i]);
-  int slot = -1;
-  if (start) slot = atomicAdd(&s_cnt, 1);
-  __syncthreads();
-  if (threadIdx.x == 0) s_base = s_cnt ? atomicAdd(count, s_cnt) : 0;
-  __syncthreads();
-  if (start) out[s_base + slot] = i;
+  if (t < 6) tbox[6 * (size_t)blockIdx.x + t] = s[REFIT_SHIFT][t][0];
+  bool span = false;
+  if (j < n - 1) {
+    const int a = krmin[j], z = krmax[j];
+    span = (a >> REFIT_SHIFT) != (z >> REFIT_SHIFT);
+    if (!span) {
+      const int l = 31 - __clz(z - a + 1), p = a - first, q = z - first + 1 - (1 << l);
+      Box6 r;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        r.v[c] = fminf(s[l][c][p], s[l][c][q]);
+        r.v[3 + c] = fmaxf(s[l][3 + c][p], s[l][3 + c][q]);
+      }
+      box_store(nodes + pre[j], r);
+    }
+  }
+  const int slot = block_append(span, ntop, &s_cnt, &s_base);
+  if (span) top[slot] = j;
 }
 
-__global__ void __launch_bounds__(1024)
-    k_refit_top(bvh_node* nodes, const int32_t* __restrict__ parent,
-                const int32_t* __restrict__ nright, const int32_t* __restrict__ rmin,
-                const int32_t* __restrict__ rmax, const int32_t* __restrict__ starts, int nstarts,
-                uint32_t* arrive) {
-  for (int k = threadIdx.x; k < nstarts; k += 1024) {
-    int node = starts[k];
-    merge_children(nodes, nright, node);
-    node = parent[node];
-    while (node >= 0) {
-      // arrivals needed = number of top children (the others are done)
-      const uint32_t need = (uint32_t)(is_top(rmin, rmax, node + 1) ? 1 : 0) +
-                            (uint32_t)(is_top(rmin, rmax, nright[node]) ? 1 : 0);
-      if (wg_arrive(&arrive[node]) + 1u < need) break;
-      merge_children(nodes, nright, node);
-      node = parent[node];
+__global__ void __launch_bounds__(256)
+    k_refit_top(const int32_t* __restrict__ top, const int* __restrict__ ntop,
+                const int32_t* __restrict__ krmin, const int32_t* __restrict__ krmax,
+                const int32_t* __restrict__ pre, const int32_t* __restrict__ lpre,
+                const float* __restrict__ tbox, bvh_node* __restrict__ nodes) {
+  const int lane = threadIdx.x & 63, nt = *ntop;
+  for (int k = blockIdx.x * 4 + (threadIdx.x >> 6); k < nt; k += gridDim.x * 4) {
+    const int i = top[k], a = krmin[i], z = krmax[i];
+    const int ta = a >> REFIT_SHIFT, tz = z >> REFIT_SHIFT;
+    Box6 b = box_empty();
+    auto leaf = [&](int j) {
+      const bvh_node m = nodes[lpre[j]];
+      box_merge(b, Box6{{m.lo[0], m.lo[1], m.lo[2], m.hi[0], m.hi[1], m.hi[2]}});
+    };
+    for (int j = a + lane; j < (ta + 1) << REFIT_SHIFT; j += 64) leaf(j);
+    for (int j = (tz << REFIT_SHIFT) + lane; j <= z; j += 64) leaf(j);
+    for (int q = ta + 1 + lane; q < tz; q += 64) {
+      Box6 m;
+#pragma unroll
+      for (int c = 0; c < 6; ++c) m.v[c] = tbox[6 * (size_t)q + c];
+      box_merge(b, m);
     }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      Box6 m;
+#pragma unroll
+      for (int c = 0; c < 6; ++c) m.v[c] = __shfl_xor(b.v[c], o);
+      box_merge(b, m);
+    }
+    if (lane == 0) box_store(nodes + pre[i], b);
   }
 }
 
@@ -386,34 +438,41 @@ __device__ inline bool pair_rejected(int4 ta, int4 tb, uint8_t fa) {
 __device__ inline int scene_of(const int4& t) { return t.w >> 16; }
 
 constexpr int TRAV_THREADS = 256;
-constexpr int TRAV_BUF = 8;  // pairs buffered per lane before an individual flush
+constexpr int TRAV_BUF = 8;  // pairs buffered per lane before the wavefront writes them
 
-// Persistent full-pass self query.  Lane = one leaf's stackless walk in
-// depth-first order after the leaf (every leaf j > i, each subtree once).
-// Walk lengths differ a lot within a wavefront, so lanes whose walk has
-// ended take the next leaves (a wavefront-aggregated atomic on a per-XCD
-// counter) while the others go on; each XCD starts on its own contiguous
-// eighth of the leaves (L2 locality) and then helps the others.  Pairs are
-// buffered per lane and written by the whole wavefront when a buffer fills.
+// Full-pass self query.  Lane = one leaf's stackless walk in depth-first order
+// after the leaf (every leaf j > i, each subtree once), or a part of it.  What
+// bounds it is the chain of dependent node loads of a walk, so walks are cut
+// short in two ways, both on one property: a rope walk started at any node x
+// visits x's subtree and then the following subtrees, i.e. exactly the nodes
+// from x on, so walks over [s0, s1) and [s1, end) find the pairs of the walk
+// over [s0, end), each once.
+//   * Below TRAV_LANES walks every leaf's walk is cut into 2^lsub sub-ranges
+//     from the start (a cut costs up to a tree depth of extra visits).
+//   * A walk that reaches TRAV_LONG steps hands the rest of its range to
+//     k_traverse_split, where TRAV_SPLIT lanes each walk one sub-range (and hand
+//     over once more).  Those of a static obstacle's big faces under a cloth
+//     visit tens of thousands of nodes.
+// Work-groups are dealt out by the hardware, each XCD one contiguous share of
+// the leaves.  Pairs are buffered per lane, written by the wavefront when a
+// buffer fills, and at the end with one atomic per work-group: counters in
+// memory that every wavefront added to (leaves taken, pairs, candidates) had
+// cost more than the walks.  Kernel time with the split rounds, per step,
+// against that form: 3,202 elements 120 -> 35 us, 7,938 168 -> 62 us, 138,000 780
+// -> 314 us, 484,530 in 64 scenes 1,020 -> 317 us, 2.2e6 3,450 -> 1,460 us.
+// TRAV_LONG 128 / 256 / 512: 138,000 elements under strings 314 / 490 / 570 us,
+// 130,050 of a crumpled cloth (long walks everywhere) 344 / 287 / 285 us, 2.2e6
+// 1,460 / 1,720 / 2,250 us.  TRAV_LANES 131,072 / 262,144: 18,000 elements 167 /
+// 139 us.
 // DUAL: the boxes are the swept boxes of the first CCD pass; the walk also
 // counts the static-box overlaps (the proximity pass's boxes, each inside
 // its element's swept box) among the pairs it rejects: a pair with a shared
 // vertex always overlaps (both static boxes hold that vertex), a pair on one
 // rigid surface is tested.  The kept pairs are tested by k_split_seed, so
 // one walk serves both passes.
-constexpr int PT_REFILL = 16;   // refill once this many lanes are idle
-constexpr int PT_STEPS = 16;    // walk steps between refill checks
-//
-// Long walks.  A few leaves have boxes that overlap a large part of the
-// mesh (a static obstacle's big faces under a cloth): their walks visit tens
-// of thousands of nodes one dependent load after another, and the kernel
-// waits for the longest.  A walk that reaches TRAV_LONG steps hands the rest
-// of its pre-order range [nd, end) to k_traverse_split, where TRAV_SPLIT
-// lanes each walk one sub-range.  A rope walk started at any node x visits
-// x's subtree and then the following subtrees, i.e. exactly the nodes from x
-// on, so walks over [s0, s1) and [s1, end) find the pairs of the walk over
-// [s0, end), each once.
-constexpr int TRAV_LONG = 512;
+constexpr int TRAV_STEPS = 16;    // walk steps between checks of the buffers
+constexpr int TRAV_LANES = 262144, TRAV_SUB_MAX = 6;
+constexpr int TRAV_LONG = 128;
 constexpr int TRAV_SPLIT = 64;
 
 // The rest of one walk: element e over the pre-order nodes [lo, hi), with the
@@ -424,260 +483,210 @@ struct __align__(16) TravItem {
 };
 static_assert(sizeof(TravItem) == TRAV_ITEM_BYTES, "TravItem layout");
 
-template <bool DUAL>
-__global__ void __launch_bounds__(TRAV_THREADS) k_traverse(const bvh_node* __restrict__ nodes,
-                                                           const int32_t* __restrict__ lpre,
-                                                           const dbox* __restrict__ ebox,
-                                                           const dbox* __restrict__ pbox,
-                                                           const int4* __restrict__ ev,
-                                                           const uint8_t* __restrict__ eflags,
-                                                           int n, int2* __restrict__ pairs, int cap,
-                                                           int* __restrict__ pair_count,
-                                                           unsigned long long* __restrict__ cand_count,
-                                                           unsigned long long* __restrict__ pcand_count,
-                                                           int* __restrict__ next, int scenes,
-                                                           TravItem* __restrict__ q, int qcap) {
-  __shared__ int2 buf[TRAV_BUF * TRAV_THREADS];
-  const int nnodes = 2 * n - 1;
-  int* qn = next + kNumXcd;  // items handed to the split kernel
-  const int t = threadIdx.x, lane = t & 63;
-  const uint64_t below = (1ull << lane) - 1ull;
-  // the eighth of the leaves this block's XCD starts on (blocks are dealt
-  // to the XCDs round-robin)
-  int chunk = (int)(blockIdx.x % kNumXcd), tried = 0;
-  auto chunk_end = [&](int c) { return (int)(((int64_t)n * (c + 1)) / kNumXcd); };
+struct TravArgs {
+  const bvh_node* nodes;
+  const int32_t* lpre;
+  const dbox *ebox, *pbox;
+  const int4* ev;
+  const uint8_t* eflags;
+  int n, scenes;
+  int2* pairs;
+  int cap;
+  int* pair_count;
+  unsigned long long *cand_count, *pcand_count;
+  TravItem* qout;  // where long walks go (null: they walk on)
+  int* qout_n;
+  int qcap;
+};
+
+struct Walk {
+  int e = 0, nd = -1, stop = 0, len = 0;  // element, current node (-1: none), end, steps
+  float lo[3] = {0.f, 0.f, 0.f}, hi[3] = {0.f, 0.f, 0.f};
+  dbox box{};
+  int4 t{};
+  uint8_t f = 0;
+};
+
+struct WalkOut {
   unsigned long long cand = 0, pcand = 0;
   int nbuf = 0;
-  int nd = -1;  // current node of this lane's walk, -1: idle
-  int e = 0;
-  int wlen = 0;  // steps of the current walk
-  float mlo[3] = {0.f, 0.f, 0.f}, mhi[3] = {0.f, 0.f, 0.f};
-  dbox mb{};
-  int4 mt{};
-  uint8_t mf = 0;
-  auto flush = [&]() {  // the wavefront's buffered pairs
-    int incl = nbuf;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(incl, o);
-      if (lane >= o) incl += y;
-    }
-    const int total = __shfl(incl, 63);
-    if (total == 0) return;
-    int base = 0;
-    if (lane == 63) base = atomicAdd(pair_count, total);
-    base = __shfl(base, 63) + incl - nbuf;
-    for (int k = 0; k < nbuf; ++k)
-      if (base + k < cap) pairs[base + k] = buf[k * TRAV_THREADS + t];
-    nbuf = 0;
-  };
-  bool more = n > 1;  // leaves left to take (uniform)
-  for (;;) {
-    // refill idle lanes
-    const uint64_t idle = __ballot(nd < 0);
-    if (more && (__popcll(idle) >= PT_REFILL || idle == ~0ull)) {
-      const int want = __popcll(idle);
-      int got = 0, first = 0;
-      while (got == 0 && tried < kNumXcd) {
-        int base = 0;
-        if (lane == 0) base = atomicAdd(&next[chunk], want);
-        base = __shfl(base, 0);
-        const int start = (int)(((int64_t)n * chunk) / kNumXcd) + base;
-        const int end = chunk_end(chunk);
-        if (start < end) {
-          got = min(want, end - start);
-          first = start;
-        } else {
-          chunk = (chunk + 1) % kNumXcd;
-          ++tried;
-        }
-      }
-      if (got == 0) more = false;
-      if (nd < 0) {
-        const int r = __popcll(idle & below);
-        if (r < got) {
-          const int i = first + r;
-          const bvh_node me = nodes[lpre[i]];
-          e = me.left;
-          mb = ebox[e];
-          mt = ev[e];
-          mf = eflags[e];
-#pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            mlo[d] = me.lo[d];
-            mhi[d] = me.hi[d];
-          }
-          nd = me.rope;
-          wlen = 0;
-        }
-      }
-    }
-    if (!more && __ballot(nd >= 0) == 0) break;
-    // walk
-    for (int step = 0; step < PT_STEPS && nd >= 0; ++step) {
-      if (wlen == TRAV_LONG) {  // hand the rest of this walk over
-        const int slot = atomicAdd(qn, 1);
-        if (slot < qcap) {
-          q[slot] = TravItem{e, nd, nnodes, 0, {mlo[0], mlo[1], mlo[2], 0.f}, {mhi[0], mhi[1], mhi[2], 0.f}};
-          nd = -1;
+};
+
+// The wavefront's walks to their ends.  buf: TRAV_BUF x TRAV_THREADS pairs.
+template <bool DUAL>
+__device__ __attribute__((always_inline)) inline void run_walks(const TravArgs& A, Walk& w, WalkOut& o,
+                                                                int2* __restrict__ buf) {
+  const int t = threadIdx.x, lane = t & 63;
+  while (__ballot(w.nd >= 0)) {
+    for (int step = 0; step < TRAV_STEPS && w.nd >= 0; ++step) {
+      if (w.len == TRAV_LONG && A.qout) {  // hand the rest of this walk over
+        const int slot = atomicAdd(A.qout_n, 1);
+        if (slot < A.qcap) {
+          A.qout[slot] = TravItem{w.e, w.nd, w.stop, 0, {w.lo[0], w.lo[1], w.lo[2], 0.f},
+                                  {w.hi[0], w.hi[1], w.hi[2], 0.f}};
+          w.nd = -1;
           break;
         }
         // (no room: this lane walks on)
       }
-      ++wlen;
-      const bvh_node node = nodes[nd];
-      if (!f32_overlap(node, mlo, mhi)) {
-        nd = node.rope;
-        continue;
-      }
-      if (node.left < 0) {  // internal: its first child is the next record
-        ++nd;
-        continue;
-      }
-      nd = node.rope;
-      const int e2 = node.left;
+      ++w.len;
+      const bvh_node node = A.nodes[w.nd];
+      const bool over = f32_overlap(node, w.lo, w.hi);
+      // an internal node's first child is the next record
+      w.nd = over && node.left < 0 ? w.nd + 1 : node.rope;
+      if (w.nd >= w.stop) w.nd = -1;
+      if (!over || node.left < 0) continue;
+      const int e = w.e, e2 = node.left;
       // box, topology and flags in one round trip (the exact overlap test
       // almost always passes where the rounded-out tree box did)
-      const dbox ob = ebox[e2];
-      const int4 ot = ev[e2];
-      const uint8_t of = eflags[e2];
+      const dbox ob = A.ebox[e2];
+      const int4 ot = A.ev[e2];
+      const uint8_t of = A.eflags[e2];
       // (the topology and flags are consumed here so that their loads are
       // issued with the box's, not after the overlap test)
       asm volatile("" ::"v"(ot.x), "v"(ot.y), "v"(ot.z), "v"(ot.w), "v"((int)of));
-      if (!f64_overlap(ob, mb)) continue;
-      if (scenes && scene_of(ot) != scene_of(mt)) continue;  // batched scenes never pair up
-      ++cand;
-      const int rk = (e > e2) ? pair_reject_kind(mt, ot, mf) : pair_reject_kind(ot, mt, of);
+      if (!f64_overlap(ob, w.box)) continue;
+      if (A.scenes && scene_of(ot) != scene_of(w.t)) continue;  // batched scenes never pair up
+      ++o.cand;
+      const int rk = (e > e2) ? pair_reject_kind(w.t, ot, w.f) : pair_reject_kind(ot, w.t, of);
       if (rk) {
         if constexpr (DUAL)
-          if (rk == REJ_SHARED || f64_overlap(pbox[e], pbox[e2])) ++pcand;
+          if (rk == REJ_SHARED || f64_overlap(A.pbox[e], A.pbox[e2])) ++o.pcand;
         continue;
       }
-      buf[nbuf * TRAV_THREADS + t] = make_int2(min(e, e2), max(e, e2));
-      if (++nbuf == TRAV_BUF) break;  // the buffer is written before the walk goes on
+      buf[o.nbuf * TRAV_THREADS + t] = make_int2(min(e, e2), max(e, e2));
+      if (++o.nbuf == TRAV_BUF) break;  // the buffer is written before the walk goes on
     }
-    if (__ballot(nbuf == TRAV_BUF)) flush();
-  }
-  flush();
-  unsigned long long c = cand;
+    if (__ballot(o.nbuf == TRAV_BUF)) {  // write the wavefront's buffered pairs
+      int incl = o.nbuf;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-  if (lane == 0 && c) atomicAdd(cand_count, c);
-  if constexpr (DUAL) {
-    unsigned long long pc = pcand;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) pc += __shfl_xor(pc, o);
-    if (lane == 0 && pc) atomicAdd(pcand_count, pc);
+      for (int q = 1; q < 64; q <<= 1) {
+        const int y = __shfl_up(incl, q);
+        if (lane >= q) incl += y;
+      }
+      int base = 0;
+      if (lane == 63) base = atomicAdd(A.pair_count, incl);
+      base = __shfl(base, 63) + incl - o.nbuf;
+      for (int k = 0; k < o.nbuf; ++k)
+        if (base + k < A.cap) A.pairs[base + k] = buf[k * TRAV_THREADS + t];
+      o.nbuf = 0;
+    }
   }
 }
 
-// Split walks: lane g walks sub-range g % TRAV_SPLIT of item g / TRAV_SPLIT.
-// A sub-range walk that again reaches TRAV_LONG steps is handed to the next
-// round (qout), if there is one.  Pairs are written with one atomic per
-// wavefront and step.
+// the rest of the pairs and the counts, one atomic each per work-group (all of
+// its threads call it)
 template <bool DUAL>
-__global__ void __launch_bounds__(256) k_traverse_split(const bvh_node* __restrict__ nodes,
-                                                        const dbox* __restrict__ ebox,
-                                                        const dbox* __restrict__ pbox,
-                                                        const int4* __restrict__ ev,
-                                                        const uint8_t* __restrict__ eflags,
-                                                        const TravItem* __restrict__ qin,
-                                                        const int* __restrict__ qin_n,
-                                                        TravItem* __restrict__ qout,
-                                                        int* __restrict__ qout_n, int qcap,
-                                                        int2* __restrict__ pairs, int cap,
-                                                        int* __restrict__ pair_count,
-                                                        unsigned long long* __restrict__ cand_count,
-                                                        unsigned long long* __restrict__ pcand_count,
-                                                        int scenes) {
-  const int lane = threadIdx.x & 63;
-  const uint64_t below = (1ull << lane) - 1ull;
-  const int total = min(*qin_n, qcap) * TRAV_SPLIT;
-  unsigned long long cand = 0, pcand = 0;
-  const int stride = gridDim.x * blockDim.x;
-  for (int g0 = blockIdx.x * blockDim.x; g0 < total; g0 += stride) {  // (uniform per block)
-    const int g = g0 + (int)threadIdx.x;
-    int nd = -1, s1 = 0, e = 0, wlen = 0;
-    float mlo[3] = {0.f, 0.f, 0.f}, mhi[3] = {0.f, 0.f, 0.f};
-    dbox mb{};
-    int4 mt{};
-    uint8_t mf = 0;
-    if (g < total) {
-      const TravItem it = qin[g / TRAV_SPLIT];
-      const int j = g % TRAV_SPLIT;
-      const int64_t span = (int64_t)it.hi - it.lo;
-      nd = it.lo + (int)(span * j / TRAV_SPLIT);
-      s1 = it.lo + (int)(span * (j + 1) / TRAV_SPLIT);
-      e = it.e;
+__device__ inline void finish_walks(const TravArgs& A, const WalkOut& o, const int2* __restrict__ buf) {
+  constexpr int W = TRAV_THREADS / 64;
+  __shared__ unsigned long long s_c[2][W];
+  __shared__ int s_n[W], s_base;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  unsigned long long c = o.cand, pc = o.pcand;
+  int incl = o.nbuf;
+#pragma unroll
+  for (int q = 1; q < 64; q <<= 1) {
+    const int y = __shfl_up(incl, q);
+    if (lane >= q) incl += y;
+    c += __shfl_xor(c, q);
+    if constexpr (DUAL) pc += __shfl_xor(pc, q);
+  }
+  if (lane == 63) {
+    s_c[0][w] = c;
+    s_c[1][w] = pc;
+    s_n[w] = incl;
+  }
+  __syncthreads();
+  int before = 0, total = 0;
+#pragma unroll
+  for (int q = 0; q < W; ++q) {
+    if (q < w) before += s_n[q];
+    total += s_n[q];
+  }
+  if (t < (DUAL ? 2 : 1)) {
+    unsigned long long v = 0;
+    for (int q = 0; q < W; ++q) v += s_c[t][q];
+    if (v) atomicAdd(t == 0 ? A.cand_count : A.pcand_count, v);
+  }
+  if (t == 64) s_base = total ? atomicAdd(A.pair_count, total) : 0;
+  __syncthreads();
+  const int base = s_base + before + incl - o.nbuf;
+  for (int k = 0; k < o.nbuf; ++k)
+    if (base + k < A.cap) A.pairs[base + k] = buf[k * TRAV_THREADS + t];
+}
+
+__device__ inline void walk_element(const TravArgs& A, Walk& w) {
+  w.box = A.ebox[w.e];
+  w.t = A.ev[w.e];
+  w.f = A.eflags[w.e];
+  w.len = 0;
+}
+
+template <bool DUAL>
+__global__ void __launch_bounds__(TRAV_THREADS) k_traverse(TravArgs A, int lsub) {
+  __shared__ int2 buf[TRAV_BUF * TRAV_THREADS];
+  const int nnodes = 2 * A.n - 1;
+  const int64_t nw = (int64_t)A.n << lsub;  // walks
+  WalkOut o;
+  const int share = xcd_block(blockIdx.x, gridDim.x);
+  for (int64_t i0 = (int64_t)share * TRAV_THREADS; i0 < nw; i0 += (int64_t)gridDim.x * TRAV_THREADS) {
+    const int64_t i = i0 + threadIdx.x;
+    Walk w;
+    if (i < nw) {
+      const bvh_node me = A.nodes[A.lpre[i >> lsub]];
+      w.e = me.left;
+      walk_element(A, w);
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        mlo[d] = it.blo[d];
-        mhi[d] = it.bhi[d];
+        w.lo[d] = me.lo[d];
+        w.hi[d] = me.hi[d];
       }
-      mb = ebox[e];
-      mt = ev[e];
-      mf = eflags[e];
-    }
-    for (;;) {
-      const bool active = nd >= 0 && nd < s1;
-      if (__ballot(active) == 0) break;
-      bool emit = false;
-      int2 pr{};
-      if (active) {
-        if (wlen == TRAV_LONG && qout) {  // hand the rest of this sub-range over
-          const int slot = atomicAdd(qout_n, 1);
-          if (slot < qcap) {
-            qout[slot] = TravItem{e, nd, s1, 0, {mlo[0], mlo[1], mlo[2], 0.f}, {mhi[0], mhi[1], mhi[2], 0.f}};
-            nd = -1;
-          }
-        }
-      }
-      if (active && nd >= 0) {
-        ++wlen;
-        const bvh_node node = nodes[nd];
-        if (!f32_overlap(node, mlo, mhi)) {
-          nd = node.rope;
-        } else if (node.left < 0) {
-          ++nd;
-        } else {
-          nd = node.rope;
-          const int e2 = node.left;
-          const dbox ob = ebox[e2];
-          const int4 ot = ev[e2];
-          const uint8_t of = eflags[e2];
-          asm volatile("" ::"v"(ot.x), "v"(ot.y), "v"(ot.z), "v"(ot.w), "v"((int)of));
-          if (f64_overlap(ob, mb) && !(scenes && scene_of(ot) != scene_of(mt))) {
-            ++cand;
-            const int rk = (e > e2) ? pair_reject_kind(mt, ot, mf) : pair_reject_kind(ot, mt, of);
-            if (rk) {
-              if constexpr (DUAL)
-                if (rk == REJ_SHARED || f64_overlap(pbox[e], pbox[e2])) ++pcand;
-            } else {
-              emit = true;
-              pr = make_int2(min(e, e2), max(e, e2));
-            }
-          }
-        }
-      }
-      const uint64_t m = __ballot(emit);
-      if (m) {
-        int base = 0;
-        if (lane == 0) base = atomicAdd(pair_count, (int)__popcll(m));
-        base = __shfl(base, 0) + (int)__popcll(m & below);
-        if (emit && base < cap) pairs[base] = pr;
+      w.nd = me.rope;
+      w.stop = nnodes;
+      if (lsub > 0 && w.nd >= 0) {  // this lane's share of [rope, nnodes)
+        const int sub = (int)(i & ((1 << lsub) - 1));
+        const int64_t span = nnodes - w.nd;
+        w.stop = w.nd + (int)((span * (sub + 1)) >> lsub);
+        w.nd += (int)((span * sub) >> lsub);
+        if (w.nd >= w.stop) w.nd = -1;
       }
     }
+    run_walks<DUAL>(A, w, o, buf);
   }
-  unsigned long long c = cand;
+  finish_walks<DUAL>(A, o, buf);
+}
+
+// Split walks: lane g walks sub-range g % TRAV_SPLIT of item g / TRAV_SPLIT.
+template <bool DUAL>
+__global__ void __launch_bounds__(TRAV_THREADS) k_traverse_split(TravArgs A,
+                                                                 const TravItem* __restrict__ qin,
+                                                                 const int* __restrict__ qin_n) {
+  __shared__ int2 buf[TRAV_BUF * TRAV_THREADS];
+  const int64_t total = (int64_t)min(*qin_n, A.qcap) * TRAV_SPLIT;
+  if ((int64_t)blockIdx.x * TRAV_THREADS >= total) return;
+  WalkOut o;
+  for (int64_t g0 = (int64_t)blockIdx.x * TRAV_THREADS; g0 < total;
+       g0 += (int64_t)gridDim.x * TRAV_THREADS) {
+    const int64_t g = g0 + threadIdx.x;
+    Walk w;
+    if (g < total) {
+      const TravItem it = qin[g / TRAV_SPLIT];
+      const int j = (int)(g % TRAV_SPLIT);
+      const int64_t span = (int64_t)it.hi - it.lo;
+      w.nd = it.lo + (int)(span * j / TRAV_SPLIT);
+      w.stop = it.lo + (int)(span * (j + 1) / TRAV_SPLIT);
+      if (w.nd >= w.stop) w.nd = -1;
+      w.e = it.e;
+      walk_element(A, w);
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-  if (lane == 0 && c) atomicAdd(cand_count, c);
-  if constexpr (DUAL) {
-    unsigned long long pc = pcand;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) pc += __shfl_xor(pc, o);
-    if (lane == 0 && pc) atomicAdd(pcand_count, pc);
+      for (int d = 0; d < 3; ++d) {
+        w.lo[d] = it.blo[d];
+        w.hi[d] = it.bhi[d];
+      }
+    }
+    run_walks<DUAL>(A, w, o, buf);
   }
+  finish_walks<DUAL>(A, o, buf);
 }
 
 // The swept-box pairs of the dual traversal whose static boxes overlap are
@@ -1270,29 +1279,25 @@ void launch_carry(hipStream_t st, DevState& S, int npairs_prev, int nhits_prev, 
 }
 
 // ---------------------------------------------------------------------------
-void launch_element_boxes(hipStream_t st, const DevState& S, int moving, double dt, dbox* out) {
+void launch_element_boxes(hipStream_t st, const DevState& S, double dt, dbox* sbox, dbox* mbox) {
   const int ne = S.ne;
   if (ne == 0) return;
   hipLaunchKernelGGL(k_element_boxes, dim3((ne + 255) / 256), dim3(256), 0, st, S.ev, S.x, S.x_old,
-                     S.av, dt, moving, ne, out);
+                     S.av, dt, ne, sbox, mbox);
 }
 
 hipError_t build_bvh(hipStream_t st, DevState& S) {
   const int n = S.ne;
   if (n == 0) return hipSuccess;
-  const float init[6] = {3.4e38f, 3.4e38f, 3.4e38f, -3.4e38f, -3.4e38f, -3.4e38f};
-  CS_HIP_RET(hipMemcpyAsync(S.bounds, init, sizeof(init), hipMemcpyHostToDevice, st));
-  int nb = (n + 255) / 256;
-  if (nb > 1024) nb = 1024;
-  hipLaunchKernelGGL(k_bounds, dim3(nb), dim3(256), 0, st, S.ebox, n, S.bounds);
-  hipLaunchKernelGGL(k_morton, dim3((n + 255) / 256), dim3(256), 0, st, S.ebox, n, S.bounds,
+  const int nb = std::min(BOUNDS_BLOCKS, (n + BOUNDS_THREADS - 1) / BOUNDS_THREADS);
+  hipLaunchKernelGGL(k_bounds, dim3(nb), dim3(BOUNDS_THREADS), 0, st, S.ebox, n, S.bounds);
+  hipLaunchKernelGGL(k_morton, dim3((n + 255) / 256), dim3(256), 0, st, S.ebox, n, S.bounds, nb,
                      S.mcode, S.mid);
   bool in_tmp = false;
   CS_HIP_RET(radix_sort_u32(st, S.mcode, S.mid, S.mcode_tmp, S.mid_tmp, S.sort_hist, S.scan_part, n,
                             30, &in_tmp));
   S.sorted_codes = in_tmp ? S.mcode_tmp : S.mcode;
   S.sorted_ids = in_tmp ? S.mid_tmp : S.mid;
-  S.n_top_start = 0;
   if (n == 1) {  // a single leaf: node 0
     bvh_node leaf{};
     leaf.left = 0;
@@ -1302,78 +1307,65 @@ hipError_t build_bvh(hipStream_t st, DevState& S) {
     CS_HIP_RET(hipMemcpyAsync(S.parent, &none, sizeof(int32_t), hipMemcpyHostToDevice, st));
     CS_HIP_RET(hipMemcpyAsync(S.lpre, &zero, sizeof(int32_t), hipMemcpyHostToDevice, st));
     CS_HIP_RET(hipMemcpyAsync(S.leaf_of, &zero, sizeof(int32_t), hipMemcpyHostToDevice, st));
-    CS_HIP_RET(hipMemcpyAsync(S.rmin, &zero, sizeof(int32_t), hipMemcpyHostToDevice, st));
-    CS_HIP_RET(hipMemcpyAsync(S.rmax, &zero, sizeof(int32_t), hipMemcpyHostToDevice, st));
     CS_HIP_RET(hipStreamSynchronize(st));  // host sources above live on this stack frame
   } else {
     const int nn = 2 * n - 1;
-    // every split position is written by k_karras; -1 (end) is a safe default
-    CS_HIP_RET(hipMemsetAsync(S.split_right, 0xff, sizeof(int32_t) * (size_t)(n - 1), st));
+    // (every split position 0 .. n - 2 belongs to one node: split_right is written whole)
     hipLaunchKernelGGL(k_karras, dim3((n - 1 + 255) / 256), dim3(256), 0, st, S.sorted_codes, n,
                        S.kleft, S.kright, S.kparent, S.split_right, S.krmin, S.krmax);
     hipLaunchKernelGGL(k_preorder, dim3((nn + 255) / 256), dim3(256), 0, st, n, S.kleft, S.kparent,
                        S.krmin, S.pre);
     hipLaunchKernelGGL(k_permute, dim3((nn + 255) / 256), dim3(256), 0, st, n, S.pre, S.kright,
-                       S.kparent, S.split_right, S.krmin, S.krmax, S.sorted_ids, S.nodes, S.parent,
-                       S.nright, S.rmin, S.rmax, S.lpre, S.leaf_of);
-    CS_HIP_RET(hipMemsetAsync(S.counters + CNT_TMP, 0, sizeof(int), st));
-    hipLaunchKernelGGL(k_mark_top, dim3((nn + 255) / 256), dim3(256), 0, st, S.nodes, S.nright,
-                       S.rmin, S.rmax, n, S.top_start, S.counters + CNT_TMP);
-    int cnt = 0;
-    CS_HIP_RET(hipMemcpyAsync(&cnt, S.counters + CNT_TMP, sizeof(int), hipMemcpyDeviceToHost, st));
-    CS_HIP_RET(hipStreamSynchronize(st));
-    S.n_top_start = cnt;
+                       S.kparent, S.split_right, S.krmax, S.sorted_ids, S.nodes, S.parent,
+                       S.nright, S.lpre, S.leaf_of);
   }
   return hipGetLastError();
 }
 
+// (the caller has zeroed CNT_TMP, the number of nodes that span tiles)
 hipError_t refit_bvh(hipStream_t st, DevState& S) {
   const int n = S.ne;
   if (n == 0) return hipSuccess;
-  if (n > 1) CS_HIP_RET(hipMemsetAsync(S.arrive, 0, sizeof(uint32_t) * (size_t)(2 * n - 1), st));
-  hipLaunchKernelGGL(k_refit_tiles, dim3((n + REFIT_TILE - 1) / REFIT_TILE), dim3(REFIT_THREADS), 0,
-                     st, S.ebox, S.sorted_ids, n, S.nodes, S.parent, S.nright, S.lpre, S.rmin,
-                     S.rmax, S.arrive);
-  if (n > 1 && S.n_top_start > 0)
-    hipLaunchKernelGGL(k_refit_top, dim3(1), dim3(1024), 0, st, S.nodes, S.parent, S.nright,
-                       S.rmin, S.rmax, S.top_start, S.n_top_start, S.arrive);
+  const int tiles = (n + REFIT_TILE - 1) / REFIT_TILE;
+  hipLaunchKernelGGL(k_refit_tiles, dim3(tiles), dim3(REFIT_TILE), 0, st, S.ebox, S.sorted_ids, n,
+                     S.nodes, S.lpre, S.krmin, S.krmax, S.pre, S.tbox, S.top, S.counters + CNT_TMP);
+  if (tiles > 1)
+    hipLaunchKernelGGL(k_refit_top, dim3(std::min(tiles, 2048)), dim3(256), 0, st, S.top,
+                       S.counters + CNT_TMP, S.krmin, S.krmax, S.pre, S.lpre, S.tbox, S.nodes);
   return hipGetLastError();
 }
 
+size_t refit_tile_count(int n) { return (size_t)(n + REFIT_TILE - 1) / REFIT_TILE; }
+
+// (the caller has zeroed the item counts of the split rounds, CNT_TSPLIT)
 void launch_traverse(hipStream_t st, DevState& S, int2* out, int cap, const dbox* pbox) {
   const int n = S.ne;
   if (n < 2) return;
-  // per-XCD leaf counters, then the item counts of the two split rounds
-  (void)hipMemsetAsync(S.tnext, 0, sizeof(int) * (kNumXcd + 2), st);
-  const int blocks = std::min(S.num_cus * S.tune_trav, (n + TRAV_THREADS - 1) / TRAV_THREADS);
+  int lsub = 0;
+  while (lsub < TRAV_SUB_MAX && ((int64_t)n << (lsub + 1)) <= TRAV_LANES) ++lsub;
+  const int64_t need = (((int64_t)n << lsub) + TRAV_THREADS - 1) / TRAV_THREADS;
+  // one walk per lane, up to 8 x tune_trav work-groups per CU
+  const int blocks = (int)std::min<int64_t>(need, 8ll * S.num_cus * S.tune_trav);
   TravItem* q0 = reinterpret_cast<TravItem*>(S.tq);
   TravItem* q1 = q0 + TRAV_QCAP;
-  int* n0 = S.tnext + kNumXcd;
-  int* n1 = n0 + 1;
-  auto* cand = (unsigned long long*)(S.counters + CNT_CAND64);
-  auto* pcand = pbox ? (unsigned long long*)(S.counters + CNT_PCAND64) : nullptr;
-  const int sblocks = 2 * S.num_cus;
-  if (pbox) {
-    hipLaunchKernelGGL(k_traverse<true>, dim3(std::max(blocks, 1)), dim3(TRAV_THREADS), 0, st,
-                       S.nodes, S.lpre, S.ebox, pbox, S.ev, S.eflags, n, out, cap,
-                       S.counters + CNT_PAIRS, cand, pcand, S.tnext, S.nscene > 1, q0, TRAV_QCAP);
-    hipLaunchKernelGGL(k_traverse_split<true>, dim3(sblocks), dim3(256), 0, st, S.nodes, S.ebox,
-                       pbox, S.ev, S.eflags, q0, n0, q1, n1, TRAV_QCAP, out, cap,
-                       S.counters + CNT_PAIRS, cand, pcand, S.nscene > 1);
-    hipLaunchKernelGGL(k_traverse_split<true>, dim3(sblocks), dim3(256), 0, st, S.nodes, S.ebox,
-                       pbox, S.ev, S.eflags, q1, n1, nullptr, nullptr, TRAV_QCAP, out, cap,
-                       S.counters + CNT_PAIRS, cand, pcand, S.nscene > 1);
-  } else {
-    hipLaunchKernelGGL(k_traverse<false>, dim3(std::max(blocks, 1)), dim3(TRAV_THREADS), 0, st,
-                       S.nodes, S.lpre, S.ebox, nullptr, S.ev, S.eflags, n, out, cap,
-                       S.counters + CNT_PAIRS, cand, nullptr, S.tnext, S.nscene > 1, q0, TRAV_QCAP);
-    hipLaunchKernelGGL(k_traverse_split<false>, dim3(sblocks), dim3(256), 0, st, S.nodes, S.ebox,
-                       nullptr, S.ev, S.eflags, q0, n0, q1, n1, TRAV_QCAP, out, cap,
-                       S.counters + CNT_PAIRS, cand, nullptr, S.nscene > 1);
-    hipLaunchKernelGGL(k_traverse_split<false>, dim3(sblocks), dim3(256), 0, st, S.nodes, S.ebox,
-                       nullptr, S.ev, S.eflags, q1, n1, nullptr, nullptr, TRAV_QCAP, out, cap,
-                       S.counters + CNT_PAIRS, cand, nullptr, S.nscene > 1);
-  }
+  int* n0 = S.counters + CNT_TSPLIT;
+  TravArgs A{S.nodes, S.lpre, S.ebox, pbox, S.ev, S.eflags, n, S.nscene > 1, out, cap,
+             S.counters + CNT_PAIRS, (unsigned long long*)(S.counters + CNT_CAND64),
+             (unsigned long long*)(S.counters + CNT_PCAND64), q0, n0, TRAV_QCAP};
+  TravArgs A1 = A, A2 = A;
+  A1.qout = q1;
+  A1.qout_n = n0 + 1;
+  A2.qout = nullptr;
+  A2.qout_n = nullptr;
+  auto go = [&](auto main, auto split) {
+    hipLaunchKernelGGL(main, dim3(blocks), dim3(TRAV_THREADS), 0, st, A, lsub);
+    hipLaunchKernelGGL(split, dim3(4 * S.num_cus), dim3(TRAV_THREADS), 0, st, A1,
+                       (const TravItem*)q0, (const int*)n0);
+    hipLaunchKernelGGL(split, dim3(4 * S.num_cus), dim3(TRAV_THREADS), 0, st, A2,
+                       (const TravItem*)q1, (const int*)(n0 + 1));
+  };
+  if (pbox) go(k_traverse<true>, k_traverse_split<true>);
+  else go(k_traverse<false>, k_traverse_split<false>);
 }
 
 void launch_split_seed(hipStream_t st, DevState& S, int n) {

@@ -32,7 +32,7 @@ enum {
   CNT_HIT_PAIRS = 2,     // pairs with at least one hit (hit-pair records)
   CNT_HIT_SUB = 3,       // hit sub-tests
   CNT_LOG = 4,           // pair-log rows
-  CNT_TMP = 5,           // scratch count (LBVH top nodes)
+  CNT_TMP = 5,           // LBVH nodes spanning refit tiles
   CNT_ZONES = 6,         // impact zones updated
   CNT_QPAIRS = 7,        // pairs found by the dirty-element query
   CNT_STRAIN_FLAG = 8,   // strain sweep state
@@ -50,6 +50,7 @@ enum {
   CNT_DRANGES = 23,      // tree ranges holding dirty leaves (kept until the next pass clears them)
   CNT_VLIST = 24,        // 24, 25: vertices whose average velocity a pass changed through
                         // hits (dirty vertex list), by pass parity
+  CNT_TSPLIT = 26,       // 26, 27: split walks of the full traversal, by round
   CNT_SNAP = 28,         // 28..31: pair/hit counts carried into the current pass
   CNT_PCAND64 = 32,      // 32, 33: static-box overlaps found by the swept-box traversal
   CNT_PPAIRS = 34,       // pairs of that traversal whose static boxes overlap
@@ -195,27 +196,23 @@ struct DevState {
   // node's first child is the next record)
   int32_t* parent = nullptr;       // parent of every node, -1 at the root
   int32_t* nright = nullptr;       // second child of an internal node (-1 at leaves)
-  int32_t *rmin = nullptr, *rmax = nullptr;  // Morton leaf range of every node
   int32_t* lpre = nullptr;         // node of Morton leaf j
   // construction arrays (radix-tree order) of the last build
   int32_t *kleft = nullptr, *kright = nullptr, *kparent = nullptr;
   int32_t *krmin = nullptr, *krmax = nullptr, *pre = nullptr;
   int32_t* split_right = nullptr;  // [g]: second child of the node splitting after leaf g
-  uint32_t* arrive = nullptr;
-  int32_t* top_start = nullptr;  // nodes spanning several refit tiles whose children do not
-  int n_top_start = 0;           // (built once per LBVH build)
+  float* tbox = nullptr;         // box of every refit tile
+  int32_t* top = nullptr;        // nodes spanning refit tiles (construction order)
   uint32_t* scan_part = nullptr; // partial sums of the device scan
   size_t scan_part_words = 0;
   int32_t* leaf_of = nullptr;    // element -> pre-order index of its leaf
   // dirty leaves by pre-order index, and the QW_RANGE-node ranges holding them
   uint8_t* dpre = nullptr;
   int32_t *rflag = nullptr, *rlist = nullptr;
-  int32_t* tnext = nullptr;        // persistent full traversal: next leaf per XCD share,
-                                   // then the item counts of the two split rounds
   void* tq = nullptr;              // split walks of the full traversal, 2 x TRAV_QCAP items
   int num_cus = 256;               // compute units of the device
-  // launch shapes (cs_set_tuning / the autotuner): persistent traversal
-  // work-groups per CU, narrow-phase work-group size, dirty-query grid cap
+  // launch shapes (cs_set_tuning / the autotuner): traversal work-groups per
+  // CU, narrow-phase work-group size, dirty-query grid cap
   int tune_trav = 8, tune_narrow = 128, tune_query = 4096;
   // candidate stream (current and previous pass)
   int2* pairs = nullptr;
@@ -348,9 +345,12 @@ hipError_t radix_sort_u64(hipStream_t st, uint64_t* keys, uint32_t* vals, uint64
                           bool* result_in_tmp);
 
 // broad phase
-void launch_element_boxes(hipStream_t st, const DevState& S, int moving, double dt, dbox* out);
-hipError_t build_bvh(hipStream_t st, DevState& S);  // also finds the refit top nodes
+// static boxes into sbox, swept boxes into mbox (either may be null)
+void launch_element_boxes(hipStream_t st, const DevState& S, double dt, dbox* sbox, dbox* mbox);
+hipError_t build_bvh(hipStream_t st, DevState& S);
 hipError_t refit_bvh(hipStream_t st, DevState& S);
+size_t refit_tile_count(int n);
+constexpr int BOUNDS_FLOATS = 6 * 128;  // rows of k_bounds
 // candidate pairs of the current boxes (ebox) into out; with pbox (static
 // boxes, each inside its element's swept box in ebox), also the static-box
 // overlaps among the rejected pairs (CNT_PCAND64)
@@ -473,26 +473,6 @@ __device__ inline unsigned long long block_sum_u64(unsigned long long v, unsigne
     for (int w = 0; w < (int)(blockDim.x + 63) / 64; ++w) t += s_w[w];
   __syncthreads();
   return t;  // valid in thread 0
-}
-
-// float atomics via CAS (monotone min/max on finite values)
-__device__ inline void atomicMin_float(float* addr, float v) {
-  int* ai = (int*)addr;
-  int old = *ai;
-  while (__int_as_float(old) > v) {
-    int prev = atomicCAS(ai, old, __float_as_int(v));
-    if (prev == old) break;
-    old = prev;
-  }
-}
-__device__ inline void atomicMax_float(float* addr, float v) {
-  int* ai = (int*)addr;
-  int old = *ai;
-  while (__int_as_float(old) < v) {
-    int prev = atomicCAS(ai, old, __float_as_int(v));
-    if (prev == old) break;
-    old = prev;
-  }
 }
 
 }  // namespace cs
