@@ -429,7 +429,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
   // the dirty-range marks of the previous pass are cleared first (their count
   // is zeroed below)
   if (S.ne >= 2) launch_clear_ranges(h->st, S);
-  // pairs, hits, hit pairs, sub-tests, query pairs, dirty elements, the
+  // pairs, hits, hit pairs, query pairs, dirty elements, the
   // 64-bit candidate counts and the dirty-range count
   // and the list of vertices this pass's hits change; the list of the
   // previous pass (the other parity) is read by this pass
@@ -437,7 +437,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
   const int* vcount_prev = S.counters + CNT_VLIST + ((pass_id & 1) ^ 1);
   launch_zero_counters(h->st, S,
                        (1u << CNT_PAIRS) | (1u << CNT_HITS) | (1u << CNT_HIT_PAIRS) |
-                           (1u << CNT_HIT_SUB) | (1u << CNT_TMP) | (1u << CNT_QPAIRS) |
+                           (1u << CNT_TMP) | (1u << CNT_QPAIRS) |
                            (1u << CNT_DIRTY) | (3u << CNT_TSPLIT) |
                            (0x3fu << CNT_CAND64) | (1u << CNT_DRANGES) |
                            (1u << (CNT_VLIST + (pass_id & 1))));
@@ -469,7 +469,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
     NP.ds_stride = h->L.ds_stride;
     NP.ds_salt = h->L.ds_salt++;
   }
-  int npairs = 0, carried_hits = 0, carried_hp = 0, carried_sub = 0, carried_pairs = 0;
+  int npairs = 0, carried_hits = 0, carried_hp = 0, carried_pairs = 0;
   unsigned long long cand = 0;
   int nq = 0;
   int nhits = 0, nhp = 0;
@@ -525,7 +525,6 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
       HIPCHK(h, grow_hit_buffers(h, nhits, nhp, 0, 0));
       if ((rc = set_counter(h, CNT_HITS, 0))) return rc;
       if ((rc = set_counter(h, CNT_HIT_PAIRS, 0))) return rc;
-      if ((rc = set_counter(h, CNT_HIT_SUB, 0))) return rc;
     }
     if (dual) {  // (counted by the split, read with the narrow phase's counters)
       npairs = h->h_counters[CNT_PPAIRS];
@@ -586,7 +585,6 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
       HIPCHK(h, grow_hit_buffers(h, nhits, nhp, 0, 0));
       if ((rc = set_counter(h, CNT_HITS, 0))) return rc;
       if ((rc = set_counter(h, CNT_HIT_PAIRS, 0))) return rc;
-      if ((rc = set_counter(h, CNT_HIT_SUB, 0))) return rc;
     }
   } else {
     // One host synchronisation per pass: the narrow phase reads the number
@@ -633,7 +631,6 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
       carried_pairs = h->h_counters[CNT_SNAP + CNT_PAIRS];
       carried_hits = h->h_counters[CNT_SNAP + CNT_HITS];
       carried_hp = h->h_counters[CNT_SNAP + CNT_HIT_PAIRS];
-      carried_sub = h->h_counters[CNT_SNAP + CNT_HIT_SUB];
       nhits = h->h_counters[CNT_HITS];
       nhp = h->h_counters[CNT_HIT_PAIRS];
       const bool q_over = nq > S.qpair_cap;
@@ -650,7 +647,6 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
       HIPCHK(h, grow_hit_buffers(h, nhits, nhp, carried_hits, carried_hp));
       if ((rc = set_counter(h, CNT_HITS, carried_hits))) return rc;
       if ((rc = set_counter(h, CNT_HIT_PAIRS, carried_hp))) return rc;
-      if ((rc = set_counter(h, CNT_HIT_SUB, carried_sub))) return rc;
     }
     narrow_n = nq;
     npairs = exact_counts && prev.npairs >= 0 ? carried_pairs + nq : -1;
@@ -689,7 +685,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
   pi.tested_pairs = narrow_n;
   pi.incremental = (incremental || seeded) ? 1 : 0;
   pi.hit_pairs = nhp;
-  pi.hit_subtests = h->h_counters[CNT_HIT_SUB];
+  pi.hit_subtests = nhits;
   if (P.log_pairs) {  // the pair log is read after every pass
     int rc = read_counters(h);
     if (rc) return rc;

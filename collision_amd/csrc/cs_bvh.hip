@@ -1215,10 +1215,7 @@ __global__ void __launch_bounds__(256) k_carry_hp(const int4* __restrict__ prev,
     keep = !dirty_e[r.x] && !dirty_e[r.y];
   }
   const int slot = block_append(keep, &counters[CNT_HIT_PAIRS], &s_cnt, &s_base);
-  if (keep) {
-    if (slot < cap) cur[slot] = r;
-    atomicAdd(&counters[CNT_HIT_SUB], __popc(r.z));
-  }
+  if (keep && slot < cap) cur[slot] = r;
 }
 
 void launch_mark_dirty(hipStream_t st, DevState& S, const int* vcount, int nzone) {

@@ -28,9 +28,8 @@ enum : int {
 // slots of the small device counter block (ints; 64-bit counts at 16..21)
 enum {
   CNT_PAIRS = 0,         // pairs in the candidate stream being built
-  CNT_HITS = 1,          // hit records
-  CNT_HIT_PAIRS = 2,     // pairs with at least one hit (hit-pair records)
-  CNT_HIT_SUB = 3,       // hit sub-tests
+  CNT_HITS = 2,          // hit records (an even index: the narrow phase adds to
+  CNT_HIT_PAIRS = 3,     // both in one 64-bit add); pairs with at least one hit
   CNT_LOG = 4,           // pair-log rows
   CNT_TMP = 5,           // LBVH nodes spanning refit tiles
   CNT_ZONES = 6,         // impact zones updated
