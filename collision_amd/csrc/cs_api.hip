@@ -214,8 +214,7 @@ void free_dev(DevState& S) {
   dfree(S.hkey); dfree(S.hkey_tmp); dfree(S.hidx); dfree(S.hidx_tmp);
   dfree(S.rkey); dfree(S.rkey_tmp); dfree(S.rval); dfree(S.rval_tmp);
   dfree(S.zmark); dfree(S.zlist); dfree(S.zkey64); dfree(S.zkey64_tmp);
-  dfree(S.zkey); dfree(S.zval); dfree(S.zval_tmp);
-  dfree(S.zhead); dfree(S.zend);
+  dfree(S.zval); dfree(S.zval_tmp);
   dfree(S.lvl_ptr); dfree(S.plog); dfree(S.counters); dfree(S.spread); dfree(S.scn); dfree(S.vscene);
   dfree(S.sslot); dfree(S.spre); dfree(S.slast);
   dfree(S.lvl_active);
@@ -1204,9 +1203,7 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   HIPCHK(h, dalloc(&S.rlist, (2 * ne - 1 + QW_RANGE - 1) / QW_RANGE));
   HIPCHK(h, dalloc(&S.zmark, nv)); HIPCHK(h, dalloc(&S.zlist, nv));
   HIPCHK(h, dalloc(&S.zkey64, nv)); HIPCHK(h, dalloc(&S.zkey64_tmp, nv));
-  HIPCHK(h, dalloc(&S.zkey, nv));
   HIPCHK(h, dalloc(&S.zval, nv)); HIPCHK(h, dalloc(&S.zval_tmp, nv));
-  HIPCHK(h, dalloc(&S.zhead, nv)); HIPCHK(h, dalloc(&S.zend, nv));
   S.n_sched = nsched;
   if (plan.nband > 0) {
     HIPCHK(h, upload_plan(S, plan));

@@ -244,9 +244,7 @@ struct DevState {
   int32_t* zmark = nullptr;
   uint32_t* zlist = nullptr;
   uint64_t *zkey64 = nullptr, *zkey64_tmp = nullptr;
-  uint32_t *zkey = nullptr, *zval = nullptr, *zval_tmp = nullptr;
-  int32_t* zhead = nullptr;  // first sorted index of each zone
-  int32_t* zend = nullptr;   // one past the last sorted index, by zone root
+  uint32_t *zval = nullptr, *zval_tmp = nullptr;
   // strain-limit schedule: slots in level order, slots of level L are
   // [lvl_ptr[L], lvl_ptr[L+1])
   int32_t* lvl_ptr = nullptr;
