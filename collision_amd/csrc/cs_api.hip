@@ -238,13 +238,13 @@ hipError_t grow_keep(T** p, int keep, size_t new_count, hipStream_t st) {
 
 // hit records: current buffer keeps its first `keep` records
 hipError_t alloc_hits(DevState& S, int cap, int keep, hipStream_t st) {
-  dfree(S.hkey); dfree(S.hkey_tmp); dfree(S.hidx); dfree(S.hidx_tmp);
+  dfree(S.hkey_tmp); dfree(S.hidx); dfree(S.hidx_tmp);
   dfree(S.rkey); dfree(S.rkey_tmp); dfree(S.rval); dfree(S.rval_tmp);
   dfree(S.hits_prev);
   S.hit_cap = cap;
   CS_HIP_RET(grow_keep(&S.hits, keep, cap, st));
   CS_HIP_RET(dalloc(&S.hits_prev, cap));
-  CS_HIP_RET(dalloc(&S.hkey, cap));
+  CS_HIP_RET(grow_keep(&S.hkey, keep, cap, st));
   CS_HIP_RET(dalloc(&S.hkey_tmp, cap));
   CS_HIP_RET(dalloc(&S.hidx, cap));
   CS_HIP_RET(dalloc(&S.hidx_tmp, cap));
@@ -375,6 +375,7 @@ hipError_t grow_hit_buffers(cs_solver* h, int nhits, int nhp, int keep_hits, int
 hipError_t narrow_call(cs_solver* h, NarrowParams NP, const int2* pairs, int npairs,
                        const int* npairs_dev, int cap) {
   if (npairs <= 0) return hipSuccess;
+  NP.hkey = h->S.hkey;
   if (NP.ccd && h->P.learned) {
     const uint32_t* perm = nullptr;
     CS_HIP_RET(launch_learned_score(h->st, h->S, h->L, pairs, npairs, npairs_dev, cap, NP.dt,
@@ -425,21 +426,19 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
   const PrevPass prev = h->prev;
   h->prev.valid = false;
   mark_pass(h, &T.e0, 2);
-  // the dirty-range marks of the previous pass are cleared first (their count
-  // is zeroed below)
-  if (S.ne >= 2) launch_clear_ranges(h->st, S);
-  // pairs, hits, hit pairs, query pairs, dirty elements, the
-  // 64-bit candidate counts and the dirty-range count
-  // and the list of vertices this pass's hits change; the list of the
-  // previous pass (the other parity) is read by this pass
+  // The dirty marks of the previous pass are cleared, then its counts: pairs,
+  // hits, hit pairs, query pairs, dirty elements, the 64-bit candidate counts,
+  // the dirty-range count and the list of vertices this pass's hits change; the
+  // list of the previous pass (the other parity) is read by this pass.  Before
+  // the proximity pass, the first of a step, the prologue has cleared all.
   int* vcount_cur = S.counters + CNT_VLIST + (pass_id & 1);
   const int* vcount_prev = S.counters + CNT_VLIST + ((pass_id & 1) ^ 1);
-  launch_zero_counters(h->st, S,
-                       (1u << CNT_PAIRS) | (1u << CNT_HITS) | (1u << CNT_HIT_PAIRS) |
-                           (1u << CNT_TMP) | (1u << CNT_QPAIRS) |
-                           (1u << CNT_DIRTY) | (3u << CNT_TSPLIT) |
-                           (0x3fu << CNT_CAND64) | (1u << CNT_DRANGES) |
-                           (1u << (CNT_VLIST + (pass_id & 1))));
+  if (kind != CS_PASS_PROXIMITY)
+    launch_pass_begin(h->st, S,
+                      (1ull << CNT_PAIRS) | (1ull << CNT_HITS) | (1ull << CNT_HIT_PAIRS) |
+                          (1ull << CNT_TMP) | (1ull << CNT_QPAIRS) | (1ull << CNT_DIRTY) |
+                          (3ull << CNT_TSPLIT) | (0x3full << CNT_CAND64) | (1ull << CNT_DRANGES) |
+                          (1ull << (CNT_VLIST + (pass_id & 1))));
   NarrowParams NP{};
   NP.dt = P.dt; NP.thickness = P.thickness; NP.round_eps = P.round_eps;
   NP.k = P.spring_k; NP.m = P.mass; NP.lambda = P.friction; NP.cr = P.restitution;
@@ -459,6 +458,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
   NP.log_pairs = P.log_pairs;
   NP.pass_id = pass_id;
   NP.spread = S.spread;
+  NP.hb = hit_id_bits(S);
   if (ccd && h->L.ds_cap > 0) {  // dataset collection (cs_learned_collect)
     NP.dsx = h->L.dsx;
     NP.dse = h->L.dse;
@@ -506,7 +506,6 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
       h->seed.valid = true;
       h->seed.npairs = npairs;
       h->seed.cand = cand;
-      HIPCHK(h, hipMemsetAsync(S.counters + CNT_PPAIRS, 0, sizeof(int), h->st));
       launch_split_seed(h->st, S, npairs);
       stream_dev = S.counters + CNT_PPAIRS;
     }
@@ -537,9 +536,9 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
     // (the proximity pass ran another test), so every pair is tested.
     launch_mark_dirty(h->st, S, vcount_prev, 0);
     mark_pass(h, &T.t0, 1);
-    if (exact_counts) launch_query_dirty(h->st, S, 0);  // seed boxes: count only
-    launch_grow_dirty(h->st, S, P.dt);  // new boxes; leaves exact, ancestors grown
-    launch_query_dirty(h->st, S, 1);
+    if (exact_counts) launch_query_dirty(h->st, S, 0, 0);  // seed boxes: count only
+    launch_grow_carry(h->st, S, P.dt, 0, 0, 0);  // new boxes; leaves exact, ancestors grown
+    launch_query_dirty(h->st, S, 1, 0);
     mark_pass(h, &T.t1, 1);
     launch_carry_pairs_from(h->st, S, S.pairs_seed, seed.npairs);
     for (int attempt = 0;; ++attempt) {
@@ -553,7 +552,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
       HIPCHK(h, dalloc(&S.qpairs, S.qpair_cap));
       HIPCHK(h, hipMemsetAsync(S.counters + CNT_QPAIRS, 0, sizeof(int), h->st));
       HIPCHK(h, hipMemsetAsync(S.counters + CNT_NEW64, 0, 2 * sizeof(int), h->st));
-      launch_query_dirty(h->st, S, 1);
+      launch_query_dirty(h->st, S, 1, 0);
     }
     carried_pairs = h->h_counters[CNT_PAIRS];
     npairs = carried_pairs + nq;
@@ -597,19 +596,15 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
     // previous boxes: count only.  The count only feeds the exact candidate
     // total of the pass (a diagnostic), so it runs when the caller asks for
     // the parity taps; otherwise the candidate total is reported as -1.
-    if (exact_counts) launch_query_dirty(h->st, S, 0);
-    launch_grow_dirty(h->st, S, P.dt);               // new boxes; leaves exact, ancestors grown
-    launch_query_dirty(h->st, S, 1);                 // current boxes: count + emit
-    mark_pass(h, &T.t1, 1);
+    if (exact_counts) launch_query_dirty(h->st, S, 0, 0);
+    // new boxes (leaves exact, ancestors grown); hits and hit pairs carried over
+    launch_grow_carry(h->st, S, P.dt, prev.nhits, prev.nhp, kind == CS_PASS_ZONE);
     // the candidate pair stream itself only feeds the exact pair count of the
     // pass; it is carried when the caller asks for exact counts
-    launch_carry(h->st, S, exact_counts ? prev.npairs : 0, prev.nhits, prev.nhp);
-    HIPCHK(h, hipMemcpyAsync(S.counters + CNT_SNAP, S.counters, sizeof(int) * 4,
-                             hipMemcpyDeviceToDevice, h->st));
+    if (exact_counts) launch_carry_pairs_from(h->st, S, S.pairs_prev, prev.npairs);
+    launch_query_dirty(h->st, S, 1, 1);  // current boxes: count + emit
+    mark_pass(h, &T.t1, 1);
     mark_pass(h, &T.e1, 2);
-    // impact-zone merges of the carried hit pairs (union order does not
-    // change the partition); their count is read on the device
-    if (kind == CS_PASS_ZONE) launch_hp_unions(h->st, S, prev.nhp, 1);
     // grid for a guess of the re-queried pair count; pairs beyond it are
     // handled after the count is known
     const int guess = std::min(S.qpair_cap, std::max(4096, 2 * prev.nq + 1024));
@@ -641,7 +636,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
         HIPCHK(h, dalloc(&S.qpairs, S.qpair_cap));
         HIPCHK(h, hipMemsetAsync(S.counters + CNT_QPAIRS, 0, sizeof(int), h->st));
         HIPCHK(h, hipMemsetAsync(S.counters + CNT_NEW64, 0, 2 * sizeof(int), h->st));
-        launch_query_dirty(h->st, S, 1);
+        launch_query_dirty(h->st, S, 1, 0);
       }
       HIPCHK(h, grow_hit_buffers(h, nhits, nhp, carried_hits, carried_hp));
       if ((rc = set_counter(h, CNT_HITS, carried_hits))) return rc;
@@ -666,12 +661,11 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
   }
   mark_pass(h, &T.e2, 2);
   launch_scene_pass(h->st, S, kind, index, nhp, P.max_ccd_passes);  // batched scenes
-  HIPCHK(h, apply_hits(h->st, S, nhits, vcount_cur, P.record_impulses != 0 && S.pimp));
+  const int nzone = kind == CS_PASS_ZONE ? h->h_counters[CNT_ZLIST] : 0;
+  HIPCHK(h, apply_hits(h->st, S, nhits, vcount_cur, P.record_impulses != 0 && S.pimp, nzone));
   HIPCHK(h, apply_bodies(h->st, S, P.mass, P.dt));  // RG impulses, body zones (updateAverageVelocity)
-  int nzone = 0;
   if (kind == CS_PASS_ZONE) {
-    nzone = h->h_counters[CNT_ZLIST];
-    HIPCHK(h, update_zones(h->st, S, P.mass, P.dt, nzone));  // (resets the zone count)
+    HIPCHK(h, update_zones(h->st, S, P.mass, P.dt, nzone));
     HIPCHK(h, update_body_zones(h->st, S, P.mass, P.dt));    // body zones hold >= 2 points
   }
   if (P.log_pairs) launch_hp_log(h->st, S, nhp, pass_id);
@@ -1399,25 +1393,17 @@ int cs_predict(cs_solver* h) {
 namespace {
 
 // The launches of a resolve before its first host synchronisation (kernels
-// only, so that they can be captured in a graph): the dirty-range marks of
-// the last pass are cleared while their count is still in the counter block,
-// then the counters, the union-find (makeSet, dcollid.cpp:1015-1031), the
-// batched scenes' pass state, the recorded impulses, the zone marks and
-// computeAverageVelocity.
+// only, so that they can be captured in a graph): the dirty marks of the last
+// pass and the counters, the batched scenes' pass state, then
+// computeAverageVelocity with the union-find (makeSet, dcollid.cpp:1015-1031),
+// the recorded impulses and the zone marks.
 void resolve_prologue(cs_solver* h, bool stats) {
   DevState& S = h->S;
   const cs_params& P = h->P;
-  if (S.ne >= 2) launch_clear_ranges(h->st, S);
-  launch_fill_u32(h->st, S.counters, COUNTER_INTS, 0u);
+  launch_pass_begin(h->st, S, ~0ull);
   if (stats) launch_fill_u32(h->st, S.spread, (int64_t)SPREAD_SLOTS * SPREAD_STRIDE, 0u);
-  launch_uf_init(h->st, S);
   launch_scene_reset(h->st, S);
-  if (P.record_impulses && S.pimp) {  // the impulses of this resolve's last pass with a hit
-    launch_fill_u32(h->st, S.pimp, (int64_t)S.nv * (int64_t)(sizeof(dvec4) / 4), 0u);
-    launch_fill_u32(h->st, S.pnum, S.nv, 0u);
-  }
-  launch_fill_u32(h->st, S.zmark, S.nv, 0u);
-  launch_average_velocity(h->st, S, P.dt);
+  launch_average_velocity(h->st, S, P.dt, P.record_impulses && S.pimp);
 }
 
 // the predictor and the resolve prologue as one graph, captured again when
@@ -1527,8 +1513,6 @@ int resolve_impl(cs_solver* h, cs_step_report* report, bool with_predict_graph) 
   if (status == CS_OK || status == CS_WARN_ZONE_CAP) {
     launch_domain_boundary(h->st, S, P.dom_lo, P.dom_hi, P.dt, P.friction, P.thickness);
     launch_final_position(h->st, S, P.dt);
-    HIPCHK(h, hipMemsetAsync(S.counters + CNT_STRAIN_FLAG, 0, sizeof(int) * 4, h->st));
-    HIPCHK(h, hipMemsetAsync(S.counters + CNT_STRAIN_LEVELS, 0, sizeof(int) * 2, h->st));
     HIPCHK(h, strain_limit(h->st, S, P.dt, P.max_strain_sweeps,
                            P.pass_timing >= 1 ? &strain_marks : nullptr));
     launch_final_velocity(h->st, S);

@@ -58,6 +58,23 @@ __host__ __device__ inline uint64_t hit_key(uint32_t lo, uint32_t hi, uint32_t s
   return ((uint64_t)lo << 36) | ((uint64_t)hi << 8) | (uint64_t)sub;
 }
 
+// Sort key of a hit: (lo, hi, sub-test) packed as tightly as the element count
+// allows (hi in hb bits, the sub-test, at most 15, in 4 bits), which keeps the
+// order of the record key and needs fewer digit passes.
+__host__ __device__ inline uint64_t hit_sort_key(uint64_t k, int hb) {
+  const uint64_t lo = k >> 36, hi = (k >> 8) & 0xFFFFFFFull, sub = k & 255u;
+  return (((lo << hb) | hi) << 4) | sub;
+}
+
+// record of a hit's point p: key = the vertex; the body spreads of an all-rigid
+// contact use points 0 and 1 with key nv + body; points without a contribution
+// get the sentinel nv + nbody and sort last
+__device__ inline uint32_t hit_record_key(const hit_rec& h, int p, int nv, int nbody) {
+  const int v = h.v[p];
+  const int b = p < 2 ? h.sb[p] : -1;
+  return (v >= 0) ? (uint32_t)v : (b >= 0 ? (uint32_t)(nv + b) : (uint32_t)(nv + nbody));
+}
+
 __device__ inline double smin(double a, double b) { return (b < a) ? b : a; }  // std::min
 __device__ inline double smax(double a, double b) { return (a < b) ? b : a; }  // std::max
 

@@ -28,6 +28,7 @@ enum : int {
 // slots of the small device counter block (ints; 64-bit counts at 16..21)
 enum {
   CNT_PAIRS = 0,         // pairs in the candidate stream being built
+  CNT_TICKET = 1,        // work-groups of launch_pass_begin that are done
   CNT_HITS = 2,          // hit records (an even index: the narrow phase adds to
   CNT_HIT_PAIRS = 3,     // both in one 64-bit add); pairs with at least one hit
   CNT_LOG = 4,           // pair-log rows
@@ -69,6 +70,8 @@ struct NarrowParams {
   int log_pairs;
   int pass_id;
   int* spread;  // [SPREAD_SLOTS][SPREAD_STRIDE] statistics (SP_*)
+  uint64_t* hkey;  // sort key of each hit record, packed with hb bits per element id
+  int hb;
   // learned form (CCD passes): the scoring kernel's per-sub-test seeds
   // (16 per pair, by pair position before reordering; sign bit set = root
   // predicted) and the reordering of the pairs (nullptr: none)
@@ -337,9 +340,14 @@ hipError_t exclusive_scan_u32(hipStream_t st, uint32_t* data, int n, uint32_t* p
 hipError_t radix_sort_u32(hipStream_t st, uint32_t* keys, uint32_t* vals, uint32_t* tmp_keys,
                           uint32_t* tmp_vals, uint32_t* hist, uint32_t* partials, int n, int bits,
                           bool* result_in_tmp);
+// iota: the values are the keys' indices (vals is only used as a buffer)
 hipError_t radix_sort_u64(hipStream_t st, uint64_t* keys, uint32_t* vals, uint64_t* tmp_keys,
                           uint32_t* tmp_vals, uint32_t* hist, uint32_t* partials, int n, int bits,
-                          bool* result_in_tmp);
+                          bool* result_in_tmp, bool iota = false);
+// up to RANK_SORT_MAX hits: their records (4 each) in canonical order
+constexpr int RANK_SORT_MAX = 32768;
+hipError_t rank_hits(hipStream_t st, const uint64_t* keys, const hit_rec* hits, int n, int nv,
+                     int nbody, uint32_t* rkey, uint32_t* rval);
 
 // broad phase
 // static boxes into sbox, swept boxes into mbox (either may be null)
@@ -359,16 +367,16 @@ void launch_split_seed(hipStream_t st, DevState& S, int n);
 // elements of the vertices the previous pass changed: *vcount hit vertices
 // in vlist and nzone zone members in zlist
 void launch_mark_dirty(hipStream_t st, DevState& S, const int* vcount, int nzone);
-// clears the previous pass's dirty-range marks; its range count is zeroed by
-// the caller afterwards (launch_zero_counters)
-void launch_clear_ranges(hipStream_t st, DevState& S);
-void launch_zero_counters(hipStream_t st, DevState& S, uint32_t mask);
+// clears the dirty marks of the previous pass and the counters in the mask
+void launch_pass_begin(hipStream_t st, DevState& S, uint64_t mask);
 constexpr int QW_RANGE_SHIFT = 3;
 constexpr int QW_RANGE = 1 << QW_RANGE_SHIFT;  // pre-order nodes per dirty-query range
-void launch_query_dirty(hipStream_t st, DevState& S, int emit);
-// the dirty elements' new swept boxes, their leaves exact and ancestors grown
-void launch_grow_dirty(hipStream_t st, DevState& S, double dt);
-void launch_carry(hipStream_t st, DevState& S, int npairs_prev, int nhits_prev, int nhp_prev);
+// snap: the counts carried into the pass are kept in CNT_SNAP..
+void launch_query_dirty(hipStream_t st, DevState& S, int emit, int snap);
+// the dirty elements' new swept boxes, their leaves exact and ancestors grown;
+// the previous pass's clean hits and hit pairs (zone: with their zone merges)
+void launch_grow_carry(hipStream_t st, DevState& S, double dt, int nhits_prev, int nhp_prev,
+                       int zone);
 // pairs of src[0..n) with no dirty element into S.pairs (count CNT_PAIRS)
 void launch_carry_pairs_from(hipStream_t st, DevState& S, const int2* src, int n);
 
@@ -381,13 +389,19 @@ void launch_narrow(hipStream_t st, DevState& S, const NarrowParams& P, const int
 hipError_t launch_learned_score(hipStream_t st, DevState& S, LearnedState& L, const int2* pairs,
                                 int npairs, const int* npairs_dev, int cap, double dt, double h,
                                 const uint32_t** perm);
-void launch_hp_unions(hipStream_t st, DevState& S, int n, int ccd);
 void launch_hp_log(hipStream_t st, DevState& S, int n, int pass_id);
 // y = f(x) with the step's elementary functions (0 acos, 1 cos, 2 sin, 3 pow(x, 1/3))
 hipError_t launch_math_eval(hipStream_t st, int fn, const double* x, double* y, int64_t n);
 
 // response
-hipError_t apply_hits(hipStream_t st, DevState& S, int nhits, int* vcount, bool record);
+// bits of an element id in the hits' sort keys
+inline int hit_id_bits(const DevState& S) {
+  int hb = 1;
+  while (hb < 32 && ((uint64_t)S.ne >> hb) != 0) ++hb;
+  return hb;
+}
+// nzone > 0: also the sort keys of the zone members, for update_zones
+hipError_t apply_hits(hipStream_t st, DevState& S, int nhits, int* vcount, bool record, int nzone);
 // movable bodies, after apply_hits: the RG part of updateAverageVelocity
 // (dcollid.cpp:728-734) and, when dt > 0, updateImpactZoneVelocityForRG
 // (dcollid.cpp:267-288): every body zone moved rigidly
@@ -397,9 +411,10 @@ hipError_t update_body_zones(hipStream_t st, DevState& S, double m, double dt);
 // updateFinalForRG (dcollid.cpp:626-675)
 void launch_final_bodies(hipStream_t st, DevState& S, double dt);
 void launch_record_origin(hipStream_t st, DevState& S);
-void launch_average_velocity(hipStream_t st, DevState& S, double dt);
+// computeAverageVelocity and the per-vertex state of a resolve (union-find, zone
+// marks and, with record, the recorded impulses)
+void launch_average_velocity(hipStream_t st, DevState& S, double dt, bool record);
 void launch_predict(hipStream_t st, DevState& S, double dt);
-void launch_uf_init(hipStream_t st, DevState& S);
 hipError_t update_zones(hipStream_t st, DevState& S, double m, double dt, int nlist);
 void launch_domain_boundary(hipStream_t st, DevState& S, const double lo[3], const double hi[3],
                             double dt, double mu, double thickness);

@@ -40,12 +40,26 @@ __global__ void k_predict(dvec4* __restrict__ x, dvec4* __restrict__ x_old,
   x[v] = n;
 }
 
-// computeAverageVelocity (dcollid.cpp:160-220)
+// computeAverageVelocity (dcollid.cpp:160-220), makeSet (dcollid.cpp:1015-1031)
+// and createImpZoneForRG (dcollid3d.cpp:54-68): every point its own zone, every
+// movable body one zone rooted at its smallest vertex; the zone marks and (pimp
+// not null) the recorded impulses of the last resolve are cleared.
 __global__ void k_average_velocity(dvec4* __restrict__ x, const dvec4* __restrict__ x_old,
                                    dvec4* __restrict__ av, double dt, int nv,
+                                   int32_t* __restrict__ uf, const int32_t* __restrict__ vbody,
+                                   const int32_t* __restrict__ bptr,
+                                   const uint32_t* __restrict__ bmem, int32_t* __restrict__ zmark,
+                                   dvec4* __restrict__ pimp, int32_t* __restrict__ pnum,
                                    int* __restrict__ err) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= nv) return;
+  const int b = vbody ? vbody[v] : -1;
+  uf[v] = b >= 0 ? (int32_t)bmem[bptr[b]] : v;
+  zmark[v] = 0;
+  if (pimp) {
+    pimp[v] = dvec4{0.0, 0.0, 0.0, 0.0};
+    pnum[v] = 0;
+  }
   const dvec4 p = x[v], o = x_old[v];
   dvec4 a;
   if (dt > CS_ROUND_EPS) {
@@ -61,35 +75,7 @@ __global__ void k_average_velocity(dvec4* __restrict__ x, const dvec4* __restric
   x[v] = o;
 }
 
-// makeSet (dcollid.cpp:1015-1031) and createImpZoneForRG (dcollid3d.cpp:54-68):
-// every point its own zone, every movable body one zone rooted at its
-// smallest vertex
-__global__ void k_uf_init(int32_t* __restrict__ uf, const int32_t* __restrict__ vbody,
-                          const int32_t* __restrict__ bptr, const uint32_t* __restrict__ bmem,
-                          int nv) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= nv) return;
-  const int b = vbody ? vbody[v] : -1;
-  uf[v] = b >= 0 ? (int32_t)bmem[bptr[b]] : v;
-}
-
-// Sort key of a hit: (lo, hi, sub-test) packed as tightly as the element
-// count allows (hi in hb bits, the sub-test, at most 15, in 4 bits), which
-// keeps the order of the record key and needs fewer digit passes.
-__global__ void k_hit_keys(const hit_rec* __restrict__ hits, int n, int hb,
-                           uint64_t* __restrict__ keys, uint32_t* __restrict__ idx) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint64_t k = hits[i].key;
-  const uint64_t lo = k >> 36, hi = (k >> 8) & 0xFFFFFFFull, sub = k & 255u;
-  keys[i] = (((lo << hb) | hi) << 4) | sub;
-  idx[i] = (uint32_t)i;
-}
-
-// one record per (hit in canonical order, point): key = the vertex; the
-// body spreads of an all-rigid contact use the slots of points 0 and 1 with
-// key nv + body; points without a contribution get the sentinel nv + nbody
-// and sort last
+// one record per (hit in canonical order, point)
 __global__ void k_expand_records(const hit_rec* __restrict__ hits,
                                  const uint32_t* __restrict__ sorted_idx, int n, int nv, int nbody,
                                  uint32_t* __restrict__ rkey, uint32_t* __restrict__ rval) {
@@ -97,24 +83,54 @@ __global__ void k_expand_records(const hit_rec* __restrict__ hits,
   if (i >= 4 * n) return;
   const int r = i >> 2, p = i & 3;
   const uint32_t h = sorted_idx[r];
-  const int v = hits[h].v[p];
-  const int b = p < 2 ? hits[h].sb[p] : -1;
-  rkey[i] = (v >= 0) ? (uint32_t)v : (b >= 0 ? (uint32_t)(nv + b) : (uint32_t)(nv + nbody));
+  rkey[i] = hit_record_key(hits[h], p, nv, nbody);
   rval[i] = h * 4u + (uint32_t)p;
 }
+
+__device__ inline int uf_root(const int32_t* uf, int x) {
+  int p = uf[x];
+  while (p != x) {
+    x = p;
+    p = uf[x];
+  }
+  return x;
+}
+
+// sort keys of the zone members: (root << vbits) | vertex, so one sort
+// orders zones by root and members by ascending vertex id
+// (also resets the zone count, which k_zone_update fills after the sort)
+struct ZoneKeys {
+  const uint32_t* zlist;
+  int n, vbits;
+  const int32_t* uf;
+  uint64_t* key;
+  uint32_t* val;
+  int* zones;
+};
 
 // One thread per vertex segment of the sorted records.  The vertex joins the
 // list of vertices whose average velocity this pass changed (vcount counts
 // it; each vertex heads one segment).  A body segment (key nv + body) adds
 // its spreads to the body's collsnImpulse_RG in canonical order, starting
 // from the value it holds (the reference never clears it), and counts them.
+// The work-groups from `nba` on compute the zone members' sort keys.
 __global__ void k_apply(const uint32_t* __restrict__ rkey, const uint32_t* __restrict__ rval,
                         int nrec, int nv, int nbody, const hit_rec* __restrict__ hits,
                         dvec4* __restrict__ av, uint8_t* __restrict__ has,
                         dvec4* __restrict__ rg_imp, int32_t* __restrict__ rg_num,
                         int32_t* __restrict__ vlist, int* __restrict__ vcount,
                         dvec4* __restrict__ pimp, int32_t* __restrict__ pnum,
-                        int* __restrict__ err) {
+                        int* __restrict__ err, int nba, ZoneKeys Z) {
+  if ((int)blockIdx.x >= nba) {
+    const int i = (blockIdx.x - nba) * blockDim.x + threadIdx.x;
+    if (i == 0) *Z.zones = 0;
+    if (i >= Z.n) return;
+    const uint32_t v = Z.zlist[i];
+    const uint32_t r = (uint32_t)uf_root(Z.uf, (int)v);
+    Z.key[i] = ((uint64_t)r << Z.vbits) | v;
+    Z.val[i] = v;
+    return;
+  }
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t v = 0;
   bool head = false, bhead = false;
@@ -177,60 +193,47 @@ static int bits_for(uint64_t maxval) {  // bits needed for values <= maxval, rou
   return b < 8 ? 8 : b;
 }
 
-hipError_t apply_hits(hipStream_t st, DevState& S, int nhits, int* vcount, bool record) {
-  if (nhits <= 0) return hipSuccess;
-  if (record) {  // a pass with hits replaces the recorded impulses
-    CS_HIP_RET(hipMemsetAsync(S.pimp, 0, sizeof(dvec4) * (size_t)S.nv, st));
-    CS_HIP_RET(hipMemsetAsync(S.pnum, 0, sizeof(int32_t) * (size_t)S.nv, st));
+static int vertex_bits(const DevState& S) {
+  int b = 1;
+  while (b < 32 && ((uint64_t)(S.nv - 1) >> b) != 0) ++b;
+  return b;
+}
+
+hipError_t apply_hits(hipStream_t st, DevState& S, int nhits, int* vcount, bool record, int nzone) {
+  if (nhits <= 0 && nzone <= 0) return hipSuccess;
+  const uint32_t *rk = nullptr, *rv = nullptr;
+  const int nrec = 4 * std::max(nhits, 0);
+  if (nhits > 0) {
+    if (record) {  // a pass with hits replaces the recorded impulses
+      CS_HIP_RET(hipMemsetAsync(S.pimp, 0, sizeof(dvec4) * (size_t)S.nv, st));
+      CS_HIP_RET(hipMemsetAsync(S.pnum, 0, sizeof(int32_t) * (size_t)S.nv, st));
+    }
+    bool in_tmp = false;
+    if (nhits <= RANK_SORT_MAX) {
+      CS_HIP_RET(rank_hits(st, S.hkey, S.hits, nhits, S.nv, S.nbody, S.rkey, S.rval));
+    } else {
+      const int hb = hit_id_bits(S);
+      const int kbits = bits_for(((((uint64_t)S.ne << hb) | (uint64_t)S.ne) << 4) | 15u);
+      CS_HIP_RET(radix_sort_u64(st, S.hkey, S.hidx, S.hkey_tmp, S.hidx_tmp, S.sort_hist, S.scan_part,
+                                nhits, kbits, &in_tmp, true));
+      hipLaunchKernelGGL(k_expand_records, dim3((nrec + 255) / 256), dim3(256), 0, st, S.hits,
+                         in_tmp ? S.hidx_tmp : S.hidx, nhits, S.nv, S.nbody, S.rkey, S.rval);
+    }
+    CS_HIP_RET(radix_sort_u32(st, S.rkey, S.rval, S.rkey_tmp, S.rval_tmp, S.sort_hist, S.scan_part,
+                              nrec, bits_for((uint64_t)S.nv + (uint64_t)S.nbody), &in_tmp));
+    rk = in_tmp ? S.rkey_tmp : S.rkey;
+    rv = in_tmp ? S.rval_tmp : S.rval;
   }
-  const int nb = (nhits + 255) / 256;
-  int hb = 1;  // bits of an element id
-  while (hb < 32 && ((uint64_t)S.ne >> hb) != 0) ++hb;
-  hipLaunchKernelGGL(k_hit_keys, dim3(nb), dim3(256), 0, st, S.hits, nhits, hb, S.hkey, S.hidx);
-  bool in_tmp = false;
-  const int kbits = bits_for(((((uint64_t)S.ne << hb) | (uint64_t)S.ne) << 4) | 15u);
-  CS_HIP_RET(radix_sort_u64(st, S.hkey, S.hidx, S.hkey_tmp, S.hidx_tmp, S.sort_hist, S.scan_part, nhits, kbits,
-                            &in_tmp));
-  const uint32_t* sidx = in_tmp ? S.hidx_tmp : S.hidx;
-  const int nrec = 4 * nhits;
-  hipLaunchKernelGGL(k_expand_records, dim3((nrec + 255) / 256), dim3(256), 0, st, S.hits, sidx,
-                     nhits, S.nv, S.nbody, S.rkey, S.rval);
-  CS_HIP_RET(radix_sort_u32(st, S.rkey, S.rval, S.rkey_tmp, S.rval_tmp, S.sort_hist, S.scan_part, nrec,
-                            bits_for((uint64_t)S.nv + (uint64_t)S.nbody), &in_tmp));
-  const uint32_t* rk = in_tmp ? S.rkey_tmp : S.rkey;
-  const uint32_t* rv = in_tmp ? S.rval_tmp : S.rval;
-  hipLaunchKernelGGL(k_apply, dim3((nrec + 255) / 256), dim3(256), 0, st, rk, rv, nrec, S.nv,
+  const ZoneKeys Z{S.zlist, nzone, vertex_bits(S), S.uf, S.zkey64, S.zval, S.counters + CNT_ZONES};
+  const int nba = (nrec + 255) / 256, nbz = (std::max(nzone, 0) + 255) / 256;
+  hipLaunchKernelGGL(k_apply, dim3(nba + nbz), dim3(256), 0, st, rk, rv, nrec, S.nv,
                      S.nbody, S.hits, S.av, S.has, S.rg_imp, S.rg_num, S.vlist, vcount,
-                     record ? S.pimp : nullptr, S.pnum, S.counters + CNT_ERR);
+                     record ? S.pimp : nullptr, S.pnum, S.counters + CNT_ERR, nba, Z);
   return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
 // impact zones
-__device__ inline int uf_root(const int32_t* uf, int x) {
-  int p = uf[x];
-  while (p != x) {
-    x = p;
-    p = uf[x];
-  }
-  return x;
-}
-
-// sort keys of the zone members: (root << vbits) | vertex, so one sort
-// orders zones by root and members by ascending vertex id
-// (also resets the zone count, which k_zone_update fills after the sort)
-__global__ void k_zone_keys(const uint32_t* __restrict__ zlist, int n, const int32_t* __restrict__ uf,
-                            int vbits, uint64_t* __restrict__ key, uint32_t* __restrict__ val,
-                            int* __restrict__ counters) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) counters[CNT_ZONES] = 0;
-  if (i >= n) return;
-  const uint32_t v = zlist[i];
-  const uint32_t r = (uint32_t)uf_root(uf, (int)v);
-  key[i] = ((uint64_t)r << vbits) | v;
-  val[i] = v;
-}
-
 // updateImpactListVelocity (dcollid3d.cpp:70-200), one 64-lane wavefront per
 // zone.  Sums run in the canonical lane order: lane l adds the terms of
 // members l, l+64, ... (ascending vertex id) from 0.0, then the 64 lane sums
@@ -449,13 +452,10 @@ __global__ void __launch_bounds__(ZONE_LANES)
 // Every vertex of a zone with two or more members took part in a union, so
 // the union calls list the members as they go (zone_touch); only the listed
 // vertices are sorted, not the whole mesh.
+// (apply_hits left the members' keys)
 hipError_t update_zones(hipStream_t st, DevState& S, double m, double dt, int nlist) {
-  if (nlist <= 0) return hipMemsetAsync(S.counters + CNT_ZONES, 0, sizeof(int), st);  // no zones
-  const int nb = (nlist + 255) / 256;
-  int vbits = 1;
-  while (vbits < 32 && ((uint64_t)(S.nv - 1) >> vbits) != 0) ++vbits;
-  hipLaunchKernelGGL(k_zone_keys, dim3(nb), dim3(256), 0, st, S.zlist, nlist, S.uf, vbits,
-                     S.zkey64, S.zval, S.counters);
+  if (nlist <= 0) return hipSuccess;  // no zones (the list only grows during a step)
+  const int vbits = vertex_bits(S);
   bool in_tmp = false;
   CS_HIP_RET(radix_sort_u64(st, S.zkey64, S.zval, S.zkey64_tmp, S.zval_tmp, S.sort_hist,
                             S.scan_part, nlist, bits_for(((uint64_t)(S.nv - 1) << vbits) | (uint64_t)(S.nv - 1)),
@@ -735,14 +735,10 @@ void launch_predict(hipStream_t st, DevState& S, double dt) {
                      dt, S.nv);
 }
 
-void launch_average_velocity(hipStream_t st, DevState& S, double dt) {
+void launch_average_velocity(hipStream_t st, DevState& S, double dt, bool record) {
   hipLaunchKernelGGL(k_average_velocity, dim3((S.nv + 255) / 256), dim3(256), 0, st, S.x, S.x_old,
-                     S.av, dt, S.nv, S.counters + CNT_ERR);
-}
-
-void launch_uf_init(hipStream_t st, DevState& S) {
-  hipLaunchKernelGGL(k_uf_init, dim3((S.nv + 255) / 256), dim3(256), 0, st, S.uf, S.vbody, S.bptr,
-                     S.bmem, S.nv);
+                     S.av, dt, S.nv, S.uf, S.vbody, S.bptr, S.bmem, S.zmark,
+                     record ? S.pimp : nullptr, S.pnum, S.counters + CNT_ERR);
 }
 
 // ---------------------------------------------------------------------------
