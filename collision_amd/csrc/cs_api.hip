@@ -95,6 +95,9 @@ struct cs_solver {
   size_t ev_used = 0;
   PrevPass prev;
   SeedPairs seed;
+  // pairs of the last full traversal (-1: none yet) of a proximity / a CCD pass:
+  // the narrow phase's grid for the next
+  int64_t pair_guess[2] = {-1, -1};
   int64_t syncs = 0;  // host synchronisations of the current resolve
   LearnedState L;           // time-of-impact proposer (learned form)
   cs_learned_stats lstats{};  // its statistics since the last cs_learned_get_stats
@@ -317,8 +320,8 @@ float elapsed(hipEvent_t a, hipEvent_t b) {
 }
 
 int read_counters(cs_solver* h) {
-  HIPCHK(h, hipMemcpyAsync(h->h_counters, h->S.counters, sizeof(int) * COUNTER_INTS,
-                           hipMemcpyDeviceToHost, h->st));
+  launch_report(h->st, h->S, h->h_counters);
+  HIPCHK(h, hipGetLastError());
   HIPCHK(h, hipStreamSynchronize(h->st));
   h->syncs++;
   return CS_OK;
@@ -478,13 +481,44 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
     else launch_element_boxes(h->st, S, P.dt, ccd ? nullptr : S.ebox, ccd ? S.ebox : nullptr);
     if (kind == CS_PASS_PROXIMITY) HIPCHK(h, build_bvh(h->st, S));
     HIPCHK(h, refit_bvh(h->st, S));
-    for (;;) {  // traversal; re-run with a larger stream if it overflowed
+    // One host synchronisation per pass: the narrow phase (and the split of a
+    // dual stream) reads the number of pairs from device memory, on a grid for a
+    // guess of it; an overflow is seen afterwards, when nothing has been tested,
+    // and pairs beyond the guess are handled once the count is known.  (The
+    // learned form sorts its stream and waits for the count first.)
+    const bool wait = ccd && P.learned;
+    const int2* stream = S.pairs;
+    const int* stream_dev = S.counters + (dual ? CNT_PPAIRS : CNT_PAIRS);
+    int64_t& last = h->pair_guess[ccd];
+    int rc;
+    int64_t guess = 0;
+    for (;;) {
+      guess = last < 0 ? S.ne : last + last / 4;
+      guess = std::min<int64_t>(S.pair_cap, std::max<int64_t>(4096, guess));
       mark_pass(h, &T.t0, 1);
-      launch_traverse(h->st, S, dual ? S.pairs_seed : S.pairs, S.pair_cap, dual ? S.pbox : nullptr);
+      launch_traverse(h->st, S, dual ? S.pairs_seed : S.pairs, S.pair_cap, dual ? S.pbox : nullptr,
+                      kind == CS_PASS_PROXIMITY);
       mark_pass(h, &T.t1, 1);
-      HIPCHK(h, hipGetLastError());
-      int rc = read_counters(h);
-      if (rc) return rc;
+      if (wait) {
+        HIPCHK(h, hipGetLastError());
+        if ((rc = read_counters(h))) return rc;
+        guess = std::min(h->h_counters[CNT_PAIRS], S.pair_cap);
+      }
+      if (dual) launch_split_seed(h->st, S, 0, (int)guess);
+      mark_pass(h, &T.e1, 2);
+      stream = S.pairs;
+      if (!wait || h->h_counters[CNT_PAIRS] <= S.pair_cap) {
+        mark_pass(h, &T.n0, 1);
+        HIPCHK(h, narrow_call(h, NP, stream, (int)guess, wait ? nullptr : stream_dev, S.pair_cap));
+        mark_pass(h, &T.n1, 1);
+        HIPCHK(h, hipGetLastError());
+        if ((rc = read_counters(h))) return rc;
+      }
+      // a non-finite average velocity ends the step before any pass, where the
+      // reference calls clean_up(ERROR) (dcollid.cpp:178-184); the traversal
+      // found no pairs then
+      if (kind == CS_PASS_PROXIMITY && (h->h_counters[CNT_ERR] & CS_DEVERR_START))
+        return device_error(h);
       npairs = h->h_counters[CNT_PAIRS];
       if (npairs <= S.pair_cap) break;
       S.pair_cap = (int)std::min<int64_t>((int64_t)npairs + npairs / 4 + 1024, INT32_MAX / 2);
@@ -496,37 +530,45 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
       HIPCHK(h, hipMemsetAsync(S.counters + CNT_CAND64, 0, 2 * sizeof(int), h->st));
       HIPCHK(h, hipMemsetAsync(S.counters + CNT_PCAND64, 0, 2 * sizeof(int), h->st));
       HIPCHK(h, hipMemsetAsync(S.counters + CNT_TSPLIT, 0, 2 * sizeof(int), h->st));
+      last = npairs;
     }
+    last = npairs;
     cand = c64(h, CNT_CAND64);
-    const int2* stream = S.pairs;
-    const int* stream_dev = nullptr;
     if (dual) {
-      // this pass's pairs are the flagged ones; their number is read on the
-      // device by the narrow phase (at most npairs)
       h->seed.valid = true;
       h->seed.npairs = npairs;
       h->seed.cand = cand;
-      launch_split_seed(h->st, S, npairs);
-      stream_dev = S.counters + CNT_PPAIRS;
     }
-    mark_pass(h, &T.e1, 2);
-    for (;;) {
-      mark_pass(h, &T.n0, 1);
-      HIPCHK(h, narrow_call(h, NP, stream, npairs, stream_dev, S.pair_cap));
+    if (npairs > guess) {  // the rest of the stream
+      int done = (int)guess;
+      if (dual) {
+        done = h->h_counters[CNT_PPAIRS];
+        launch_split_seed(h->st, S, (int)guess, npairs);
+        HIPCHK(h, hipGetLastError());
+        if ((rc = read_counters(h))) return rc;
+      }
+      const int all = dual ? h->h_counters[CNT_PPAIRS] : npairs;
+      HIPCHK(h, narrow_call(h, NP, stream + done, all - done, nullptr, 0));
       mark_pass(h, &T.n1, 1);
       HIPCHK(h, hipGetLastError());
-      int rc = read_counters(h);
-      if (rc) return rc;
+      if ((rc = read_counters(h))) return rc;
+    }
+    if (dual) {  // this pass's pairs are the flagged ones
+      npairs = h->h_counters[CNT_PPAIRS];
+      cand = c64(h, CNT_PCAND64);
+    }
+    for (;;) {
       nhits = h->h_counters[CNT_HITS];
       nhp = h->h_counters[CNT_HIT_PAIRS];
       if (nhits <= S.hit_cap && nhp <= S.hp_cap) break;
       HIPCHK(h, grow_hit_buffers(h, nhits, nhp, 0, 0));
       if ((rc = set_counter(h, CNT_HITS, 0))) return rc;
       if ((rc = set_counter(h, CNT_HIT_PAIRS, 0))) return rc;
-    }
-    if (dual) {  // (counted by the split, read with the narrow phase's counters)
-      npairs = h->h_counters[CNT_PPAIRS];
-      cand = c64(h, CNT_PCAND64);
+      mark_pass(h, &T.n0, 1);
+      HIPCHK(h, narrow_call(h, NP, stream, npairs, nullptr, 0));
+      mark_pass(h, &T.n1, 1);
+      HIPCHK(h, hipGetLastError());
+      if ((rc = read_counters(h))) return rc;
     }
     narrow_n = npairs;
   } else if (seeded) {
@@ -536,53 +578,67 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
     // (the proximity pass ran another test), so every pair is tested.
     launch_mark_dirty(h->st, S, vcount_prev, 0);
     mark_pass(h, &T.t0, 1);
-    if (exact_counts) launch_query_dirty(h->st, S, 0, 0);  // seed boxes: count only
+    if (exact_counts) launch_query_dirty(h->st, S, 0, 0, CNT_QPAIRS, 1);  // seed boxes: count only
     launch_grow_carry(h->st, S, P.dt, 0, 0, 0);  // new boxes; leaves exact, ancestors grown
-    launch_query_dirty(h->st, S, 1, 0);
+    launch_query_dirty(h->st, S, 1, 0, CNT_PAIRS, exact_counts);
     mark_pass(h, &T.t1, 1);
     launch_carry_pairs_from(h->st, S, S.pairs_seed, seed.npairs);
+    mark_pass(h, &T.e1, 2);
+    // one host synchronisation, as in the full pass
+    const bool wait = P.learned != 0;
+    int rc;
+    int64_t guess = 0;
     for (int attempt = 0;; ++attempt) {
-      int rc = read_counters(h);
-      if (rc) return rc;
-      nq = h->h_counters[CNT_QPAIRS];
-      if (nq <= S.qpair_cap) break;
+      guess = std::min<int64_t>(S.pair_cap, (int64_t)seed.npairs + seed.npairs / 4 + 4096);
+      if (wait) {
+        HIPCHK(h, hipGetLastError());
+        if ((rc = read_counters(h))) return rc;
+        guess = std::min(h->h_counters[CNT_PAIRS], S.pair_cap);
+      }
+      if (!wait || h->h_counters[CNT_PAIRS] <= S.pair_cap) {
+        mark_pass(h, &T.n0, 1);
+        HIPCHK(h, narrow_call(h, NP, S.pairs, (int)guess, wait ? nullptr : S.counters + CNT_PAIRS,
+                              S.pair_cap));
+        mark_pass(h, &T.n1, 1);
+        HIPCHK(h, hipGetLastError());
+        if ((rc = read_counters(h))) return rc;
+      }
+      npairs = h->h_counters[CNT_PAIRS];
+      if (npairs <= S.pair_cap) break;
       if (attempt > 4) return fail(h, CS_ERR_INTERNAL, "query stream keeps overflowing");
-      S.qpair_cap = nq + nq / 2 + 1024;
-      dfree(S.qpairs);
-      HIPCHK(h, dalloc(&S.qpairs, S.qpair_cap));
-      HIPCHK(h, hipMemsetAsync(S.counters + CNT_QPAIRS, 0, sizeof(int), h->st));
-      HIPCHK(h, hipMemsetAsync(S.counters + CNT_NEW64, 0, 2 * sizeof(int), h->st));
-      launch_query_dirty(h->st, S, 1, 0);
-    }
-    carried_pairs = h->h_counters[CNT_PAIRS];
-    npairs = carried_pairs + nq;
-    if (npairs > S.pair_cap) {
       const int cap = (int)std::min<int64_t>((int64_t)npairs + npairs / 4 + 1024, INT32_MAX / 2);
-      HIPCHK(h, grow_keep(&S.pairs, carried_pairs, cap, h->st));
+      HIPCHK(h, grow_keep(&S.pairs, 0, cap, h->st));
       dfree(S.pairs_prev);
       HIPCHK(h, dalloc(&S.pairs_prev, cap));
-      HIPCHK(h, grow_keep(&S.pairs_seed, 0, cap, h->st));
+      HIPCHK(h, grow_keep(&S.pairs_seed, seed.npairs, cap, h->st));
       S.pair_cap = cap;
+      HIPCHK(h, hipMemsetAsync(S.counters + CNT_PAIRS, 0, sizeof(int), h->st));
+      HIPCHK(h, hipMemsetAsync(S.counters + CNT_QPAIRS, 0, sizeof(int), h->st));
+      HIPCHK(h, hipMemsetAsync(S.counters + CNT_NEW64, 0, 2 * sizeof(int), h->st));
+      launch_query_dirty(h->st, S, 1, 0, CNT_PAIRS, exact_counts);
+      launch_carry_pairs_from(h->st, S, S.pairs_seed, seed.npairs);
     }
-    if (nq > 0)
-      HIPCHK(h, hipMemcpyAsync(S.pairs + carried_pairs, S.qpairs, sizeof(int2) * (size_t)nq,
-                               hipMemcpyDeviceToDevice, h->st));
-    cand = exact_counts ? seed.cand - c64(h, CNT_OLD64) + c64(h, CNT_NEW64) : ~0ull;
-    mark_pass(h, &T.e1, 2);
-    narrow_n = npairs;
-    for (;;) {
-      mark_pass(h, &T.n0, 1);
-      HIPCHK(h, narrow_call(h, NP, S.pairs, npairs, nullptr, 0));
+    nq = h->h_counters[CNT_QPAIRS];
+    if (npairs > guess) {  // the rest of the stream
+      HIPCHK(h, narrow_call(h, NP, S.pairs + guess, npairs - (int)guess, nullptr, 0));
       mark_pass(h, &T.n1, 1);
       HIPCHK(h, hipGetLastError());
-      int rc = read_counters(h);
-      if (rc) return rc;
+      if ((rc = read_counters(h))) return rc;
+    }
+    cand = exact_counts ? seed.cand - c64(h, CNT_OLD64) + c64(h, CNT_NEW64) : ~0ull;
+    narrow_n = npairs;
+    for (;;) {
       nhits = h->h_counters[CNT_HITS];
       nhp = h->h_counters[CNT_HIT_PAIRS];
       if (nhits <= S.hit_cap && nhp <= S.hp_cap) break;
       HIPCHK(h, grow_hit_buffers(h, nhits, nhp, 0, 0));
       if ((rc = set_counter(h, CNT_HITS, 0))) return rc;
       if ((rc = set_counter(h, CNT_HIT_PAIRS, 0))) return rc;
+      mark_pass(h, &T.n0, 1);
+      HIPCHK(h, narrow_call(h, NP, S.pairs, npairs, nullptr, 0));
+      mark_pass(h, &T.n1, 1);
+      HIPCHK(h, hipGetLastError());
+      if ((rc = read_counters(h))) return rc;
     }
   } else {
     // One host synchronisation per pass: the narrow phase reads the number
@@ -596,13 +652,13 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
     // previous boxes: count only.  The count only feeds the exact candidate
     // total of the pass (a diagnostic), so it runs when the caller asks for
     // the parity taps; otherwise the candidate total is reported as -1.
-    if (exact_counts) launch_query_dirty(h->st, S, 0, 0);
+    if (exact_counts) launch_query_dirty(h->st, S, 0, 0, CNT_QPAIRS, 1);
     // new boxes (leaves exact, ancestors grown); hits and hit pairs carried over
     launch_grow_carry(h->st, S, P.dt, prev.nhits, prev.nhp, kind == CS_PASS_ZONE);
     // the candidate pair stream itself only feeds the exact pair count of the
     // pass; it is carried when the caller asks for exact counts
     if (exact_counts) launch_carry_pairs_from(h->st, S, S.pairs_prev, prev.npairs);
-    launch_query_dirty(h->st, S, 1, 1);  // current boxes: count + emit
+    launch_query_dirty(h->st, S, 1, 1, CNT_QPAIRS, exact_counts);  // current boxes: count + emit
     mark_pass(h, &T.t1, 1);
     mark_pass(h, &T.e1, 2);
     // grid for a guess of the re-queried pair count; pairs beyond it are
@@ -636,7 +692,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
         HIPCHK(h, dalloc(&S.qpairs, S.qpair_cap));
         HIPCHK(h, hipMemsetAsync(S.counters + CNT_QPAIRS, 0, sizeof(int), h->st));
         HIPCHK(h, hipMemsetAsync(S.counters + CNT_NEW64, 0, 2 * sizeof(int), h->st));
-        launch_query_dirty(h->st, S, 1, 0);
+        launch_query_dirty(h->st, S, 1, 0, CNT_QPAIRS, exact_counts);
       }
       HIPCHK(h, grow_hit_buffers(h, nhits, nhp, carried_hits, carried_hp));
       if ((rc = set_counter(h, CNT_HITS, carried_hits))) return rc;
@@ -1147,6 +1203,7 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   HIPCHK(h, dalloc(&S.krmin, std::max(ne - 1, 1))); HIPCHK(h, dalloc(&S.krmax, std::max(ne - 1, 1)));
   HIPCHK(h, dalloc(&S.split_right, std::max(ne - 1, 1)));
   HIPCHK(h, dalloc(&S.tbox, 6 * refit_tile_count(ne))); HIPCHK(h, dalloc(&S.top, std::max(ne - 1, 1)));
+  h->pair_guess[0] = h->pair_guess[1] = -1;
   S.pair_cap = (int)std::min<int64_t>(3ll * ne + 4096, INT32_MAX / 2);
   HIPCHK(h, dalloc(&S.pairs, S.pair_cap));
   HIPCHK(h, dalloc(&S.pairs_prev, S.pair_cap));
@@ -1479,12 +1536,8 @@ int resolve_impl(cs_solver* h, cs_step_report* report, bool with_predict_graph) 
   int pass_id = 0;
   bool any = false;
   int status = CS_OK;
-  // a non-finite average velocity ends the step before any pass, where the
-  // reference calls clean_up(ERROR) (dcollid.cpp:178-184)
-  if ((rc = read_counters(h))) return rc;
-  if (h->h_counters[CNT_ERR]) status = device_error(h);
   // detectProximity (dcollid.cpp:390-406)
-  if (!status) {
+  {
     rc = run_pass(h, CS_PASS_PROXIMITY, 0, pass_id++, &any);
     if (rc) status = rc;
   }

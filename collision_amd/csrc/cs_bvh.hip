@@ -498,6 +498,7 @@ struct TravArgs {
   TravItem* qout;  // where long walks go (null: they walk on)
   int* qout_n;
   int qcap;
+  const int* err;  // not null: no walk when the flag is set
 };
 
 struct Walk {
@@ -626,6 +627,7 @@ __device__ inline void walk_element(const TravArgs& A, Walk& w) {
 template <bool DUAL>
 __global__ void __launch_bounds__(TRAV_THREADS) k_traverse(TravArgs A, int lsub) {
   __shared__ int2 buf[TRAV_BUF * TRAV_THREADS];
+  if (A.err && *A.err) return;
   const int nnodes = 2 * A.n - 1;
   const int64_t nw = (int64_t)A.n << lsub;  // walks
   WalkOut o;
@@ -696,13 +698,18 @@ __global__ void __launch_bounds__(TRAV_THREADS) k_traverse_split(TravArgs A,
 constexpr int SPLIT_ITEMS = 16;
 constexpr int SPLIT_TILE = 256 * SPLIT_ITEMS;
 __global__ void __launch_bounds__(256) k_split_seed(const int2* __restrict__ seed, int n,
+                                                    int first, int cap,
                                                     const dbox* __restrict__ pbox,
                                                     int2* __restrict__ prox,
                                                     int* __restrict__ counters) {
   __shared__ int s_off[256];
   __shared__ int s_base;
   const int t = threadIdx.x;
-  const int base_i = blockIdx.x * SPLIT_TILE;
+  const int total = counters[CNT_PAIRS];
+  if (total > cap) return;  // the stream overflowed: it is walked again
+  n = min(n, total);
+  const int base_i = first + blockIdx.x * SPLIT_TILE;
+  if (base_i >= n) return;
   int2 p[SPLIT_ITEMS];
   uint32_t keep = 0u;
 #pragma unroll
@@ -917,8 +924,17 @@ __device__ inline void grow_dirty(const GrowArgs& G, int nd, int block, int bloc
 constexpr int QW_FCAP = 1024;  // frontier nodes of one level
 constexpr int QW_LCAP = 1024;  // leaves collected by one range
 
+// advances the length of the query's own stream, or (count CNT_PAIRS) that of the
+// pair stream and with it the query's count
+__device__ inline int add_pairs(int* __restrict__ counters, int count, int n) {
+  if (count == CNT_QPAIRS) return atomicAdd(&counters[CNT_QPAIRS], n);
+  static_assert(CNT_PAIRS % 2 == 0 && CNT_QPAIRS == CNT_PAIRS + 1, "one 64-bit word");
+  return (int)(uint32_t)atomicAdd((unsigned long long*)&counters[CNT_PAIRS],
+                                  (unsigned long long)n | (unsigned long long)n << 32);
+}
+
 __device__ inline void flush_pairs(int2* buf, int nbuf, int2* __restrict__ qpairs, int qcap,
-                                   int* __restrict__ counters) {
+                                   int* __restrict__ counters, int count) {
   // exclusive scan of nbuf over the wavefront, one atomic per wavefront
   const int lane = threadIdx.x & 63;
   int incl = nbuf;
@@ -930,7 +946,7 @@ __device__ inline void flush_pairs(int2* buf, int nbuf, int2* __restrict__ qpair
   const int total = __shfl(incl, 63);
   if (total == 0) return;
   int base = 0;
-  if (lane == 63) base = atomicAdd(&counters[CNT_QPAIRS], total);
+  if (lane == 63) base = add_pairs(counters, count, total);
   base = __shfl(base, 63) + incl - nbuf;
   for (int q = 0; q < nbuf; ++q)
     if (base + q < qcap) qpairs[base + q] = buf[q * 64 + lane];
@@ -941,8 +957,8 @@ __global__ void __launch_bounds__(64) k_query_ranges(
     const dbox* __restrict__ ebox, const int4* __restrict__ ev,
     const uint8_t* __restrict__ eflags, const uint8_t* __restrict__ dirty_e,
     const uint8_t* __restrict__ dpre, const int32_t* __restrict__ rlist, int npre, int emit,
-    int scenes, int snap,
-    int2* __restrict__ qpairs, int qcap, int* __restrict__ counters) {
+    int scenes, int snap, int exact,
+    int2* __restrict__ qpairs, int qcap, int count, int* __restrict__ counters) {
   __shared__ int32_t fr[2][QW_FCAP];
   __shared__ int2 lv[QW_LCAP];  // (pre-order index, element)
   // the range's dirty elements (the queries), compacted: box and pre-order
@@ -1053,7 +1069,7 @@ __global__ void __launch_bounds__(64) k_query_ranges(
         buf[nbuf * 64 + lane] = pr;
         ++nbuf;
       } else {
-        const int slot = atomicAdd(&counters[CNT_QPAIRS], 1);
+        const int slot = add_pairs(counters, count, 1);
         if (slot < qcap) qpairs[slot] = pr;
       }
     };
@@ -1128,13 +1144,14 @@ __global__ void __launch_bounds__(64) k_query_ranges(
         take(e, mt, mf, e2, ev[e2], eflags[e2]);
       }
     }
-    if (emit) flush_pairs(buf, nbuf, qpairs, qcap, counters);
+    if (emit) flush_pairs(buf, nbuf, qpairs, qcap, counters, count);
     __syncthreads();
   }
   unsigned long long c = cand;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-  if (lane == 0 && c) atomicAdd((unsigned long long*)(counters + (emit ? CNT_NEW64 : CNT_OLD64)), c);
+  if (exact && lane == 0 && c)
+    atomicAdd((unsigned long long*)(counters + (emit ? CNT_NEW64 : CNT_OLD64)), c);
 }
 
 // Start of a pass (or of a step): clears the dirty marks that the previous pass
@@ -1291,12 +1308,13 @@ void launch_grow_carry(hipStream_t st, DevState& S, double dt, int nhits_prev, i
                      st, G, C, bh, bp, S.counters);
 }
 
-void launch_query_dirty(hipStream_t st, DevState& S, int emit, int snap) {
+void launch_query_dirty(hipStream_t st, DevState& S, int emit, int snap, int count, int exact) {
   if (S.ne < 2) return;
   const int npre = 2 * S.ne - 1;
   hipLaunchKernelGGL(k_query_ranges, dim3(std::min((npre + 63) / 64, S.tune_query)), dim3(64), 0, st,
                      S.nodes, S.nright, S.ebox, S.ev, S.eflags, S.dirty_e, S.dpre, S.rlist, npre,
-                     emit, S.nscene > 1, snap, S.qpairs, S.qpair_cap, S.counters);
+                     emit, S.nscene > 1, snap, exact, count == CNT_PAIRS ? S.pairs : S.qpairs,
+                     count == CNT_PAIRS ? S.pair_cap : S.qpair_cap, count, S.counters);
 }
 
 void launch_carry_pairs_from(hipStream_t st, DevState& S, const int2* src, int n) {
@@ -1365,7 +1383,8 @@ hipError_t refit_bvh(hipStream_t st, DevState& S) {
 size_t refit_tile_count(int n) { return (size_t)(n + REFIT_TILE - 1) / REFIT_TILE; }
 
 // (the caller has zeroed the item counts of the split rounds, CNT_TSPLIT)
-void launch_traverse(hipStream_t st, DevState& S, int2* out, int cap, const dbox* pbox) {
+void launch_traverse(hipStream_t st, DevState& S, int2* out, int cap, const dbox* pbox,
+                     bool check) {
   const int n = S.ne;
   if (n < 2) return;
   int lsub = 0;
@@ -1378,14 +1397,20 @@ void launch_traverse(hipStream_t st, DevState& S, int2* out, int cap, const dbox
   int* n0 = S.counters + CNT_TSPLIT;
   TravArgs A{S.nodes, S.lpre, S.ebox, pbox, S.ev, S.eflags, n, S.nscene > 1, out, cap,
              S.counters + CNT_PAIRS, (unsigned long long*)(S.counters + CNT_CAND64),
-             (unsigned long long*)(S.counters + CNT_PCAND64), q0, n0, TRAV_QCAP};
+             (unsigned long long*)(S.counters + CNT_PCAND64), q0, n0, TRAV_QCAP,
+             check ? S.counters + CNT_ERR : nullptr};
   TravArgs A1 = A, A2 = A;
   A1.qout = q1;
   A1.qout_n = n0 + 1;
   A2.qout = nullptr;
   A2.qout_n = nullptr;
+  // where a share of the tree has no more nodes than a walk may take, no walk is
+  // handed over and the rounds for them are not launched (up to 4,032 elements)
+  const bool rounds = ((2 * (int64_t)n) >> lsub) + 1 > TRAV_LONG;
+  if (!rounds) A.qout = nullptr;
   auto go = [&](auto main, auto split) {
     hipLaunchKernelGGL(main, dim3(blocks), dim3(TRAV_THREADS), 0, st, A, lsub);
+    if (!rounds) return;
     hipLaunchKernelGGL(split, dim3(4 * S.num_cus), dim3(TRAV_THREADS), 0, st, A1,
                        (const TravItem*)q0, (const int*)n0);
     hipLaunchKernelGGL(split, dim3(4 * S.num_cus), dim3(TRAV_THREADS), 0, st, A2,
@@ -1395,10 +1420,10 @@ void launch_traverse(hipStream_t st, DevState& S, int2* out, int cap, const dbox
   else go(k_traverse<false>, k_traverse_split<false>);
 }
 
-void launch_split_seed(hipStream_t st, DevState& S, int n) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_split_seed, dim3((n + SPLIT_TILE - 1) / SPLIT_TILE), dim3(256), 0, st,
-                     S.pairs_seed, n, S.pbox, S.pairs, S.counters);
+void launch_split_seed(hipStream_t st, DevState& S, int first, int n) {
+  if (n <= first) return;
+  hipLaunchKernelGGL(k_split_seed, dim3((n - first + SPLIT_TILE - 1) / SPLIT_TILE), dim3(256), 0, st,
+                     S.pairs_seed, n, first, S.pair_cap, S.pbox, S.pairs, S.counters);
 }
 
 }  // namespace cs

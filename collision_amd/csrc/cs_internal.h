@@ -23,18 +23,20 @@ enum : uint8_t { EF_TRI = 1, EF_RIGID = 2 };
 enum : int {
   CS_DEVERR_NONFINITE = 1,   // where the reference calls clean_up(ERROR)
   CS_DEVERR_STRAIN = 4,      // strain-limit schedule inconsistency
+  CS_DEVERR_START = 8,       // (with NONFINITE) found before the first pass
 };
 
 // slots of the small device counter block (ints; 64-bit counts at 16..21)
 enum {
   CNT_PAIRS = 0,         // pairs in the candidate stream being built
-  CNT_TICKET = 1,        // work-groups of launch_pass_begin that are done
+  CNT_QPAIRS = 1,        // pairs found by the dirty-element query (the next index: where
+                         // they join the pair stream, both advance in one 64-bit add)
   CNT_HITS = 2,          // hit records (an even index: the narrow phase adds to
   CNT_HIT_PAIRS = 3,     // both in one 64-bit add); pairs with at least one hit
   CNT_LOG = 4,           // pair-log rows
   CNT_TMP = 5,           // LBVH nodes spanning refit tiles
   CNT_ZONES = 6,         // impact zones updated
-  CNT_QPAIRS = 7,        // pairs found by the dirty-element query
+  CNT_TICKET = 7,        // work-groups of launch_pass_begin that are done
   CNT_STRAIN_FLAG = 8,   // strain sweep state
   CNT_STRAIN_EDGES = 9,
   CNT_STRAIN_DEGEN = 10,
@@ -286,6 +288,8 @@ enum {
   SCN_FIELDS
 };
 void launch_scene_reset(hipStream_t st, DevState& S);
+// the counters into (pinned) host memory
+void launch_report(hipStream_t st, DevState& S, int* host);
 void launch_fill_u32(hipStream_t st, void* p, int64_t words, uint32_t v);
 // after a pass's narrow phase: scene of each of its nhp hit pairs, then the
 // per-scene state machine of the reference's pass loop
@@ -359,10 +363,12 @@ constexpr int BOUNDS_FLOATS = 6 * 128;  // rows of k_bounds
 // candidate pairs of the current boxes (ebox) into out; with pbox (static
 // boxes, each inside its element's swept box in ebox), also the static-box
 // overlaps among the rejected pairs (CNT_PCAND64)
-void launch_traverse(hipStream_t st, DevState& S, int2* out, int cap, const dbox* pbox);
-// the pairs of S.pairs_seed[0..n) whose static boxes overlap into S.pairs
-// (count CNT_PPAIRS, also added to CNT_PCAND64)
-void launch_split_seed(hipStream_t st, DevState& S, int n);
+void launch_traverse(hipStream_t st, DevState& S, int2* out, int cap, const dbox* pbox,
+                     bool check);
+// the pairs of S.pairs_seed[first..n) (at most the CNT_PAIRS found; none if those
+// overflowed the stream) whose static boxes overlap into S.pairs (count
+// CNT_PPAIRS, also added to CNT_PCAND64)
+void launch_split_seed(hipStream_t st, DevState& S, int first, int n);
 // incremental passes
 // elements of the vertices the previous pass changed: *vcount hit vertices
 // in vlist and nzone zone members in zlist
@@ -371,8 +377,10 @@ void launch_mark_dirty(hipStream_t st, DevState& S, const int* vcount, int nzone
 void launch_pass_begin(hipStream_t st, DevState& S, uint64_t mask);
 constexpr int QW_RANGE_SHIFT = 3;
 constexpr int QW_RANGE = 1 << QW_RANGE_SHIFT;  // pre-order nodes per dirty-query range
-// snap: the counts carried into the pass are kept in CNT_SNAP..
-void launch_query_dirty(hipStream_t st, DevState& S, int emit, int snap);
+// snap: the counts carried into the pass are kept in CNT_SNAP..; count: the
+// stream that the pairs join, CNT_QPAIRS (S.qpairs) or CNT_PAIRS (S.pairs); exact:
+// the candidates are counted (CNT_OLD64 / CNT_NEW64)
+void launch_query_dirty(hipStream_t st, DevState& S, int emit, int snap, int count, int exact);
 // the dirty elements' new swept boxes, their leaves exact and ancestors grown;
 // the previous pass's clean hits and hit pairs (zone: with their zone merges)
 void launch_grow_carry(hipStream_t st, DevState& S, double dt, int nhits_prev, int nhp_prev,

@@ -974,7 +974,12 @@ __global__ void __launch_bounds__(THREADS, 3)
              const dvec4* __restrict__ av, const uint8_t* __restrict__ fixed, NarrowParams P,
              ZoneList Z, hit_rec* __restrict__ hits, int hit_cap, int4* __restrict__ hp,
              int hp_cap, int* __restrict__ counters) {
-  const int n = npairs_dev ? min(min(*npairs_dev, cap), npairs) : npairs;
+  int n = npairs;
+  if (npairs_dev) {
+    const int found = *npairs_dev;
+    if (found > cap) return;  // the stream overflowed: it is filled and tested again
+    n = min(found, npairs);
+  }
   // XCD-contiguous shares of the pairs: the hardware deals work-groups to the
   // 8 XCDs round-robin, so the first `busy` of them (those the pair count
   // needs; with a count read on the device the grid may be larger) are spread

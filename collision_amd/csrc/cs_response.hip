@@ -70,7 +70,8 @@ __global__ void k_average_velocity(dvec4* __restrict__ x, const dvec4* __restric
     a.x = a.y = a.z = 0.0;
   }
   a.w = 0.0;
-  if (!isfinite(a.x) || !isfinite(a.y) || !isfinite(a.z)) atomicOr(err, CS_DEVERR_NONFINITE);
+  if (!isfinite(a.x) || !isfinite(a.y) || !isfinite(a.z))
+    atomicOr(err, CS_DEVERR_NONFINITE | CS_DEVERR_START);
   av[v] = a;
   x[v] = o;
 }
@@ -728,6 +729,15 @@ void launch_fill_u32(hipStream_t st, void* p, int64_t words, uint32_t v) {
   if (words <= 0) return;
   const int64_t blocks = std::min<int64_t>((words + 255) / 256, 4096);
   hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)blocks), dim3(256), 0, st, (uint32_t*)p, words, v);
+}
+
+// A kernel rather than a copy command: one launch before a synchronisation.
+__global__ void k_report(const int* __restrict__ counters, int* __restrict__ host) {
+  if (threadIdx.x < CNT_INTS) host[threadIdx.x] = counters[threadIdx.x];
+}
+
+void launch_report(hipStream_t st, DevState& S, int* host) {
+  hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, st, S.counters, host);
 }
 
 void launch_predict(hipStream_t st, DevState& S, double dt) {
