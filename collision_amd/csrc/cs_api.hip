@@ -98,6 +98,7 @@ struct cs_solver {
   // pairs of the last full traversal (-1: none yet) of a proximity / a CCD pass:
   // the narrow phase's grid for the next
   int64_t pair_guess[2] = {-1, -1};
+  unsigned report_seq = 0;  // of the last report of the counters
   int64_t syncs = 0;  // host synchronisations of the current resolve
   LearnedState L;           // time-of-impact proposer (learned form)
   cs_learned_stats lstats{};  // its statistics since the last cs_learned_get_stats
@@ -319,11 +320,25 @@ float elapsed(hipEvent_t a, hipEvent_t b) {
   return 0.f;
 }
 
-int read_counters(cs_solver* h) {
-  launch_report(h->st, h->S, h->h_counters);
+// Counters of everything launched so far.  Within a step the host polls the
+// sequence number that the report writes behind them, which it sees some
+// microseconds before the stream's completion signal (a workload's pass over a
+// 256 x 256 drape, 33 waits per step, 14.97 -> 14.21 ms, over strings 2.79 ->
+// 2.63 ms); the stream is queried now and then, so that an error on it ends
+// the wait.
+int read_counters(cs_solver* h, bool whole_stream = false) {
+  const int seq = (int)++h->report_seq;
+  launch_report(h->st, h->S, h->h_counters, seq);
   HIPCHK(h, hipGetLastError());
-  HIPCHK(h, hipStreamSynchronize(h->st));
   h->syncs++;
+  if (!whole_stream) {
+    for (unsigned spins = 1;; ++spins) {
+      if (__atomic_load_n(h->h_counters + CNT_INTS, __ATOMIC_ACQUIRE) == seq) return CS_OK;
+      __builtin_ia32_pause();
+      if (spins % 16384 == 0 && hipStreamQuery(h->st) != hipErrorNotReady) break;
+    }
+  }
+  HIPCHK(h, hipStreamSynchronize(h->st));
   return CS_OK;
 }
 
@@ -1014,11 +1029,12 @@ int cs_create(cs_solver** out, const cs_params* p) {
     return fail(nullptr, CS_ERR_ARG, "device ordinal out of range");
   }
   if (hipSetDevice(h->P.device) != hipSuccess || hipStreamCreate(&h->st) != hipSuccess ||
-      hipHostMalloc((void**)&h->h_counters, sizeof(int) * COUNTER_INTS) != hipSuccess) {
+      hipHostMalloc((void**)&h->h_counters, sizeof(int) * (COUNTER_INTS + 1)) != hipSuccess) {
     delete h;
     return fail(nullptr, CS_ERR_HIP, "HIP stream / pinned buffer creation failed");
   }
   init_scratch(h->P.device);  // the staging array of cs_zone_labels_noalloc
+  h->h_counters[COUNTER_INTS] = 0;
   *out = h;
   return CS_OK;
 }
@@ -1573,7 +1589,7 @@ int resolve_impl(cs_solver* h, cs_step_report* report, bool with_predict_graph) 
     HIPCHK(h, hipGetLastError());
   }
   mark(h, &t_end);
-  rc = read_counters(h);
+  rc = read_counters(h, true);
   if (rc) return rc;
   if (R.n_zone_passes) R.n_zones = h->h_counters[CNT_ZONES] + S.nbody;
   for (size_t i = 0; i < h->passes.size() && i < h->ptimes.size(); ++i) {

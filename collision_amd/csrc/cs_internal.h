@@ -288,8 +288,8 @@ enum {
   SCN_FIELDS
 };
 void launch_scene_reset(hipStream_t st, DevState& S);
-// the counters into (pinned) host memory
-void launch_report(hipStream_t st, DevState& S, int* host);
+// the counters into host[0 .. CNT_INTS) (pinned), then seq into host[CNT_INTS]
+void launch_report(hipStream_t st, DevState& S, int* host, int seq);
 void launch_fill_u32(hipStream_t st, void* p, int64_t words, uint32_t v);
 // after a pass's narrow phase: scene of each of its nhp hit pairs, then the
 // per-scene state machine of the reference's pass loop

@@ -731,13 +731,18 @@ void launch_fill_u32(hipStream_t st, void* p, int64_t words, uint32_t v) {
   hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)blocks), dim3(256), 0, st, (uint32_t*)p, words, v);
 }
 
-// A kernel rather than a copy command: one launch before a synchronisation.
-__global__ void k_report(const int* __restrict__ counters, int* __restrict__ host) {
+// A kernel rather than a copy command, one launch; the sequence number behind
+// the counters is written last, so a host that waits for it sees them all.
+__global__ void __launch_bounds__(64) k_report(const int* __restrict__ counters, int* host, int seq) {
   if (threadIdx.x < CNT_INTS) host[threadIdx.x] = counters[threadIdx.x];
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(host + CNT_INTS, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-void launch_report(hipStream_t st, DevState& S, int* host) {
-  hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, st, S.counters, host);
+void launch_report(hipStream_t st, DevState& S, int* host, int seq) {
+  hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, st, S.counters, host, seq);
 }
 
 void launch_predict(hipStream_t st, DevState& S, double dt) {
