@@ -178,41 +178,36 @@ __device__ inline cs_dd cs_dd_mul_d(cs_dd a, double b) {
 __device__ inline double cs_dd_round(cs_dd a) { return cs_fast_two_sum(a.hi, a.lo).hi; }
 __device__ inline cs_dd cs_dd_neg(cs_dd a) { return cs_dd{-a.hi, -a.lo}; }
 
-__device__ inline cs_dd cs_sin_dd(cs_dd r) {
-  const double hi[15] = {1.0, -0.16666666666666666, 0.008333333333333333, -0.0001984126984126984,
-                         2.7557319223985893e-06, -2.505210838544172e-08, 1.6059043836821613e-10,
-                         -7.647163731819816e-13, 2.8114572543455206e-15, -8.22063524662433e-18,
-                         1.9572941063391263e-20, -3.868170170630684e-23, 6.446950284384474e-26,
-                         -9.183689863795546e-29, 1.1309962886447716e-31};
-  const double lo[9] = {0.0, -9.25185853854297e-18, 1.1564823173178714e-19,
-                        -1.7209558293420705e-22, -1.858393274046472e-22, 1.448814070935912e-24,
-                        1.2585294588752098e-26, -7.03872877733453e-30, 1.6508842730861433e-31};
+// sin r or cos r by their Maclaurin series, the coefficients chosen per lane:
+// lanes of one wavefront that need the one and the other run a single chain
+// (each coefficient hi + lo; lo from the ninth term on is not needed)
+__device__ inline cs_dd cs_trig_dd(cs_dd r, bool sine) {
+  const double shi[15] = {1.0, -0.16666666666666666, 0.008333333333333333, -0.0001984126984126984,
+                          2.7557319223985893e-06, -2.505210838544172e-08, 1.6059043836821613e-10,
+                          -7.647163731819816e-13, 2.8114572543455206e-15, -8.22063524662433e-18,
+                          1.9572941063391263e-20, -3.868170170630684e-23, 6.446950284384474e-26,
+                          -9.183689863795546e-29, 1.1309962886447716e-31};
+  const double slo[9] = {0.0, -9.25185853854297e-18, 1.1564823173178714e-19,
+                         -1.7209558293420705e-22, -1.858393274046472e-22, 1.448814070935912e-24,
+                         1.2585294588752098e-26, -7.03872877733453e-30, 1.6508842730861433e-31};
+  const double chi[15] = {1.0, -0.5, 0.041666666666666664, -0.001388888888888889,
+                          2.48015873015873e-05, -2.755731922398589e-07, 2.08767569878681e-09,
+                          -1.1470745597729725e-11, 4.779477332387385e-14, -1.5619206968586225e-16,
+                          4.110317623312165e-19, -8.896791392450574e-22, 1.6117375710961184e-24,
+                          -2.4795962632247976e-27, 3.279889237069838e-30};
+  const double clo[9] = {0.0, 0.0, 2.3129646346357427e-18, 5.300543954373577e-20,
+                         2.1511947866775882e-23, -2.3767714622250297e-23, -1.20734505911326e-25,
+                         -2.0655512752830745e-28, 4.399205485834081e-31};
   const cs_dd r2 = cs_dd_mul(r, r);
-  double t = hi[14];
+  double t = sine ? shi[14] : chi[14];
 #pragma unroll
-  for (int k = 13; k >= 9; --k) t = t * r2.hi + hi[k];
+  for (int k = 13; k >= 9; --k) t = t * r2.hi + (sine ? shi[k] : chi[k]);
   cs_dd acc{t, 0.0};
 #pragma unroll
-  for (int k = 8; k >= 0; --k) acc = cs_dd_add(cs_dd_mul(acc, r2), cs_dd{hi[k], lo[k]});
-  return cs_dd_mul(acc, r);
-}
-__device__ inline cs_dd cs_cos_dd(cs_dd r) {
-  const double hi[15] = {1.0, -0.5, 0.041666666666666664, -0.001388888888888889,
-                         2.48015873015873e-05, -2.755731922398589e-07, 2.08767569878681e-09,
-                         -1.1470745597729725e-11, 4.779477332387385e-14, -1.5619206968586225e-16,
-                         4.110317623312165e-19, -8.896791392450574e-22, 1.6117375710961184e-24,
-                         -2.4795962632247976e-27, 3.279889237069838e-30};
-  const double lo[9] = {0.0, 0.0, 2.3129646346357427e-18, 5.300543954373577e-20,
-                        2.1511947866775882e-23, -2.3767714622250297e-23, -1.20734505911326e-25,
-                        -2.0655512752830745e-28, 4.399205485834081e-31};
-  const cs_dd r2 = cs_dd_mul(r, r);
-  double t = hi[14];
-#pragma unroll
-  for (int k = 13; k >= 9; --k) t = t * r2.hi + hi[k];
-  cs_dd acc{t, 0.0};
-#pragma unroll
-  for (int k = 8; k >= 0; --k) acc = cs_dd_add(cs_dd_mul(acc, r2), cs_dd{hi[k], lo[k]});
-  return acc;
+  for (int k = 8; k >= 0; --k)
+    acc = cs_dd_add(cs_dd_mul(acc, r2), cs_dd{sine ? shi[k] : chi[k], sine ? slo[k] : clo[k]});
+  const cs_dd odd = cs_dd_mul(acc, r);
+  return sine ? odd : acc;
 }
 
 // x = k pi/2 + r, |r| <= pi/4 (+ rounding); returns k mod 4
@@ -230,7 +225,7 @@ __device__ inline double cs_det_cos(double x) {
   if (!(fabs(x) < 1e9)) return x - x;
   cs_dd r;
   const int q = cs_reduce(x, &r);
-  cs_dd v = (q & 1) ? cs_sin_dd(r) : cs_cos_dd(r);
+  cs_dd v = cs_trig_dd(r, q & 1);
   if (q == 1 || q == 2) v = cs_dd_neg(v);
   return cs_dd_round(v);
 }
@@ -240,7 +235,7 @@ __device__ inline double cs_det_sin(double x) {
   if (x == 0.0) return x;
   cs_dd r;
   const int q = cs_reduce(x, &r);
-  cs_dd v = (q & 1) ? cs_cos_dd(r) : cs_sin_dd(r);
+  cs_dd v = cs_trig_dd(r, !(q & 1));
   if (q >= 2) v = cs_dd_neg(v);
   return cs_dd_round(v);
 }
@@ -268,7 +263,7 @@ __device__ inline double cs_asin_seed(double z) {
 __device__ inline cs_dd cs_asin_dd(cs_dd z) {
   const double y0 = cs_asin_seed(z.hi);
   const cs_dd y{y0, 0.0};
-  const cs_dd s = cs_sin_dd(y), c = cs_cos_dd(y);
+  const cs_dd s = cs_trig_dd(y, true), c = cs_trig_dd(y, false);
   const cs_dd d = cs_dd_add(s, cs_dd_neg(z));
   const double corr = d.hi / c.hi;
   return cs_two_sum(y0, -corr);

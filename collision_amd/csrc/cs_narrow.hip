@@ -19,6 +19,7 @@
 // dcollid3d.cpp:222-229, 300-302, 319-321) by a lock-free union-find whose
 // roots are the smallest vertex id of each zone.
 #include <algorithm>
+#include <type_traits>
 
 #include "cs_internal.h"
 #include "cs_pairs.h"
@@ -526,10 +527,26 @@ __device__ bool d_is_coplanar(const Sub& S, double dt, double roots[4]) {
 
 // roots / *coplanar: isCoplanar's outcome for a CCD sub-test (roots -1 and
 // false when the certified screen decided it)
+// The forms of the narrow kernel, each compiled by itself, so that none pays for
+// the registers of another.  As one kernel all had 168 VGPRs (3 wavefronts per
+// SIMD) and 128 B of scratch per lane.  Now, at 2.6e6 pairs of a 1024 x 1024
+// drape with strings: proximity 119 VGPRs, 4 wavefronts, no scratch, 0.80 ->
+// 0.67 ms; whole CCD streams 168, 3 wavefronts, 64 B, 2.11 -> 1.98 ms (2
+// wavefronts without scratch: 2.5 ms); the re-queried pairs of incremental
+// passes, a few thousand that do not fill the card and end with their slowest
+// sub-test, 181 VGPRs without scratch, 85 launches 3.06 -> 2.55 ms (168: 2.99).
+enum NarrowKind {
+  NK_PROX,   // proximity
+  NK_MIXED,  // proximity with the FP32 screen
+  NK_CCD,    // CCD with the certified screen: whole streams
+  NK_REST,   // CCD without it: the re-queried pairs of incremental passes
+  NK_EXTRA   // CCD, learned form or collecting samples
+};
+template <int KIND>
 __device__ bool d_subtest(const Sub& S, bool is_pt, const NarrowParams& P, Contrib& C, int* err,
                           double roots[4], bool* coplanar, int known) {
   double c[4][3];
-  if (!P.ccd) {
+  if constexpr (KIND == NK_PROX || KIND == NK_MIXED) {
 #pragma unroll
     for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -542,8 +559,9 @@ __device__ bool d_subtest(const Sub& S, bool is_pt, const NarrowParams& P, Contr
   *coplanar = false;
   // known: 1 = the certified screen already proved isCoplanar false, 0 = it
   // could not, -1 = not screened yet
-  if (known == 1) return false;
-  if (known < 0 && P.screen && d_coplanar_certainly_false(S, P.dt)) return false;
+  if (KIND == NK_EXTRA && known == 1) return false;
+  if ((KIND == NK_CCD || (KIND == NK_EXTRA && known < 0 && P.screen)) &&
+      d_coplanar_certainly_false(S, P.dt)) return false;
   if (!d_is_coplanar(S, P.dt, roots)) return false;
   *coplanar = true;
   for (int r = 0; r < 4; ++r) {
@@ -827,12 +845,14 @@ struct StagedVertex {
   int fixed, body, pad0, pad1;
 };
 
+template <int KIND>
 __device__ __attribute__((always_inline)) inline void narrow_lane(
     int64_t gl, const int2* __restrict__ pairs, int npairs, const int4* __restrict__ ev,
     const dvec4* __restrict__ x_old, const dvec4* __restrict__ av,
     const uint8_t* __restrict__ fixed, const NarrowParams& P, const ZoneList& Z,
     hit_rec* __restrict__ hits, int hit_cap, int4* __restrict__ hp, int hp_cap,
     int* __restrict__ counters, StagedVertex* __restrict__ stage) {
+  constexpr bool ccd = KIND >= NK_CCD, extra = KIND == NK_EXTRA, mixed = KIND == NK_MIXED;
   int* err = counters + CNT_ERR;
   const int64_t i = gl / SUB_GROUP;
   const int s = (int)(gl % SUB_GROUP);
@@ -841,7 +861,7 @@ __device__ __attribute__((always_inline)) inline void narrow_lane(
   int g[6] = {0, 0, 0, 0, 0, 0};
   int64_t pi = i;  // position of the pair in the stream
   if (i < npairs) {
-    if (P.perm) pi = P.perm[i];
+    if (extra && P.perm) pi = P.perm[i];
     pair_points(pairs[pi], ev, &A, &B, &kind, &nsub, g);
   }
   const bool active = s < nsub;
@@ -850,7 +870,7 @@ __device__ __attribute__((always_inline)) inline void narrow_lane(
   MixedErr me{0.0f, 0.0f, 0.0f};
   int known = -1;     // learned form: the screen's verdict for this slot
   float lcode = 0.0f;
-  if (P.ccd && P.lseed && active) {
+  if (extra && P.lseed && active) {
     lcode = P.lseed[pi * SUB_GROUP + s];
     known = lcode == SEED_CERTAIN ? 1 : 0;
   }
@@ -876,7 +896,7 @@ __device__ __attribute__((always_inline)) inline void narrow_lane(
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   if (active) {
     bool is_pt;
-    subtest_points(kind, s, P.ccd, q, &is_pt);
+    subtest_points(kind, s, ccd, q, &is_pt);
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       const StagedVertex& v = stage[q[p]];
@@ -891,16 +911,16 @@ __device__ __attribute__((always_inline)) inline void narrow_lane(
         if (q[p] == k) vid = g[k];
       q[p] = vid;  // from here on: global vertex ids
     }
-    if (P.mixed && !P.ccd) {
+    if (mixed) {
       rejected = is_pt ? screen_pt(S, P.thickness, P.round_eps, P.mixed_stats, &me)
                        : screen_ee(S, P.thickness, P.mixed_stats, &me);
     }
-    if (!rejected) hit = d_subtest(S, is_pt, P, C, err, roots, &coplanar, known);
-    if (P.ccd && P.ds_cap > 0) collect_subtest(S, P, B, A, s, coplanar, roots);
+    if (!rejected) hit = d_subtest<KIND>(S, is_pt, P, C, err, roots, &coplanar, known);
+    if (extra && P.ds_cap > 0) collect_subtest(S, P, B, A, s, coplanar, roots);
   }
   int* sp = P.spread + (blockIdx.x & (SPREAD_SLOTS - 1)) * SPREAD_STRIDE;
-  if (P.ccd && P.lseed) learned_stats(P, known == 0, coplanar, roots, lcode, S, sp);
-  if (P.mixed && !P.ccd) {  // every lane of the wavefront takes part
+  if (extra && P.lseed) learned_stats(P, known == 0, coplanar, roots, lcode, S, sp);
+  if (mixed) {  // every lane of the wavefront takes part
     const uint64_t rb = __ballot(active && rejected), kb = __ballot(active && !rejected);
     float md = 0.0f, mp = 0.0f, mr = 0.0f;
     if (P.mixed_stats) {
@@ -967,8 +987,11 @@ __device__ __attribute__((always_inline)) inline void narrow_lane(
 
 // npairs_dev != nullptr: the pair count is read on the device (clamped to
 // cap); the grid covers the first npairs pairs of it
-template <int THREADS>
-__global__ void __launch_bounds__(THREADS, 3)
+// wavefronts per SIMD that the registers are cut for
+constexpr int narrow_waves(int kind) { return kind == NK_REST ? 2 : kind <= NK_MIXED ? 4 : 3; }
+
+template <int THREADS, int KIND>
+__global__ void __launch_bounds__(THREADS, narrow_waves(KIND))
     k_narrow(const int2* __restrict__ pairs, int npairs, const int* __restrict__ npairs_dev,
              int cap, const int4* __restrict__ ev, const dvec4* __restrict__ x_old,
              const dvec4* __restrict__ av, const uint8_t* __restrict__ fixed, NarrowParams P,
@@ -990,7 +1013,7 @@ __global__ void __launch_bounds__(THREADS, 3)
   const int64_t gl = (int64_t)b * THREADS + threadIdx.x;
   if ((gl & ~63ll) >= (int64_t)n * SUB_GROUP) return;  // whole wavefronts past the end
   __shared__ StagedVertex stage[THREADS / SUB_GROUP][6];
-  narrow_lane(gl, pairs, n, ev, x_old, av, fixed, P, Z, hits, hit_cap, hp, hp_cap, counters,
+  narrow_lane<KIND>(gl, pairs, n, ev, x_old, av, fixed, P, Z, hits, hit_cap, hp, hp_cap, counters,
               stage[threadIdx.x / SUB_GROUP]);
 }
 
@@ -1007,9 +1030,22 @@ void launch_narrow(hipStream_t st, DevState& S, const NarrowParams& P, const int
                        cap, S.ev, S.x_old, S.av, S.fixed, P, zone_list(S), S.hits, S.hit_cap, S.hp,
                        S.hp_cap, S.counters);
   };
-  if (T == 64) go(k_narrow<64>);
-  else if (T == 256) go(k_narrow<256>);
-  else go(k_narrow<128>);
+  auto size = [&](auto kind) {
+    constexpr int K = decltype(kind)::value;
+    if (T == 64) go(k_narrow<64, K>);
+    else if (T == 256) go(k_narrow<256, K>);
+    else go(k_narrow<128, K>);
+  };
+  if (!P.ccd) {
+    if (P.mixed) size(std::integral_constant<int, NK_MIXED>{});
+    else size(std::integral_constant<int, NK_PROX>{});
+  } else if (P.lseed || P.ds_cap > 0) {
+    size(std::integral_constant<int, NK_EXTRA>{});
+  } else if (P.screen) {
+    size(std::integral_constant<int, NK_CCD>{});
+  } else {
+    size(std::integral_constant<int, NK_REST>{});
+  }
 }
 
 // Learned form, step 1: the certified coplanarity screen of every CCD
