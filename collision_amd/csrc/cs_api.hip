@@ -778,6 +778,35 @@ int check_ready(cs_solver* h) {
   return CS_OK;
 }
 
+// Device memory for the arrays of one inference or gradient call: kept with the
+// handle for the next call where it is small (four allocations and frees, up to
+// 40 us, per call before), given back at once where it is large.
+struct LearnedWorkspace {
+  float* p = nullptr;
+  bool temporary = false;
+  hipError_t error = hipSuccess;
+  LearnedWorkspace(LearnedState& L, size_t floats) {
+    if (floats * sizeof(float) > LearnedState::WS_KEEP) {
+      temporary = true;
+      error = dalloc(&p, floats);
+      return;
+    }
+    if (floats > L.ws_floats) {
+      dfree(L.ws);
+      L.ws_floats = 0;
+      const size_t n = std::min(floats + floats / 2, LearnedState::WS_KEEP / sizeof(float));
+      if ((error = dalloc(&L.ws, n)) != hipSuccess) return;
+      L.ws_floats = n;
+    }
+    p = L.ws;
+  }
+  ~LearnedWorkspace() {
+    if (temporary) dfree(p);
+  }
+  LearnedWorkspace(const LearnedWorkspace&) = delete;
+  LearnedWorkspace& operator=(const LearnedWorkspace&) = delete;
+};
+
 // The banded strain-limit plan, with more bands (smaller vertex windows) as
 // long as a window does not fit; false when none does (elements in random
 // order over a large mesh: every band then meets most vertices at once).
@@ -2017,17 +2046,15 @@ int cs_learned_infer(cs_solver* h, const float* x, float* out, int64_t n) {
   if (!h->L.ready) return fail(h, CS_ERR_ARG, "no weights have been set");
   if (n == 0) return CS_OK;
   HIPCHK(h, hipSetDevice(h->P.device));
-  float *dx = nullptr, *dout = nullptr;
-  hipError_t e = dalloc(&dx, (size_t)n * 24);
-  if (e == hipSuccess) e = dalloc(&dout, (size_t)n * 2);
+  LearnedWorkspace ws(h->L, (size_t)n * 26);
+  hipError_t e = ws.error;
+  float* dout = ws.p + (size_t)n * 24;
   if (e == hipSuccess)
-    e = hipMemcpyAsync(dx, x, sizeof(float) * 24 * (size_t)n, hipMemcpyHostToDevice, h->st);
-  if (e == hipSuccess) e = learned_infer(h->L, h->st, dx, n, dout);
+    e = hipMemcpyAsync(ws.p, x, sizeof(float) * 24 * (size_t)n, hipMemcpyHostToDevice, h->st);
+  if (e == hipSuccess) e = learned_infer(h->L, h->st, ws.p, n, dout);
   if (e == hipSuccess)
     e = hipMemcpyAsync(out, dout, sizeof(float) * 2 * (size_t)n, hipMemcpyDeviceToHost, h->st);
   if (e == hipSuccess) e = hipStreamSynchronize(h->st);
-  dfree(dx);
-  dfree(dout);
   if (e != hipSuccess) return fail(h, CS_ERR_HIP, std::string("learned inference: ") + hipGetErrorString(e));
   return CS_OK;
 }
@@ -2037,29 +2064,26 @@ int cs_learned_grad(cs_solver* h, const float* x, const float* exists, const flo
   if (!h || !x || !exists || !toi || !grad || n <= 0 || n > (1 << 24)) return CS_ERR_ARG;
   if (!h->L.ready) return fail(h, CS_ERR_ARG, "no weights have been set");
   HIPCHK(h, hipSetDevice(h->P.device));
-  float *dx = nullptr, *de = nullptr, *dt = nullptr, *dl = nullptr;
-  hipError_t e = dalloc(&dx, (size_t)n * 24);
-  if (e == hipSuccess) e = dalloc(&de, (size_t)n);
-  if (e == hipSuccess) e = dalloc(&dt, (size_t)n);
-  if (e == hipSuccess) e = dalloc(&dl, 1);
+  LearnedState& L = h->L;
+  const size_t out_bytes = sizeof(float) * (CS_MLP_PARAMS + 1);  // gradient, loss
+  LearnedWorkspace ws(L, (size_t)n * 26);
+  hipError_t e = ws.error;
+  if (e == hipSuccess && !L.host_grad) e = hipHostMalloc((void**)&L.host_grad, out_bytes);
+  float *dx = ws.p, *de = ws.p + (size_t)n * 24, *dt = de + n;
   if (e == hipSuccess)
     e = hipMemcpyAsync(dx, x, sizeof(float) * 24 * (size_t)n, hipMemcpyHostToDevice, h->st);
   if (e == hipSuccess)
     e = hipMemcpyAsync(de, exists, sizeof(float) * (size_t)n, hipMemcpyHostToDevice, h->st);
   if (e == hipSuccess)
     e = hipMemcpyAsync(dt, toi, sizeof(float) * (size_t)n, hipMemcpyHostToDevice, h->st);
-  if (e == hipSuccess) e = learned_grad(h->L, h->st, dx, de, dt, nullptr, (int)n, dl);
   if (e == hipSuccess)
-    e = hipMemcpyAsync(grad, h->L.grad, sizeof(float) * CS_MLP_PARAMS, hipMemcpyDeviceToHost, h->st);
-  float l = 0.f;
-  if (e == hipSuccess) e = hipMemcpyAsync(&l, dl, sizeof(float), hipMemcpyDeviceToHost, h->st);
+    e = learned_grad(L, h->st, dx, de, dt, nullptr, (int)n, L.grad + CS_MLP_PARAMS);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(L.host_grad, L.grad, out_bytes, hipMemcpyDeviceToHost, h->st);
   if (e == hipSuccess) e = hipStreamSynchronize(h->st);
-  dfree(dx);
-  dfree(de);
-  dfree(dt);
-  dfree(dl);
   if (e != hipSuccess) return fail(h, CS_ERR_HIP, std::string("learned gradient: ") + hipGetErrorString(e));
-  if (loss) *loss = l;
+  std::memcpy(grad, L.host_grad, sizeof(float) * CS_MLP_PARAMS);
+  if (loss) *loss = L.host_grad[CS_MLP_PARAMS];
   return CS_OK;
 }
 

@@ -318,6 +318,12 @@ struct LearnedState {
   int64_t ds_alloc = 0, ds_cap = 0;
   int32_t ds_stride = 1;
   uint32_t ds_salt = 0;
+  // inputs and outputs of cs_learned_infer / cs_learned_grad (kept up to WS_KEEP
+  // bytes) and the pinned copy of a gradient and its loss
+  float* ws = nullptr;
+  size_t ws_floats = 0;
+  float* host_grad = nullptr;
+  static constexpr size_t WS_KEEP = 64u << 20;
   // training partials
   float *gpart = nullptr, *lpart = nullptr;
   int train_tiles = 0;

@@ -373,7 +373,7 @@ hipError_t learned_alloc(LearnedState& L) {
   CS_HIP_RET(lalloc(&L.w, MF_NPARAM));
   CS_HIP_RET(lalloc(&L.m, MF_NPARAM));
   CS_HIP_RET(lalloc(&L.v, MF_NPARAM));
-  CS_HIP_RET(lalloc(&L.grad, MF_NPARAM));
+  CS_HIP_RET(lalloc(&L.grad, MF_NPARAM + 1));  // (a gradient call's loss behind it)
   CS_HIP_RET(lalloc(&L.wb, MB_TOTAL));
   CS_HIP_RET(lalloc(&L.ds_count, 1));
   return hipMemset(L.ds_count, 0, sizeof(unsigned long long));
@@ -384,7 +384,8 @@ void learned_free(LearnedState& L) {
   lfree(L.ds_count); lfree(L.dsx); lfree(L.dse); lfree(L.dst);
   lfree(L.seeds); lfree(L.list); lfree(L.count);
   lfree(L.keys); lfree(L.idx); lfree(L.tkeys); lfree(L.tidx);
-  lfree(L.hist); lfree(L.part); lfree(L.gpart); lfree(L.lpart);
+  lfree(L.hist); lfree(L.part); lfree(L.gpart); lfree(L.lpart); lfree(L.ws);
+  if (L.host_grad) (void)hipHostFree(L.host_grad);
   L = LearnedState();
 }
 
