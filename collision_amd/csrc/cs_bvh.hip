@@ -915,12 +915,17 @@ __device__ inline void grow_dirty(const GrowArgs& G, int nd, int block, int bloc
 // One wavefront per QW_RANGE-node range of the pre-order layout that holds dirty
 // leaves: the range's dirty leaves are neighbours in Morton order, so the
 // union of their boxes is small.  The wavefront descends the tree breadth
-// first with that union box, one level per step with every lane loading one
-// node of the frontier, collects the leaves the union box overlaps, and each
-// lane then tests its own element against them with the exact boxes.  The
-// number of dependent loads is the tree depth rather than the length of a
-// single-lane walk.  A frontier or leaf list too large for LDS falls back to
-// one stackless walk per lane.
+// first with that union box, collects the leaves the union box overlaps, and
+// each lane then tests its own element against them with the exact boxes.  A
+// frontier or leaf list too large for LDS falls back to one stackless walk per
+// lane.  A zone pass has a few hundred ranges of about 27 leaves each in a tree
+// 27 levels deep, so the steps of the descent, a dependent load each, bound the
+// kernel.  A step follows chains of up to QW_CHAIN first children, so there are
+// about half as many steps as levels.  Query and growth per step (87 passes at
+// 1024 x 1024, 33 at 256 x 256, 8 with many ranges on a wavy 256 x 256 sheet):
+// 3.95, 1.10, 0.92 ms one level at a time, 3.60, 0.98, 0.80 with chains of 2,
+// 3.40, 0.94, 0.81 with 4, 3.66, 1.00, 0.99 with 8.
+constexpr int QW_CHAIN = 4;    // records of one first-child chain read at a time
 constexpr int QW_FCAP = 1024;  // frontier nodes of one level
 constexpr int QW_LCAP = 1024;  // leaves collected by one range
 
@@ -981,15 +986,18 @@ __global__ void __launch_bounds__(64) k_query_ranges(
   // round-robin placement spreads them over all XCDs
   for (int ri = blockIdx.x; ri < nr; ri += gridDim.x) {
     const int si = QW_RANGE * rlist[ri] + lane;  // this lane's node
-    const bool act = lane < QW_RANGE && si < npre && dpre[si];
     bvh_node me{};
+    bool act = false;
+    if (lane < QW_RANGE && si < npre) {
+      me = nodes[si];
+      act = dpre[si];
+    }
     dbox mb{};
     int4 mt{};
     uint8_t mf = 0;
     int e = -1;
     float ulo[3] = {3.4e38f, 3.4e38f, 3.4e38f}, uhi[3] = {-3.4e38f, -3.4e38f, -3.4e38f};
     if (act) {
-      me = nodes[si];
       e = me.left;
       mb = ebox[e];
       mt = ev[e];
@@ -1001,13 +1009,22 @@ __global__ void __launch_bounds__(64) k_query_ranges(
       }
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
+    for (int o = QW_RANGE / 2; o > 0; o >>= 1)
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
         ulo[d] = fminf(ulo[d], __shfl_xor(ulo[d], o));
         uhi[d] = fmaxf(uhi[d], __shfl_xor(uhi[d], o));
       }
-    // breadth-first descent with the union box
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {  // (the lanes past the range hold empty boxes)
+      ulo[d] = __shfl(ulo[d], 0);
+      uhi[d] = __shfl(uhi[d], 0);
+    }
+    // Breadth-first descent with the union box.  A node's first child is the
+    // next record, so QW_CHAIN lanes take a frontier node and the records
+    // behind it: as far as the boxes overlap they go down the chain of first
+    // children, and only second children (and what follows the last record)
+    // wait for the next step.
     if (lane == 0) fr[0][0] = 0;
     __syncthreads();
     int cur = 0, nfr = 1, nlv = 0;
@@ -1015,38 +1032,35 @@ __global__ void __launch_bounds__(64) k_query_ranges(
     const uint64_t below = (1ull << lane) - 1ull;
     while (nfr > 0) {
       int nnext = 0;
-      for (int b = 0; b < nfr; b += 64) {
-        const int i = b + lane;
-        bool kl = false, ki = false;
+      for (int b = 0; b < nfr; b += 64 / QW_CHAIN) {
+        const int i = b + lane / QW_CHAIN, j = lane % QW_CHAIN;
+        bool ov = false, inner = false;
         int node = 0, c2 = 0, left = -1;
-        if (i < nfr) {
-          node = fr[cur][i];
+        if (i < nfr) node = fr[cur][i] + j;
+        if (i < nfr && node < npre) {
           const bvh_node N = nodes[node];
-          const int r2 = nright[node];
-          if (f32_overlap(N, ulo, uhi)) {
-            if (N.left >= 0) {
-              kl = true;
-              left = N.left;
-            } else {
-              ki = true;
-              c2 = r2;
-            }
-          }
+          c2 = nright[node];
+          left = N.left;
+          inner = left < 0;
+          ov = f32_overlap(N, ulo, uhi);
         }
-        const uint64_t ml = __ballot(kl), mi = __ballot(ki);
-        if (kl) {
+        // reached: every record before this one of the four is gone down from
+        const uint32_t before = (1u << j) - 1u;
+        const uint32_t down = (uint32_t)(__ballot(ov && inner) >> (lane - j));
+        const bool reached = ov && (down & before) == before;
+        const uint64_t ml = __ballot(reached && !inner), mi = __ballot(reached && inner);
+        const uint64_t mc = __ballot(reached && inner && j == QW_CHAIN - 1);
+        if (reached && !inner) {
           const int q = nlv + __popcll(ml & below);
           if (q < QW_LCAP) lv[q] = make_int2(node, left);
         }
-        if (ki) {
-          const int q = nnext + 2 * __popcll(mi & below);
-          if (q + 1 < QW_FCAP) {
-            fr[cur ^ 1][q] = node + 1;
-            fr[cur ^ 1][q + 1] = c2;
-          }
+        if (reached && inner) {
+          const int q = nnext + __popcll(mi & below) + __popcll(mc & below);
+          if (q < QW_FCAP) fr[cur ^ 1][q] = c2;
+          if (j == QW_CHAIN - 1 && q + 1 < QW_FCAP) fr[cur ^ 1][q + 1] = node + 1;
         }
         nlv += __popcll(ml);
-        nnext += 2 * __popcll(mi);
+        nnext += __popcll(mi) + __popcll(mc);
       }
       __syncthreads();
       if (nlv > QW_LCAP || nnext > QW_FCAP) {
