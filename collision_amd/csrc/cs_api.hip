@@ -1499,13 +1499,13 @@ namespace {
 // pass and the counters, the batched scenes' pass state, then
 // computeAverageVelocity with the union-find (makeSet, dcollid.cpp:1015-1031),
 // the recorded impulses and the zone marks.
-void resolve_prologue(cs_solver* h, bool stats) {
+void resolve_prologue(cs_solver* h, bool stats, bool predict) {
   DevState& S = h->S;
   const cs_params& P = h->P;
   launch_pass_begin(h->st, S, ~0ull);
   if (stats) launch_fill_u32(h->st, S.spread, (int64_t)SPREAD_SLOTS * SPREAD_STRIDE, 0u);
   launch_scene_reset(h->st, S);
-  launch_average_velocity(h->st, S, P.dt, P.record_impulses && S.pimp);
+  launch_average_velocity(h->st, S, P.dt, P.record_impulses && S.pimp, predict);
 }
 
 // the predictor and the resolve prologue as one graph, captured again when
@@ -1523,8 +1523,7 @@ int ensure_step_graph(cs_solver* h, bool stats) {
   h->graph_exec = nullptr;
   h->graph = nullptr;
   HIPCHK(h, hipStreamBeginCapture(h->st, hipStreamCaptureModeThreadLocal));
-  launch_predict(h->st, h->S, h->P.dt);
-  resolve_prologue(h, stats);
+  resolve_prologue(h, stats, true);
   hipGraph_t g = nullptr;
   const hipError_t e = hipStreamEndCapture(h->st, &g);
   if (e != hipSuccess) return fail(h, CS_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(e));
@@ -1534,8 +1533,9 @@ int ensure_step_graph(cs_solver* h, bool stats) {
   return CS_OK;
 }
 
-// with_predict_graph: the predictor runs first, inside the captured graph
-int resolve_impl(cs_solver* h, cs_step_report* report, bool with_predict_graph) {
+// predict: the predictor runs first (with graph_step the prologue with it as a
+// captured graph)
+int resolve_impl(cs_solver* h, cs_step_report* report, bool predict) {
   int rc = check_ready(h);
   if (rc) return rc;
   if (h->P.learned && !h->L.ready)
@@ -1569,13 +1569,13 @@ int resolve_impl(cs_solver* h, cs_step_report* report, bool with_predict_graph) 
     HIPCHK(h, dalloc(&S.pimp, S.nv));
     HIPCHK(h, dalloc(&S.pnum, S.nv));
   }
-  if (with_predict_graph) {
+  if (predict && P.graph_step) {
     if ((rc = ensure_step_graph(h, spread_stats))) return rc;
     mark(h, &t0);
     HIPCHK(h, hipGraphLaunch(h->graph_exec, h->st));
   } else {
     mark(h, &t0);
-    resolve_prologue(h, spread_stats);
+    resolve_prologue(h, spread_stats, predict);
   }
   HIPCHK(h, hipGetLastError());
   int pass_id = 0;
@@ -1609,8 +1609,7 @@ int resolve_impl(cs_solver* h, cs_step_report* report, bool with_predict_graph) 
   }
   mark(h, &t_strain0);
   if (status == CS_OK || status == CS_WARN_ZONE_CAP) {
-    launch_domain_boundary(h->st, S, P.dom_lo, P.dom_hi, P.dt, P.friction, P.thickness);
-    launch_final_position(h->st, S, P.dt);
+    launch_final_position(h->st, S, P.dom_lo, P.dom_hi, P.dt, P.friction);
     HIPCHK(h, strain_limit(h->st, S, P.dt, P.max_strain_sweeps,
                            P.pass_timing >= 1 ? &strain_marks : nullptr));
     launch_final_velocity(h->st, S);
@@ -1736,8 +1735,14 @@ int resolve_impl(cs_solver* h, cs_step_report* report, bool with_predict_graph) 
 
 int cs_resolve(cs_solver* h, cs_step_report* report) { return resolve_impl(h, report, false); }
 
+// the resolve of a step will not be refused (a refused one leaves the predicted
+// state, as cs_predict followed by cs_resolve does)
+static bool step_ready(const cs_solver* h) {
+  return h->assembled && h->state_set && !(h->P.learned && !h->L.ready);
+}
+
 int cs_step(cs_solver* h, cs_step_report* report) {
-  if (h && h->P.graph_step) return resolve_impl(h, report, true);
+  if (h && (h->P.graph_step || step_ready(h))) return resolve_impl(h, report, true);
   int rc = cs_predict(h);
   if (rc) return rc;
   return cs_resolve(h, report);
@@ -1746,12 +1751,12 @@ int cs_step(cs_solver* h, cs_step_report* report) {
 namespace {
 
 int resolve_batch_impl(cs_solver* h, cs_step_report* report, cs_scene_report* per_scene,
-                       int32_t nscene, bool with_predict_graph) {
+                       int32_t nscene, bool predict) {
   if (!h) return CS_ERR_ARG;
   if (!h->assembled) return fail(h, CS_ERR_ARG, "cs_assemble has not been called");
   if (h->S.nscene <= 1 || nscene != h->S.nscene || !per_scene)
     return fail(h, CS_ERR_ARG, "nscene must equal the assembled batch's scene count");
-  const int rc = resolve_impl(h, report, with_predict_graph);
+  const int rc = resolve_impl(h, report, predict);
   if (rc != CS_OK && rc != CS_WARN_ZONE_CAP) return rc;
   std::vector<int32_t> f((size_t)SCN_FIELDS * nscene);
   HIPCHK(h, hipMemcpyAsync(f.data(), h->S.scn, sizeof(int32_t) * f.size(), hipMemcpyDeviceToHost,
@@ -1779,7 +1784,9 @@ int cs_resolve_batch(cs_solver* h, cs_step_report* report, cs_scene_report* per_
 
 int cs_step_batch(cs_solver* h, cs_step_report* report, cs_scene_report* per_scene,
                   int32_t nscene) {
-  if (h && h->P.graph_step) return resolve_batch_impl(h, report, per_scene, nscene, true);
+  if (h && (h->P.graph_step ||
+            (step_ready(h) && h->S.nscene > 1 && nscene == h->S.nscene && per_scene)))
+    return resolve_batch_impl(h, report, per_scene, nscene, true);
   int rc = cs_predict(h);
   if (rc) return rc;
   return cs_resolve_batch(h, report, per_scene, nscene);

@@ -28,17 +28,50 @@
 
 namespace cs {
 
+// the box centre of element e into the running bounds m
+__device__ inline void centre_bounds(const dbox& b, float m[6]) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const float c = (float)(0.5 * (b.lo[d] + b.hi[d]));
+    m[d] = fminf(m[d], c);
+    m[3 + d] = fmaxf(m[3 + d], c);
+  }
+}
+
+// The bounds of a work-group's threads into its row.  The rows are reduced by
+// every work-group of k_morton (no atomics: 6,144 of them on six addresses took
+// 50-110 us).
+constexpr int BOUNDS_BLOCKS = 128, BOUNDS_THREADS = 512;
+template <int THREADS>
+__device__ inline void bounds_row(float m[6], float* __restrict__ bounds) {
+  __shared__ float s[6][THREADS / 64];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      m[d] = fminf(m[d], __shfl_xor(m[d], o));
+      m[3 + d] = fmaxf(m[3 + d], __shfl_xor(m[3 + d], o));
+    }
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int d = 0; d < 6; ++d) s[d][threadIdx.x >> 6] = m[d];
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    const int d = threadIdx.x;
+    float r = s[d][0];
+    for (int w = 1; w < THREADS / 64; ++w) r = d < 3 ? fminf(r, s[d][w]) : fmaxf(r, s[d][w]);
+    bounds[6 * blockIdx.x + d] = r;
+  }
+}
+
 // Element boxes (the reference's min/max_{static,moving}_coord,
 // dcollid.cpp:852-932), inflated by 1e-6: static boxes into sbox, swept boxes
 // into mbox, either may be null.
-__global__ void __launch_bounds__(256) k_element_boxes(const int4* __restrict__ ev,
-                                                       const dvec4* __restrict__ x,
-                                                       const dvec4* __restrict__ x_old,
-                                                       const dvec4* __restrict__ av, double dt, int ne,
-                                                       dbox* __restrict__ sbox,
-                                                       dbox* __restrict__ mbox) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
+// m: the bounds of the box centres (of mbox where there is one).
+__device__ inline void element_box(const int4* __restrict__ ev, const dvec4* __restrict__ x,
+                                   const dvec4* __restrict__ x_old, const dvec4* __restrict__ av,
+                                   double dt, int e, dbox* __restrict__ sbox,
+                                   dbox* __restrict__ mbox, float m[6]) {
   const int4 t = ev[e];
   const int np = (t.z >= 0) ? 3 : 2;
   const int vid[3] = {t.x, t.y, t.z};
@@ -89,43 +122,32 @@ __global__ void __launch_bounds__(256) k_element_boxes(const int4* __restrict__ 
       b.hi[d] = hi[k][d] + CS_BOX_EPS;
     }
     out[k][e] = b;
+    if (k == 1 || !mbox) centre_bounds(b, m);
   }
 }
 
-// min/max of the box centres (FP32): one row of six per work-group, reduced by
-// every work-group of k_morton (no atomics: 6,144 of them on six addresses
-// took 50-110 us)
-constexpr int BOUNDS_BLOCKS = 128, BOUNDS_THREADS = 512;
+__global__ void __launch_bounds__(256) k_element_boxes(const int4* __restrict__ ev,
+                                                       const dvec4* __restrict__ x,
+                                                       const dvec4* __restrict__ x_old,
+                                                       const dvec4* __restrict__ av, double dt, int ne,
+                                                       dbox* __restrict__ sbox,
+                                                       dbox* __restrict__ mbox,
+                                                       float* __restrict__ bounds) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  float m[6] = {3.4e38f, 3.4e38f, 3.4e38f, -3.4e38f, -3.4e38f, -3.4e38f};
+  if (e < ne) element_box(ev, x, x_old, av, dt, e, sbox, mbox, m);
+  if (bounds) bounds_row<256>(m, bounds);
+}
+
+// The bounds of all box centres where the boxes take more work-groups than there
+// are rows; up to 32,768 elements k_element_boxes writes the rows itself (one
+// launch less, 2.6 us).
 __global__ void __launch_bounds__(BOUNDS_THREADS) k_bounds(const dbox* __restrict__ ebox, int ne,
                                                            float* __restrict__ bounds) {
-  __shared__ float s[6][BOUNDS_THREADS / 64];
   float m[6] = {3.4e38f, 3.4e38f, 3.4e38f, -3.4e38f, -3.4e38f, -3.4e38f};
-  for (int e = blockIdx.x * BOUNDS_THREADS + threadIdx.x; e < ne; e += gridDim.x * BOUNDS_THREADS) {
-    const dbox b = ebox[e];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const float c = (float)(0.5 * (b.lo[d] + b.hi[d]));
-      m[d] = fminf(m[d], c);
-      m[3 + d] = fmaxf(m[3 + d], c);
-    }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      m[d] = fminf(m[d], __shfl_xor(m[d], o));
-      m[3 + d] = fmaxf(m[3 + d], __shfl_xor(m[3 + d], o));
-    }
-  if ((threadIdx.x & 63) == 0)
-#pragma unroll
-    for (int d = 0; d < 6; ++d) s[d][threadIdx.x >> 6] = m[d];
-  __syncthreads();
-  if (threadIdx.x < 6) {
-    const int d = threadIdx.x;
-    float r = s[d][0];
-    for (int w = 1; w < BOUNDS_THREADS / 64; ++w) r = d < 3 ? fminf(r, s[d][w]) : fmaxf(r, s[d][w]);
-    bounds[6 * blockIdx.x + d] = r;
-  }
+  for (int e = blockIdx.x * BOUNDS_THREADS + threadIdx.x; e < ne; e += gridDim.x * BOUNDS_THREADS)
+    centre_bounds(ebox[e], m);
+  bounds_row<BOUNDS_THREADS>(m, bounds);
 }
 
 __device__ inline uint32_t expand_bits10(uint32_t v) {
@@ -1341,15 +1363,19 @@ void launch_carry_pairs_from(hipStream_t st, DevState& S, const int2* src, int n
 void launch_element_boxes(hipStream_t st, const DevState& S, double dt, dbox* sbox, dbox* mbox) {
   const int ne = S.ne;
   if (ne == 0) return;
-  hipLaunchKernelGGL(k_element_boxes, dim3((ne + 255) / 256), dim3(256), 0, st, S.ev, S.x, S.x_old,
-                     S.av, dt, ne, sbox, mbox);
+  const int nb = (ne + 255) / 256;
+  hipLaunchKernelGGL(k_element_boxes, dim3(nb), dim3(256), 0, st, S.ev, S.x, S.x_old, S.av, dt, ne,
+                     sbox, mbox, nb <= BOUNDS_BLOCKS ? S.bounds : nullptr);
 }
 
 hipError_t build_bvh(hipStream_t st, DevState& S) {
   const int n = S.ne;
   if (n == 0) return hipSuccess;
-  const int nb = std::min(BOUNDS_BLOCKS, (n + BOUNDS_THREADS - 1) / BOUNDS_THREADS);
-  hipLaunchKernelGGL(k_bounds, dim3(nb), dim3(BOUNDS_THREADS), 0, st, S.ebox, n, S.bounds);
+  int nb = (n + 255) / 256;  // rows that k_element_boxes wrote
+  if (nb > BOUNDS_BLOCKS) {
+    nb = std::min(BOUNDS_BLOCKS, (n + BOUNDS_THREADS - 1) / BOUNDS_THREADS);
+    hipLaunchKernelGGL(k_bounds, dim3(nb), dim3(BOUNDS_THREADS), 0, st, S.ebox, n, S.bounds);
+  }
   hipLaunchKernelGGL(k_morton, dim3((n + 255) / 256), dim3(256), 0, st, S.ebox, n, S.bounds, nb,
                      S.mcode, S.mid);
   bool in_tmp = false;

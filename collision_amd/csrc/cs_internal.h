@@ -425,14 +425,15 @@ hipError_t update_body_zones(hipStream_t st, DevState& S, double m, double dt);
 // updateFinalForRG (dcollid.cpp:626-675)
 void launch_final_bodies(hipStream_t st, DevState& S, double dt);
 void launch_record_origin(hipStream_t st, DevState& S);
-// computeAverageVelocity and the per-vertex state of a resolve (union-find, zone
-// marks and, with record, the recorded impulses)
-void launch_average_velocity(hipStream_t st, DevState& S, double dt, bool record);
+// computeAverageVelocity, with predict after the predictor, and the per-vertex
+// state of a resolve (union-find, zone marks and, with record, the recorded
+// impulses)
+void launch_average_velocity(hipStream_t st, DevState& S, double dt, bool record, bool predict);
 void launch_predict(hipStream_t st, DevState& S, double dt);
 hipError_t update_zones(hipStream_t st, DevState& S, double m, double dt, int nlist);
-void launch_domain_boundary(hipStream_t st, DevState& S, const double lo[3], const double hi[3],
-                            double dt, double mu, double thickness);
-void launch_final_position(hipStream_t st, DevState& S, double dt);
+// detectDomainBoundaryCollision and updateFinalPosition
+void launch_final_position(hipStream_t st, DevState& S, const double lo[3], const double hi[3],
+                           double dt, double mu);
 // marks != nullptr: a pair of events around every k_strain_pipe launch is
 // appended (the caller reads and destroys them)
 hipError_t strain_limit(hipStream_t st, DevState& S, double dt, int max_sweeps,

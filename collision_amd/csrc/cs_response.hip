@@ -43,9 +43,11 @@ __global__ void k_predict(dvec4* __restrict__ x, dvec4* __restrict__ x_old,
 // computeAverageVelocity (dcollid.cpp:160-220), makeSet (dcollid.cpp:1015-1031)
 // and createImpZoneForRG (dcollid3d.cpp:54-68): every point its own zone, every
 // movable body one zone rooted at its smallest vertex; the zone marks and (pimp
-// not null) the recorded impulses of the last resolve are cleared.
-__global__ void k_average_velocity(dvec4* __restrict__ x, const dvec4* __restrict__ x_old,
-                                   dvec4* __restrict__ av, double dt, int nv,
+// not null) the recorded impulses of the last resolve are cleared.  With vel not
+// null the predictor (k_predict) runs first: the velocities are those of its
+// positions, which the step then leaves in favour of x_old, where they were.
+__global__ void k_average_velocity(dvec4* __restrict__ x, dvec4* __restrict__ x_old,
+                                   const dvec4* __restrict__ vel, dvec4* __restrict__ av, double dt, int nv,
                                    int32_t* __restrict__ uf, const int32_t* __restrict__ vbody,
                                    const int32_t* __restrict__ bptr,
                                    const uint32_t* __restrict__ bmem, int32_t* __restrict__ zmark,
@@ -60,7 +62,17 @@ __global__ void k_average_velocity(dvec4* __restrict__ x, const dvec4* __restric
     pimp[v] = dvec4{0.0, 0.0, 0.0, 0.0};
     pnum[v] = 0;
   }
-  const dvec4 p = x[v], o = x_old[v];
+  dvec4 p = x[v], o;
+  if (vel) {
+    const dvec4 u = vel[v];
+    o = p;
+    p.x = o.x + dt * u.x;
+    p.y = o.y + dt * u.y;
+    p.z = o.z + dt * u.z;
+    x_old[v] = o;
+  } else {
+    o = x_old[v];
+  }
   dvec4 a;
   if (dt > CS_ROUND_EPS) {
     a.x = (p.x - o.x) / dt;
@@ -73,7 +85,7 @@ __global__ void k_average_velocity(dvec4* __restrict__ x, const dvec4* __restric
   if (!isfinite(a.x) || !isfinite(a.y) || !isfinite(a.z))
     atomicOr(err, CS_DEVERR_NONFINITE | CS_DEVERR_START);
   av[v] = a;
-  x[v] = o;
+  if (!vel) x[v] = o;
 }
 
 // one record per (hit in canonical order, point)
@@ -572,18 +584,22 @@ void launch_zone_labels(hipStream_t st, DevState& S, int32_t* out) {
 // that leaves the average velocity unchanged leaves every later visit with
 // the same input, so the loop stops there; a later visit can still change a
 // point whose x_old lies outside the box, when the friction of an earlier
-// visit shortens its inward move.  Movable rigid-body points are skipped.
-__global__ void k_domain(dvec4* __restrict__ av, dvec4* __restrict__ x,
-                         const dvec4* __restrict__ x_old, uint8_t* __restrict__ has,
-                         const int32_t* __restrict__ vadj_ptr, const int32_t* __restrict__ vbody,
-                         int nv, double lo0, double lo1, double lo2, double hi0, double hi1,
-                         double hi2, double dt, double mu, double thickness, double mach_eps) {
+// visit shortens its inward move.  Movable rigid-body points are skipped.  The
+// position that the reference sets on a face is overwritten by
+// updateFinalPosition (dcollid.cpp:562-584), which follows and is the end of the
+// same kernel.
+__global__ void k_final_position(dvec4* __restrict__ av, dvec4* __restrict__ x,
+                                 const dvec4* __restrict__ x_old, uint8_t* __restrict__ has,
+                                 const int32_t* __restrict__ vadj_ptr,
+                                 const int32_t* __restrict__ vbody, int nv, double lo0, double lo1,
+                                 double lo2, double hi0, double hi1, double hi2, double dt,
+                                 double mu, double mach_eps) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= nv) return;
-  if (vbody && vbody[v] >= 0) return;
-  const int visits = vadj_ptr[v + 1] - vadj_ptr[v];
-  dvec4 a4 = av[v], o4 = x_old[v], c4 = x[v];
-  double a[3] = {a4.x, a4.y, a4.z}, o[3] = {o4.x, o4.y, o4.z}, c[3] = {c4.x, c4.y, c4.z};
+  const bool body = vbody && vbody[v] >= 0;
+  const int visits = body ? 0 : vadj_ptr[v + 1] - vadj_ptr[v];
+  const dvec4 a4 = av[v], o4 = x_old[v];
+  double a[3] = {a4.x, a4.y, a4.z}, o[3] = {o4.x, o4.y, o4.z};
   const double L[3] = {lo0, lo1, lo2}, U[3] = {hi0, hi1, hi2};
   bool touched = false;
   for (int visit = 0; visit < visits; ++visit) {
@@ -596,12 +612,10 @@ __global__ void k_domain(dvec4* __restrict__ av, dvec4* __restrict__ x,
         touched = true;
         dv = fabs(a[j]);
         a[j] = 0.0;
-        c[j] = L[j] + thickness;
       } else if (cand >= U[j]) {
         touched = true;
         dv = fabs(a[j]);
         a[j] = 0.0;
-        c[j] = U[j] - thickness;
       }
     }
     const double preVt = mag3(a);
@@ -617,29 +631,15 @@ __global__ void k_domain(dvec4* __restrict__ av, dvec4* __restrict__ x,
       break;
   }
   if (touched) has[v] = 1;
-  av[v] = dvec4{a[0], a[1], a[2], 0.0};
-  x[v] = dvec4{c[0], c[1], c[2], 0.0};
+  if (!body) av[v] = dvec4{a[0], a[1], a[2], 0.0};
+  x[v] = dvec4{o[0] + a[0] * dt, o[1] + a[1] * dt, o[2] + a[2] * dt, 0.0};
 }
 
-void launch_domain_boundary(hipStream_t st, DevState& S, const double lo[3], const double hi[3],
-                            double dt, double mu, double thickness) {
-  hipLaunchKernelGGL(k_domain, dim3((S.nv + 255) / 256), dim3(256), 0, st, S.av, S.x, S.x_old,
+void launch_final_position(hipStream_t st, DevState& S, const double lo[3], const double hi[3],
+                           double dt, double mu) {
+  hipLaunchKernelGGL(k_final_position, dim3((S.nv + 255) / 256), dim3(256), 0, st, S.av, S.x, S.x_old,
                      S.has, S.vadj_ptr, S.vbody, S.nv, lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], dt,
-                     mu, thickness, CS_MACH_EPS);
-}
-
-// updateFinalPosition (dcollid.cpp:562-584)
-__global__ void k_final_position(dvec4* __restrict__ x, const dvec4* __restrict__ x_old,
-                                 const dvec4* __restrict__ av, double dt, int nv) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= nv) return;
-  const dvec4 o = x_old[v], a = av[v];
-  x[v] = dvec4{o.x + a.x * dt, o.y + a.y * dt, o.z + a.z * dt, 0.0};
-}
-
-void launch_final_position(hipStream_t st, DevState& S, double dt) {
-  hipLaunchKernelGGL(k_final_position, dim3((S.nv + 255) / 256), dim3(256), 0, st, S.x, S.x_old,
-                     S.av, dt, S.nv);
+                     mu, CS_MACH_EPS);
 }
 
 // updateFinalVelocity (dcollid.cpp:598-624)
@@ -750,9 +750,9 @@ void launch_predict(hipStream_t st, DevState& S, double dt) {
                      dt, S.nv);
 }
 
-void launch_average_velocity(hipStream_t st, DevState& S, double dt, bool record) {
+void launch_average_velocity(hipStream_t st, DevState& S, double dt, bool record, bool predict) {
   hipLaunchKernelGGL(k_average_velocity, dim3((S.nv + 255) / 256), dim3(256), 0, st, S.x, S.x_old,
-                     S.av, dt, S.nv, S.uf, S.vbody, S.bptr, S.bmem, S.zmark,
+                     predict ? S.vel : nullptr, S.av, dt, S.nv, S.uf, S.vbody, S.bptr, S.bmem, S.zmark,
                      record ? S.pimp : nullptr, S.pnum, S.counters + CNT_ERR);
 }
 

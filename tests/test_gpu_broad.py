@@ -24,7 +24,8 @@ def loose_bonds(count, spread, length=0.02):
 
 @pytest.mark.parametrize("full", [0, 1], ids=["incremental", "full"])
 @pytest.mark.parametrize("count,spread", [(1, 0.1), (2, 0.02), (255, 0.3), (256, 0.3), (257, 0.3),
-                                          (513, 0.05), (1025, 0.4), (4097, 0.7)])
+                                          (513, 0.05), (1025, 0.4), (4097, 0.7),
+                                          (32768, 1.5), (32769, 1.5)])
 def test_candidates_match_the_oracle(count, spread, full):
     run_parity(loose_bonds(count, spread), steps=2, gpu_kw=dict(force_full_passes=full))
 
