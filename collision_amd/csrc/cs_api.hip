@@ -1494,7 +1494,7 @@ int cs_predict(cs_solver* h) {
 
 namespace {
 
-// The launches of a resolve before its first host synchronisation (kernels
+// The launches of a resolve before its first pass (kernels
 // only, so that they can be captured in a graph): the dirty marks of the last
 // pass and the counters, the batched scenes' pass state, then
 // computeAverageVelocity with the union-find (makeSet, dcollid.cpp:1015-1031),

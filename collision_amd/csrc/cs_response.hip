@@ -9,7 +9,7 @@
 //    updateAverageVelocity (dcollid.cpp:677-751).  No atomics touch values,
 //    so results are deterministic.
 //  * update_zones: union-find roots (smallest vertex id of each zone) ->
-//    stable sort of vertices by root -> one lane per zone computes the rigid
+//    stable sort of vertices by root -> one wavefront per zone computes the rigid
 //    motion of updateImpactListVelocity (dcollid3d.cpp:70-200) over its
 //    members in ascending vertex id.
 //  * strain_limit: reduceSuperelast (dcollid.cpp:486-596) is an in-place

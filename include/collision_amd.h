@@ -82,8 +82,8 @@ typedef struct cs_params {
                                    largest FP32 error (cs_step_report.mx_*) */
     int32_t graph_step;         /* 1: cs_step / cs_step_batch replay one captured HIP graph
                                    of the predictor and the resolve prologue (every launch
-                                   before the step's first host synchronisation) instead
-                                   of launching them one by one; results are identical */
+                                   before the step's first pass) instead of launching
+                                   them one by one; results are identical */
     int32_t autotune;           /* 1: the first 8 steps after cs_assemble time launch-shape
                                    candidates (cs_tuning) and keep the fastest; with the
                                    environment variable CS_TUNE_CACHE naming a file, the
