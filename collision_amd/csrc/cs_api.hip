@@ -98,6 +98,7 @@ struct cs_solver {
   // pairs of the last full traversal (-1: none yet) of a proximity / a CCD pass:
   // the narrow phase's grid for the next
   int64_t pair_guess[2] = {-1, -1};
+  bool counts_clear = false;  // the last pass's apply has cleared the next one's counts
   unsigned report_seq = 0;  // of the last report of the counters
   int64_t syncs = 0;  // host synchronisations of the current resolve
   LearnedState L;           // time-of-impact proposer (learned form)
@@ -444,19 +445,22 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
   const PrevPass prev = h->prev;
   h->prev.valid = false;
   mark_pass(h, &T.e0, 2);
-  // The dirty marks of the previous pass are cleared, then its counts: pairs,
-  // hits, hit pairs, query pairs, dirty elements, the 64-bit candidate counts,
-  // the dirty-range count and the list of vertices this pass's hits change; the
-  // list of the previous pass (the other parity) is read by this pass.  Before
-  // the proximity pass, the first of a step, the prologue has cleared all.
+  // Counts of a pass, zero when it starts: pairs, hits, hit pairs, query pairs,
+  // dirty elements and ranges, the 64-bit candidate counts and the list of
+  // vertices its hits change (the list of the previous pass, the other parity, is
+  // read).  The apply of the previous pass has cleared them, and before the
+  // proximity pass, the first of a step, the prologue; a pass without hits leaves
+  // them to the next.
+  auto counts_of = [](int pass) {
+    return (1ull << CNT_PAIRS) | (1ull << CNT_HITS) | (1ull << CNT_HIT_PAIRS) | (1ull << CNT_TMP) |
+           (1ull << CNT_QPAIRS) | (1ull << CNT_DIRTY) | (3ull << CNT_TSPLIT) |
+           (0x3full << CNT_CAND64) | (1ull << CNT_DRANGES) | (1ull << (CNT_VLIST + (pass & 1)));
+  };
   int* vcount_cur = S.counters + CNT_VLIST + (pass_id & 1);
   const int* vcount_prev = S.counters + CNT_VLIST + ((pass_id & 1) ^ 1);
-  if (kind != CS_PASS_PROXIMITY)
-    launch_pass_begin(h->st, S,
-                      (1ull << CNT_PAIRS) | (1ull << CNT_HITS) | (1ull << CNT_HIT_PAIRS) |
-                          (1ull << CNT_TMP) | (1ull << CNT_QPAIRS) | (1ull << CNT_DIRTY) |
-                          (3ull << CNT_TSPLIT) | (0x3full << CNT_CAND64) | (1ull << CNT_DRANGES) |
-                          (1ull << (CNT_VLIST + (pass_id & 1))));
+  if (kind != CS_PASS_PROXIMITY && !h->counts_clear)
+    launch_clear_counters(h->st, S, counts_of(pass_id));
+  h->counts_clear = false;
   NarrowParams NP{};
   NP.dt = P.dt; NP.thickness = P.thickness; NP.round_eps = P.round_eps;
   NP.k = P.spring_k; NP.m = P.mass; NP.lambda = P.friction; NP.cr = P.restitution;
@@ -591,7 +595,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
     // vertices that pass's hits changed queried again under their new boxes
     // (the incremental scheme below); no narrow-phase result carries over
     // (the proximity pass ran another test), so every pair is tested.
-    launch_mark_dirty(h->st, S, vcount_prev, 0);
+    HIPCHK(h, launch_mark_dirty(h->st, S, vcount_prev, 0));
     mark_pass(h, &T.t0, 1);
     if (exact_counts) launch_query_dirty(h->st, S, 0, 0, CNT_QPAIRS, 1);  // seed boxes: count only
     launch_grow_carry(h->st, S, P.dt, 0, 0, 0);  // new boxes; leaves exact, ancestors grown
@@ -662,7 +666,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
     // phase appends to them, and overflows are detected afterwards (the
     // narrow phase only appends records and performs idempotent zone
     // merges, so it can be run again).
-    launch_mark_dirty(h->st, S, vcount_prev, prev.nzone);
+    HIPCHK(h, launch_mark_dirty(h->st, S, vcount_prev, prev.nzone));
     mark_pass(h, &T.t0, 1);
     // previous boxes: count only.  The count only feeds the exact candidate
     // total of the pass (a diagnostic), so it runs when the caller asks for
@@ -733,7 +737,8 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
   mark_pass(h, &T.e2, 2);
   launch_scene_pass(h->st, S, kind, index, nhp, P.max_ccd_passes);  // batched scenes
   const int nzone = kind == CS_PASS_ZONE ? h->h_counters[CNT_ZLIST] : 0;
-  HIPCHK(h, apply_hits(h->st, S, nhits, vcount_cur, P.record_impulses != 0 && S.pimp, nzone));
+  HIPCHK(h, apply_hits(h->st, S, nhits, vcount_cur, P.record_impulses != 0 && S.pimp, nzone,
+                       counts_of(pass_id + 1), &h->counts_clear));
   HIPCHK(h, apply_bodies(h->st, S, P.mass, P.dt));  // RG impulses, body zones (updateAverageVelocity)
   if (kind == CS_PASS_ZONE) {
     HIPCHK(h, update_zones(h->st, S, P.mass, P.dt, nzone));
@@ -1261,7 +1266,7 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   HIPCHK(h, dalloc(&S.hp, S.hp_cap));
   HIPCHK(h, dalloc(&S.hp_prev, S.hp_cap));
   HIPCHK(h, dalloc(&S.leaf_of, ne));
-  HIPCHK(h, dalloc(&S.dirty_e, ((size_t)ne + 3) & ~(size_t)3));
+  HIPCHK(h, dalloc(&S.dirty_e, ne));
   HIPCHK(h, dalloc(&S.dlist, ne));
   HIPCHK(h, dalloc(&S.vlist, nv));
   // vertex -> elements, in element order
@@ -1331,11 +1336,12 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   HIPCHK(h, hipMemcpy(S.fixed, fixed.data(), nv, hipMemcpyHostToDevice));
   HIPCHK(h, hipMemset(S.counters, 0, sizeof(int) * COUNTER_INTS));
   HIPCHK(h, hipMemset(S.has, 0, nv));
-  HIPCHK(h, hipMemset(S.dirty_e, 0, ((size_t)ne + 3) & ~(size_t)3));
+  S.dirty_epoch = 0;
+  HIPCHK(h, hipMemset(S.dirty_e, 0, sizeof(uint32_t) * (size_t)ne));
   HIPCHK(h, hipMemcpy(S.vadj_ptr, vptr.data(), sizeof(int32_t) * ((size_t)nv + 1), hipMemcpyHostToDevice));
   HIPCHK(h, hipMemcpy(S.vadj, vadj.data(), sizeof(int32_t) * vadj.size(), hipMemcpyHostToDevice));
-  HIPCHK(h, hipMemset(S.dpre, 0, 2 * (size_t)ne - 1));
-  HIPCHK(h, hipMemset(S.rflag, 0, sizeof(int32_t) * ((2 * (size_t)ne - 1 + QW_RANGE - 1) / QW_RANGE)));
+  HIPCHK(h, hipMemset(S.dpre, 0, sizeof(uint32_t) * (2 * (size_t)ne - 1)));
+  HIPCHK(h, hipMemset(S.rflag, 0, sizeof(uint32_t) * ((2 * (size_t)ne - 1 + QW_RANGE - 1) / QW_RANGE)));
   if (nbody > 0) {
     // members ascending by vertex id, and in order of first appearance in
     // element order (updateFinalForRG's visiting order)
@@ -1502,7 +1508,7 @@ namespace {
 void resolve_prologue(cs_solver* h, bool stats, bool predict) {
   DevState& S = h->S;
   const cs_params& P = h->P;
-  launch_pass_begin(h->st, S, ~0ull);
+  launch_clear_counters(h->st, S, ~0ull);
   if (stats) launch_fill_u32(h->st, S.spread, (int64_t)SPREAD_SLOTS * SPREAD_STRIDE, 0u);
   launch_scene_reset(h->st, S);
   launch_average_velocity(h->st, S, P.dt, P.record_impulses && S.pimp, predict);

@@ -777,12 +777,14 @@ __global__ void __launch_bounds__(256) k_split_seed(const int2* __restrict__ see
 // elements under the previous boxes) + (the same under the new boxes).
 
 
-// dirty_e[e] = element has a dirty vertex; list of dirty elements, each
+// dirty_e[e] = epoch: element has a dirty vertex; list of dirty elements, each
 // once.  The dirty vertices are those the last pass changed: the vertices of
 // its hits (vlist, nvl of them) and, after a zone pass, the movable members
 // of the impact zones (zlist, nzone of them).  Their elements are found
 // through the vertex -> element table, one thread per (vertex, MD_SLOTS-th
-// element); a word atomic on the element's flag byte keeps the first finder.
+// element); an exchange on the element's word keeps the first finder.  The
+// marks are the number of the marking, so none is cleared (a launch per pass,
+// 4 us of about 100, when they were bytes).
 constexpr int MD_SLOTS = 8;
 __global__ void __launch_bounds__(256) k_mark_dirty(const int32_t* __restrict__ vlist,
                                                     const int* __restrict__ vcount,
@@ -790,11 +792,11 @@ __global__ void __launch_bounds__(256) k_mark_dirty(const int32_t* __restrict__ 
                                                     const uint8_t* __restrict__ fixed,
                                                     const int32_t* __restrict__ vadj_ptr,
                                                     const int32_t* __restrict__ vadj,
-                                                    uint8_t* __restrict__ dirty_e,
+                                                    uint32_t* __restrict__ dirty_e, uint32_t epoch,
                                                     int32_t* __restrict__ dlist,
                                                     const int32_t* __restrict__ enode,
-                                                    uint8_t* __restrict__ dpre,
-                                                    int32_t* __restrict__ rflag,
+                                                    uint32_t* __restrict__ dpre,
+                                                    uint32_t* __restrict__ rflag,
                                                     int32_t* __restrict__ rlist,
                                                     int* __restrict__ counters) {
   const int nvl = *vcount;
@@ -819,8 +821,7 @@ __global__ void __launch_bounds__(256) k_mark_dirty(const int32_t* __restrict__ 
       bool first = false;
       if (live) {
         e = vadj[a];
-        const uint32_t bit = 1u << (8 * (e & 3));
-        first = !(atomicOr(reinterpret_cast<uint32_t*>(dirty_e + (e & ~3)), bit) & bit);
+        first = atomicExch(&dirty_e[e], epoch) != epoch;
       }
       const int slot = wave_append(first, &counters[CNT_DIRTY]);
       bool new_range = false;
@@ -829,9 +830,9 @@ __global__ void __launch_bounds__(256) k_mark_dirty(const int32_t* __restrict__ 
         dlist[slot] = e;
         // the leaf, and its QW_RANGE-node range of the pre-order layout
         const int p = enode[e];
-        dpre[p] = 1;
+        dpre[p] = epoch;
         r = p >> QW_RANGE_SHIFT;
-        new_range = atomicExch(&rflag[r], 1) == 0;
+        new_range = atomicExch(&rflag[r], epoch) != epoch;
       }
       const int rs = wave_append(new_range, &counters[CNT_DRANGES]);
       if (new_range) rlist[rs] = r;
@@ -982,8 +983,8 @@ __device__ inline void flush_pairs(int2* buf, int nbuf, int2* __restrict__ qpair
 __global__ void __launch_bounds__(64) k_query_ranges(
     const bvh_node* __restrict__ nodes, const int32_t* __restrict__ nright,
     const dbox* __restrict__ ebox, const int4* __restrict__ ev,
-    const uint8_t* __restrict__ eflags, const uint8_t* __restrict__ dirty_e,
-    const uint8_t* __restrict__ dpre, const int32_t* __restrict__ rlist, int npre, int emit,
+    const uint8_t* __restrict__ eflags, const uint32_t* __restrict__ dirty_e,
+    const uint32_t* __restrict__ dpre, uint32_t epoch, const int32_t* __restrict__ rlist, int npre, int emit,
     int scenes, int snap, int exact,
     int2* __restrict__ qpairs, int qcap, int count, int* __restrict__ counters) {
   __shared__ int32_t fr[2][QW_FCAP];
@@ -1012,7 +1013,7 @@ __global__ void __launch_bounds__(64) k_query_ranges(
     bool act = false;
     if (lane < QW_RANGE && si < npre) {
       me = nodes[si];
-      act = dpre[si];
+      act = dpre[si] == epoch;
     }
     dbox mb{};
     int4 mt{};
@@ -1136,7 +1137,7 @@ __global__ void __launch_bounds__(64) k_query_ranges(
           ob = ebox[e2];
           ot = ev[e2];
           of = eflags[e2];
-          od = dirty_e[e2];
+          od = dirty_e[e2] == epoch;
         }
         // overlaps first (a bit per query), rejects and output afterwards
         uint64_t hits = 0;
@@ -1174,7 +1175,7 @@ __global__ void __launch_bounds__(64) k_query_ranges(
         nd = node.rope;
         const int e2 = node.left;
         if (j == si) continue;
-        const uint8_t od = dirty_e[e2];
+        const bool od = dirty_e[e2] == epoch;
         if (od && j < si) continue;  // counted from e2
         if (!f64_overlap(ebox[e2], mb)) continue;
         take(e, mt, mf, e2, ev[e2], eflags[e2]);
@@ -1190,42 +1191,15 @@ __global__ void __launch_bounds__(64) k_query_ranges(
     atomicAdd((unsigned long long*)(counters + (emit ? CNT_NEW64 : CNT_OLD64)), c);
 }
 
-// Start of a pass (or of a step): clears the dirty marks that the previous pass
-// listed, then the counters whose bits are set in mask, among them the lists'
-// lengths.  The work-group that is done last clears the counters; those that the
-// lists do not need leave at once, also when they start after that (their index
-// is then not below the number needed for empty lists, 1).
-__global__ void __launch_bounds__(256) k_pass_begin(const int32_t* __restrict__ rlist, int npre,
-                                                    uint8_t* __restrict__ dpre,
-                                                    int32_t* __restrict__ rflag,
-                                                    const int32_t* __restrict__ dlist,
-                                                    uint8_t* __restrict__ dirty_e, uint64_t mask,
-                                                    int* counters) {
-  __shared__ int last;
-  const int t = threadIdx.x;
-  const int nr = counters[CNT_DRANGES], nd = counters[CNT_DIRTY];
-  const int per = 256 / QW_RANGE, k0 = t % QW_RANGE;  // ranges per work-group and round
-  const int need = min((int)gridDim.x, max(1, max((nr + per - 1) / per, (nd + 255) / 256)));
-  if ((int)blockIdx.x >= need) return;
-  for (int ri = per * blockIdx.x + t / QW_RANGE; ri < nr; ri += per * need) {
-    const int r = rlist[ri];
-    const int p = QW_RANGE * r + k0;
-    if (p < npre) dpre[p] = 0;
-    if (k0 == 0) rflag[r] = 0;
-  }
-  for (int k = blockIdx.x * 256 + t; k < nd; k += need * 256) dirty_e[dlist[k]] = 0;
-  __syncthreads();
-  if (t == 0) last = need == 1 || atomicAdd(&counters[CNT_TICKET], 1) == need - 1;
-  __syncthreads();
-  if (last && t < CNT_INTS && (t == CNT_TICKET || (mask >> t & 1ull))) counters[t] = 0;
+__global__ void k_clear_counters(uint64_t mask, int* __restrict__ counters) {
+  clear_counters(mask, counters);
 }
-static_assert(CNT_INTS <= 64, "one bit of the mask per counter");
 
 // carry clean pairs of the previous pass
 constexpr int CARRY_ITEMS = 16;
 __global__ void __launch_bounds__(256) k_carry_pairs(const int2* __restrict__ prev, int n,
-                                                     const uint8_t* __restrict__ dirty_e,
-                                                     int2* __restrict__ cur, int cap,
+                                                     const uint32_t* __restrict__ dirty_e,
+                                                     uint32_t epoch, int2* __restrict__ cur, int cap,
                                                      int* __restrict__ counters) {
   __shared__ int s_off[256];
   __shared__ int s_base;
@@ -1240,7 +1214,7 @@ __global__ void __launch_bounds__(256) k_carry_pairs(const int2* __restrict__ pr
     keep[q] = false;
     if (i < n) {
       p[q] = prev[i];
-      keep[q] = !dirty_e[p[q].x] && !dirty_e[p[q].y];
+      keep[q] = dirty_e[p[q].x] != epoch && dirty_e[p[q].y] != epoch;
     }
     nk += keep[q] ? 1 : 0;
   }
@@ -1267,7 +1241,8 @@ struct CarryArgs {
   const hit_rec* hits_prev;
   const int4* hp_prev;
   int nhits, nhp;
-  const uint8_t* dirty_e;
+  const uint32_t* dirty_e;
+  uint32_t epoch;
   hit_rec* hits;
   uint64_t* hkey;
   int hit_cap, hb;
@@ -1294,7 +1269,7 @@ __global__ void __launch_bounds__(256) k_grow_carry(GrowArgs G, CarryArgs C, int
     if (i < C.nhits) {
       key = C.hits_prev[i].key;
       const int lo = (int)(key >> 36), hi = (int)((key >> 8) & 0xFFFFFFFull);
-      keep = !C.dirty_e[lo] && !C.dirty_e[hi];
+      keep = C.dirty_e[lo] != C.epoch && C.dirty_e[hi] != C.epoch;
     }
     const int slot = block_append(keep, &counters[CNT_HITS], &s_cnt, &s_base);
     if (keep && slot < C.hit_cap) {
@@ -1307,7 +1282,7 @@ __global__ void __launch_bounds__(256) k_grow_carry(GrowArgs G, CarryArgs C, int
     bool keep = false;
     if (i < C.nhp) {
       r = C.hp_prev[i];
-      keep = !C.dirty_e[r.x] && !C.dirty_e[r.y];
+      keep = C.dirty_e[r.x] != C.epoch && C.dirty_e[r.y] != C.epoch;
     }
     const int slot = block_append(keep, &counters[CNT_HIT_PAIRS], &s_cnt, &s_base);
     if (keep && slot < C.hp_cap) C.hp[slot] = r;
@@ -1318,17 +1293,24 @@ __global__ void __launch_bounds__(256) k_grow_carry(GrowArgs G, CarryArgs C, int
   }
 }
 
-void launch_mark_dirty(hipStream_t st, DevState& S, const int* vcount, int nzone) {
+hipError_t launch_mark_dirty(hipStream_t st, DevState& S, const int* vcount, int nzone) {
+  if (++S.dirty_epoch == 0) {  // after 2^32 - 1 markings the old numbers come again
+    const size_t npre = 2 * (size_t)S.ne - 1;
+    CS_HIP_RET(hipMemsetAsync(S.dirty_e, 0, sizeof(uint32_t) * (size_t)S.ne, st));
+    CS_HIP_RET(hipMemsetAsync(S.dpre, 0, sizeof(uint32_t) * npre, st));
+    CS_HIP_RET(hipMemsetAsync(S.rflag, 0, sizeof(uint32_t) * ((npre + QW_RANGE - 1) / QW_RANGE), st));
+    S.dirty_epoch = 1;
+  }
   // grid for a typical list; longer lists are walked grid-stride
   hipLaunchKernelGGL(k_mark_dirty, dim3(std::min((MD_SLOTS * S.nv + 255) / 256, 256)), dim3(256),
                      0, st, S.vlist, vcount, S.zlist, nzone, S.fixed, S.vadj_ptr, S.vadj,
-                     S.dirty_e, S.dlist, S.leaf_of, S.dpre, S.rflag, S.rlist, S.counters);
+                     S.dirty_e, S.dirty_epoch, S.dlist, S.leaf_of, S.dpre, S.rflag, S.rlist,
+                     S.counters);
+  return hipGetLastError();
 }
 
-void launch_pass_begin(hipStream_t st, DevState& S, uint64_t mask) {
-  const int npre = std::max(2 * S.ne - 1, 0);
-  hipLaunchKernelGGL(k_pass_begin, dim3(std::min(npre / 256 + 1, 512)), dim3(256), 0, st, S.rlist,
-                     npre, S.dpre, S.rflag, S.dlist, S.dirty_e, mask, S.counters);
+void launch_clear_counters(hipStream_t st, DevState& S, uint64_t mask) {
+  hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(64), 0, st, mask, S.counters);
 }
 
 void launch_grow_carry(hipStream_t st, DevState& S, double dt, int nhits_prev, int nhp_prev,
@@ -1336,7 +1318,7 @@ void launch_grow_carry(hipStream_t st, DevState& S, double dt, int nhits_prev, i
   if (S.ne == 0) return;
   const GrowArgs G{S.ev, S.x_old, S.av, dt, S.dlist, S.ebox, S.leaf_of, S.nodes, S.parent,
                    S.ne >= 2 ? 1 : 0};
-  const CarryArgs C{S.hits_prev, S.hp_prev, nhits_prev, nhp_prev, S.dirty_e, S.hits, S.hkey,
+  const CarryArgs C{S.hits_prev, S.hp_prev, nhits_prev, nhp_prev, S.dirty_e, S.dirty_epoch, S.hits, S.hkey,
                     S.hit_cap, hit_id_bits(S), S.hp, S.hp_cap, zone, S.ev, S.vbody, zone_list(S)};
   const int bh = (nhits_prev + 255) / 256, bp = (nhp_prev + 255) / 256;
   // growth: grid for a typical dirty list; longer lists are walked grid-stride
@@ -1348,7 +1330,7 @@ void launch_query_dirty(hipStream_t st, DevState& S, int emit, int snap, int cou
   if (S.ne < 2) return;
   const int npre = 2 * S.ne - 1;
   hipLaunchKernelGGL(k_query_ranges, dim3(std::min((npre + 63) / 64, S.tune_query)), dim3(64), 0, st,
-                     S.nodes, S.nright, S.ebox, S.ev, S.eflags, S.dirty_e, S.dpre, S.rlist, npre,
+                     S.nodes, S.nright, S.ebox, S.ev, S.eflags, S.dirty_e, S.dpre, S.dirty_epoch, S.rlist, npre,
                      emit, S.nscene > 1, snap, exact, count == CNT_PAIRS ? S.pairs : S.qpairs,
                      count == CNT_PAIRS ? S.pair_cap : S.qpair_cap, count, S.counters);
 }
@@ -1356,7 +1338,7 @@ void launch_query_dirty(hipStream_t st, DevState& S, int emit, int snap, int cou
 void launch_carry_pairs_from(hipStream_t st, DevState& S, const int2* src, int n) {
   if (n > 0)
     hipLaunchKernelGGL(k_carry_pairs, dim3((n + 256 * CARRY_ITEMS - 1) / (256 * CARRY_ITEMS)), dim3(256), 0, st,
-                       src, n, S.dirty_e, S.pairs, S.pair_cap, S.counters);
+                       src, n, S.dirty_e, S.dirty_epoch, S.pairs, S.pair_cap, S.counters);
 }
 
 // ---------------------------------------------------------------------------

@@ -36,7 +36,6 @@ enum {
   CNT_LOG = 4,           // pair-log rows
   CNT_TMP = 5,           // LBVH nodes spanning refit tiles
   CNT_ZONES = 6,         // impact zones updated
-  CNT_TICKET = 7,        // work-groups of launch_pass_begin that are done
   CNT_STRAIN_FLAG = 8,   // strain sweep state
   CNT_STRAIN_EDGES = 9,
   CNT_STRAIN_DEGEN = 10,
@@ -211,8 +210,9 @@ struct DevState {
   size_t scan_part_words = 0;
   int32_t* leaf_of = nullptr;    // element -> pre-order index of its leaf
   // dirty leaves by pre-order index, and the QW_RANGE-node ranges holding them
-  uint8_t* dpre = nullptr;
-  int32_t *rflag = nullptr, *rlist = nullptr;
+  uint32_t* dpre = nullptr;
+  uint32_t* rflag = nullptr;
+  int32_t* rlist = nullptr;
   void* tq = nullptr;              // split walks of the full traversal, 2 x TRAV_QCAP items
   int num_cus = 256;               // compute units of the device
   // launch shapes (cs_set_tuning / the autotuner): traversal work-groups per
@@ -232,7 +232,8 @@ struct DevState {
   int4* hp_prev = nullptr;
   int hp_cap = 0;
   // vertices / elements whose average velocity changed since the last narrow phase
-  uint8_t* dirty_e = nullptr;   // padded to whole 32-bit words (word atomics mark it)
+  uint32_t* dirty_e = nullptr;  // element, node (dpre) or range (rflag) is dirty: it holds
+  uint32_t dirty_epoch = 0;     // the number of the last marking (no marks to clear)
   int32_t* dlist = nullptr;
   dbox* pbox = nullptr;         // static (proximity) boxes, beside the swept ones in ebox
   int2* pairs_seed = nullptr;   // swept-box candidate pairs of the proximity pass
@@ -378,9 +379,9 @@ void launch_split_seed(hipStream_t st, DevState& S, int first, int n);
 // incremental passes
 // elements of the vertices the previous pass changed: *vcount hit vertices
 // in vlist and nzone zone members in zlist
-void launch_mark_dirty(hipStream_t st, DevState& S, const int* vcount, int nzone);
-// clears the dirty marks of the previous pass and the counters in the mask
-void launch_pass_begin(hipStream_t st, DevState& S, uint64_t mask);
+hipError_t launch_mark_dirty(hipStream_t st, DevState& S, const int* vcount, int nzone);
+// clears the counters in the mask
+void launch_clear_counters(hipStream_t st, DevState& S, uint64_t mask);
 constexpr int QW_RANGE_SHIFT = 3;
 constexpr int QW_RANGE = 1 << QW_RANGE_SHIFT;  // pre-order nodes per dirty-query range
 // snap: the counts carried into the pass are kept in CNT_SNAP..; count: the
@@ -414,8 +415,11 @@ inline int hit_id_bits(const DevState& S) {
   while (hb < 32 && ((uint64_t)S.ne >> hb) != 0) ++hb;
   return hb;
 }
-// nzone > 0: also the sort keys of the zone members, for update_zones
-hipError_t apply_hits(hipStream_t st, DevState& S, int nhits, int* vcount, bool record, int nzone);
+// nzone > 0: also the sort keys of the zone members, for update_zones; the
+// counters in `clear` are zeroed for the next pass (*cleared: false when nothing
+// had to be launched)
+hipError_t apply_hits(hipStream_t st, DevState& S, int nhits, int* vcount, bool record, int nzone,
+                      uint64_t clear, bool* cleared);
 // movable bodies, after apply_hits: the RG part of updateAverageVelocity
 // (dcollid.cpp:728-734) and, when dt > 0, updateImpactZoneVelocityForRG
 // (dcollid.cpp:267-288): every body zone moved rigidly
@@ -470,6 +474,12 @@ __device__ inline int xcd_block(int b, int G) {
 
 // slot in a list for the lanes with want set, one atomic per wavefront;
 // every active lane of the wavefront calls it
+// one wavefront of a kernel zeroes the counters in the mask
+static_assert(CNT_INTS <= 64, "one bit of the mask per counter");
+__device__ inline void clear_counters(uint64_t mask, int* counters) {
+  if (threadIdx.x < CNT_INTS && (mask >> threadIdx.x & 1ull)) counters[threadIdx.x] = 0;
+}
+
 __device__ inline int wave_append(bool want, int* counter) {
   const uint64_t m = __ballot(want);
   if (m == 0) return -1;

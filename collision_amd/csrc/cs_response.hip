@@ -126,14 +126,18 @@ struct ZoneKeys {
 // it; each vertex heads one segment).  A body segment (key nv + body) adds
 // its spreads to the body's collsnImpulse_RG in canonical order, starting
 // from the value it holds (the reference never clears it), and counts them.
-// The work-groups from `nba` on compute the zone members' sort keys.
+// The work-groups from `nba` on compute the zone members' sort keys; the first
+// work-group clears counters for the next pass.
 __global__ void k_apply(const uint32_t* __restrict__ rkey, const uint32_t* __restrict__ rval,
                         int nrec, int nv, int nbody, const hit_rec* __restrict__ hits,
                         dvec4* __restrict__ av, uint8_t* __restrict__ has,
                         dvec4* __restrict__ rg_imp, int32_t* __restrict__ rg_num,
                         int32_t* __restrict__ vlist, int* __restrict__ vcount,
                         dvec4* __restrict__ pimp, int32_t* __restrict__ pnum,
-                        int* __restrict__ err, int nba, ZoneKeys Z) {
+                        int* __restrict__ counters, uint64_t clear, int nba, ZoneKeys Z) {
+  int* err = counters + CNT_ERR;
+  // (nothing between this kernel and the next pass reads them)
+  if (blockIdx.x == 0) clear_counters(clear, counters);
   if ((int)blockIdx.x >= nba) {
     const int i = (blockIdx.x - nba) * blockDim.x + threadIdx.x;
     if (i == 0) *Z.zones = 0;
@@ -212,8 +216,10 @@ static int vertex_bits(const DevState& S) {
   return b;
 }
 
-hipError_t apply_hits(hipStream_t st, DevState& S, int nhits, int* vcount, bool record, int nzone) {
-  if (nhits <= 0 && nzone <= 0) return hipSuccess;
+hipError_t apply_hits(hipStream_t st, DevState& S, int nhits, int* vcount, bool record, int nzone,
+                      uint64_t clear, bool* cleared) {
+  *cleared = nhits > 0 || nzone > 0;
+  if (!*cleared) return hipSuccess;
   const uint32_t *rk = nullptr, *rv = nullptr;
   const int nrec = 4 * std::max(nhits, 0);
   if (nhits > 0) {
@@ -241,7 +247,7 @@ hipError_t apply_hits(hipStream_t st, DevState& S, int nhits, int* vcount, bool 
   const int nba = (nrec + 255) / 256, nbz = (std::max(nzone, 0) + 255) / 256;
   hipLaunchKernelGGL(k_apply, dim3(nba + nbz), dim3(256), 0, st, rk, rv, nrec, S.nv,
                      S.nbody, S.hits, S.av, S.has, S.rg_imp, S.rg_num, S.vlist, vcount,
-                     record ? S.pimp : nullptr, S.pnum, S.counters + CNT_ERR, nba, Z);
+                     record ? S.pimp : nullptr, S.pnum, S.counters, clear, nba, Z);
   return hipGetLastError();
 }
 
