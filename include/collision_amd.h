@@ -317,7 +317,7 @@ int cs_learned_get_stats(cs_solver *h, cs_learned_stats *out);
 
 /* ---- launch shapes (no counterpart in the reference) ----
  * the full traversal's grid (at most 8 x 4, 8, 16 or 32 work-groups per CU),
- * narrow-phase work-group size (64, 128, 256) and the dirty-element query's grid cap
+ * narrow-phase work-group size for whole streams (64, 128, 256) and the dirty-element query's grid cap
  * (1024 .. 8192); the results of a step do not depend on them */
 typedef struct cs_tuning {
     int32_t traverse_blocks_per_cu;
