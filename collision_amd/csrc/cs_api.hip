@@ -930,6 +930,7 @@ hipError_t upload_plan(DevState& S, const StrainPlan& P) {
   B.nband = P.nband;
   B.n_levels = P.n_levels;
   B.cap = P.cap;
+  B.steps = (int64_t)P.steps();
   std::vector<uint8_t> host;
   std::vector<std::pair<void**, size_t>> at;
   auto put = [&](auto** dst, const auto& v) {

@@ -143,6 +143,10 @@ constexpr int SB_PROG_STRIDE = 16;  // ints between two tasks' progress words (6
 constexpr int SB_STAT_INTS = 32;
 struct StrainBands {
   int nband = 0, n_levels = 0, cap = 0;
+  int64_t steps = 0;        // of one sweep, all bands together
+  // device clock ticks after which a wait gives up, and the most that count
+  // between two looks at the clock
+  long long wait_ticks = 0, look_ticks = 0;
   uint8_t* blob = nullptr;  // the allocation of everything below but the records
   StrainRec* rec = nullptr;
   int32_t *step_ptr = nullptr, *step_level = nullptr;
@@ -443,7 +447,7 @@ void launch_final_position(hipStream_t st, DevState& S, const double lo[3], cons
 hipError_t strain_limit(hipStream_t st, DevState& S, double dt, int max_sweeps,
                         std::vector<hipEvent_t>* marks);
 // cs_strain.hip: the same by bands (S.bands.nband > 0)
-hipError_t strain_bands_setup(const DevState& S);
+hipError_t strain_bands_setup(DevState& S);
 hipError_t strain_limit_bands(hipStream_t st, DevState& S, double dt, int max_sweeps,
                               std::vector<hipEvent_t>* marks);
 // cs_schedule.hip (host)

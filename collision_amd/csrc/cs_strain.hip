@@ -47,7 +47,7 @@ namespace {
 
 constexpr int SB_IMPORT = STRAIN_IMPORT_WAVES;
 constexpr int SB_THREADS = 64 * (2 + SB_IMPORT);
-constexpr int SB_SPIN = 1 << 24;  // polls before a wait gives up (seconds; it then reports an error)
+constexpr int SB_POLLS = 256;  // polls of a wait between looks at the clock and the abort flags
 
 // words of DevState::bands.stat
 enum { SBS_TICKET = 0, SBS_DONE = 1, SBS_EDGES = 2, SBS_DEGEN = 2 + SB_MAX_SWEEPS, SBS_EVALS, SBS_ABORT };
@@ -81,16 +81,26 @@ __device__ inline void lds_publish(int* p, int v) {
   if ((threadIdx.x & 63) == 0) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// spin bookkeeping of one wait: false when it must be given up
+// The bookkeeping of one wait: false when it must be given up, because another
+// wait was or because it has lasted longer than all steps of the launch could
+// take one after another (strain_wait_us; only an inconsistent plan does).  It
+// is measured in time, not in polls: a wait in LDS polls some ten times faster
+// than one in memory.  Time between two looks counts up to B.look_ticks, so
+// that a wavefront that was not running meanwhile does not run out of it.
 struct Spin {
   int n = 0;
-  __device__ inline bool go(const int* s_abort, int* stat) {
-    if (++n & 255) return true;
+  long long last = 0, ticks = 0;
+  __device__ inline bool go(const int* s_abort, const StrainBands& B) {
+    if (++n < SB_POLLS) return true;
+    n = 0;
     if (lds_load(s_abort)) return false;
-    if (__hip_atomic_load(stat + SBS_ABORT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
-    if (n >= SB_SPIN) {
+    if (__hip_atomic_load(B.stat + SBS_ABORT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
+    const long long now = (long long)wall_clock64();
+    if (last) ticks += min(now - last, B.look_ticks);
+    last = now;
+    if (ticks >= B.wait_ticks) {
       if ((threadIdx.x & 63) == 0)
-        __hip_atomic_store(stat + SBS_ABORT, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(B.stat + SBS_ABORT, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return false;
     }
     return true;
@@ -247,7 +257,7 @@ __global__ void __launch_bounds__(SB_THREADS)
       const int g = s >> 2;
       if ((s & 63) == 0 && s > 0) lv = B.step_level[step0 + min(s + lane, nstep)];
       for (Spin sp; lds_load(&s_imp[g % SB_IMPORT]) <= g;) {
-        if (!sp.go(&s_abort, stat)) {
+        if (!sp.go(&s_abort, B)) {
           ok = false;
           break;
         }
@@ -364,7 +374,7 @@ __global__ void __launch_bounds__(SB_THREADS)
           seen = v;
           return true;
         }
-        if (!sp.go(&s_abort, stat)) return false;
+        if (!sp.go(&s_abort, B)) return false;
         __builtin_amdgcn_s_sleep(1);
       }
     };
@@ -400,7 +410,7 @@ __global__ void __launch_bounds__(SB_THREADS)
       }
       // places of vertices that left more than STRAIN_AHEAD groups ago
       for (Spin sp; lds_load(&s_done) < STRAIN_GROUP * (g - STRAIN_AHEAD);) {
-        if (!sp.go(&s_abort, stat)) {
+        if (!sp.go(&s_abort, B)) {
           ok = false;
           break;
         }
@@ -460,7 +470,7 @@ __global__ void __launch_bounds__(SB_THREADS)
     for (int done = 0; done < nstep;) {
       int n = done;
       for (Spin sp; (n = lds_load(&s_step)) <= done;) {
-        if (!sp.go(&s_abort, stat)) {
+        if (!sp.go(&s_abort, B)) {
           ok = false;
           break;
         }
@@ -521,7 +531,13 @@ __global__ void __launch_bounds__(SB_THREADS)
   }
 }
 
-hipError_t strain_bands_setup(const DevState& S) {
+hipError_t strain_bands_setup(DevState& S) {
+  StrainBands& B = S.bands;
+  int device = 0, khz = 0;
+  CS_HIP_RET(hipGetDevice(&device));
+  CS_HIP_RET(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device));
+  B.wait_ticks = strain_wait_us(B.steps, SB_MAX_SWEEPS) * khz / 1000;
+  B.look_ticks = 10ll * khz;  // 10 ms
   if ((size_t)S.bands.cap * sizeof(BandVertex) <= 65536) return hipSuccess;
   // (the same bound for every handle: a later, smaller one must not lower it)
   return hipFuncSetAttribute(reinterpret_cast<const void*>(k_strain_bands),

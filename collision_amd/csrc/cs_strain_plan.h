@@ -162,6 +162,13 @@ inline int strain_band_count(int64_t nsched, int n_levels) {
   return n;
 }
 
+// Microseconds after which a wait of a task means that the plan is broken.  A
+// task may wait for everything before it: where a vertex's visits span all levels
+// (a ring of bonds, a fan) sweep k only begins when sweep k - 1 is nearly over, and
+// bands can depend on each other in the same way.  A step takes 0.2 to 1 us, its
+// imports and exports included about 2, so 5 for each step of each sweep.
+inline int64_t strain_wait_us(int64_t steps, int sweeps) { return 2000000 + 5 * steps * sweeps; }
+
 // Whole components much shorter than the schedule (strings, small pieces) are
 // moved to other levels, first fit: at most STRAIN_SHIFT_WIDTH elements of the
 // band their first element lies in on any level they occupy (the fewest where
