@@ -1443,9 +1443,9 @@ int cs_set_state(cs_solver* h, const double* x, const double* vel, const uint8_t
     HIPCHK(h, hipMemcpyAsync(S.stage + n3, vel, sizeof(double) * n3, hipMemcpyHostToDevice, h->st));
     if (has_collsn) HIPCHK(h, hipMemcpyAsync(hc, has_collsn, S.nv, hipMemcpyHostToDevice, h->st));
     launch_unpack_state(h->st, S, S.stage, S.stage + n3, has_collsn ? hc : nullptr);
-    HIPCHK(h, hipStreamSynchronize(h->st));  // the caller may reuse its arrays
   }
   HIPCHK(h, hipGetLastError());
+  HIPCHK(h, hipStreamSynchronize(h->st));  // (the caller may reuse its arrays)
   if (S.nbody > 0) {  // initSurfaceState clears the RG accumulators (cdinit.cpp:192-197)
     HIPCHK(h, hipMemset(S.rg_imp, 0, sizeof(dvec4) * S.nbody));
     HIPCHK(h, hipMemset(S.rg_num, 0, sizeof(int32_t) * S.nbody));
