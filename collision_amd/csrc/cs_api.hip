@@ -950,20 +950,23 @@ hipError_t upload_plan(DevState& S, const StrainPlan& P) {
   put(&B.lo, P.lo);
   put(&B.up_ptr, P.up_ptr);
   put(&B.up, P.up);
-  put(&B.slot, P.slot);
+  put(&B.row_ptr, P.rec.first);
+  std::vector<int32_t> slot(P.slot.size());
+  for (size_t e = 0; e < slot.size(); ++e) slot[e] = P.slot[e] < 0 ? -1 : P.rec.at((size_t)P.slot[e]);
+  put(&B.slot, slot);
   size_t total = host.size();
   auto reserve = [&](auto** dst, size_t bytes) {
     const size_t off = (total + 255) & ~(size_t)255;
     total = off + bytes;
     at.push_back({(void**)dst, off});
   };
-  reserve(&B.pre, P.rec.size());
+  reserve(&B.pre, P.rec.packed.size());
   reserve(&B.prog, sizeof(int) * (size_t)SB_MAX_SWEEPS * P.nband * SB_PROG_STRIDE);
   reserve(&B.stat, sizeof(int) * SB_STAT_INTS);
   CS_HIP_RET(dalloc(&B.blob, total));
   for (auto& a : at) *a.first = B.blob + a.second;
   CS_HIP_RET(hipMemcpy(B.blob, host.data(), host.size(), hipMemcpyHostToDevice));
-  CS_HIP_RET(upload(&B.rec, P.rec));
+  CS_HIP_RET(upload(&B.rec, P.rec.packed));
   return strain_bands_setup(S);
 }
 

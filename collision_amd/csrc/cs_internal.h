@@ -150,6 +150,7 @@ struct StrainBands {
   uint8_t* blob = nullptr;  // the allocation of everything below but the records
   StrainRec* rec = nullptr;
   int32_t *step_ptr = nullptr, *step_level = nullptr;
+  int32_t* row_ptr = nullptr;  // first record of every step
   int32_t* grp_ptr = nullptr;
   StrainGroup* grp = nullptr;
   StrainImport* imp = nullptr;

@@ -237,25 +237,36 @@ __global__ void __launch_bounds__(SB_THREADS)
   const int NL = B.n_levels;
   int* stat = B.stat;
   if (wave == 0) {
-    // --- the steps.  Records (static, one 2 KB row per step) are loaded one
-    // group ahead into registers.
+    // --- the steps.  Records (static) are loaded one group ahead into
+    // registers.  The lanes past the step's last element hold that one's record
+    // (so that their stamp reads meet it in LDS and not in other banks) and take
+    // no part.
     static_assert(STRAIN_GROUP == 4, "unrolled by hand");
-    const StrainRec* rec = B.rec + (size_t)step0 * STRAIN_STEP_SLOTS + lane;
-    const uint8_t* pre = B.pre + (size_t)step0 * STRAIN_STEP_SLOTS + lane;
+    const int32_t* row_ptr = B.row_ptr + step0;
     StrainRec r[4];
-    int pr[4];
+    int pr[4], n[4];
+    // step u's record and pre-check byte: records [row, end), none past the last step
+    // (one past it is read then)
+    auto load = [&](int u, int row, int end) {
+      n[u] = end - row;
+      const unsigned i = min(lane, max(end - row - 1, 0));
+      r[u] = (B.rec + row)[i];
+      pr[u] = k == 0 ? (B.pre + row)[i] : 0;
+    };
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const size_t row = (size_t)min(u, nstep - 1) * STRAIN_STEP_SLOTS;
-      r[u] = rec[row];
-      pr[u] = k == 0 ? pre[row] : 0;
-    }
+    for (int u = 0; u < 4; ++u) load(u, row_ptr[min(u, nstep)], row_ptr[min(u + 1, nstep)]);
+    // of the 64 steps from s on: levels; first records a group later, and one more
     int lv = B.step_level[step0 + min(lane, nstep)];
+    int rw = row_ptr[min(4 + lane, nstep)], rw1 = row_ptr[min(5 + lane, nstep)];
     int edges = 0, degen = 0, evals = 0;
     bool ok = true;
     for (int s = 0; s < nstep && ok; s += 4) {
       const int g = s >> 2;
-      if ((s & 63) == 0 && s > 0) lv = B.step_level[step0 + min(s + lane, nstep)];
+      if ((s & 63) == 0 && s > 0) {
+        lv = B.step_level[step0 + min(s + lane, nstep)];
+        rw = row_ptr[min(s + 4 + lane, nstep)];
+        rw1 = row_ptr[min(s + 5 + lane, nstep)];
+      }
       for (Spin sp; lds_load(&s_imp[g % SB_IMPORT]) <= g;) {
         if (!sp.go(&s_abort, B)) {
           ok = false;
@@ -280,7 +291,7 @@ __global__ void __launch_bounds__(SB_THREADS)
         if (wrote) stamps(u);
         // (place[2] of a bond repeats place[0])
         const StrainRec& q = r[u];
-        const bool act = s + u < nstep && q.np && (pr[u] || t[u][0] >= thr || t[u][1] >= thr || t[u][2] >= thr);
+        const bool act = lane < n[u] && (pr[u] || t[u][0] >= thr || t[u][1] >= thr || t[u][2] >= thr);
         if (__ballot(act)) {
           if (act) {
             BandVertex* w[3] = {win + q.place[0], win + q.place[1], win + q.place[2]};
@@ -335,11 +346,8 @@ __global__ void __launch_bounds__(SB_THREADS)
           wrote = true;
           lds_publish(&s_step, min(s + u + 1, nstep));
         }
-        // the record of the same step of the next group (no branch on the
-        // band's end: the row of the last step is read again)
-        const size_t row = (size_t)min(s + u + 4, nstep - 1) * STRAIN_STEP_SLOTS;
-        r[u] = rec[row];
-        pr[u] = k == 0 ? pre[row] : 0;
+        // the same step of the next group
+        load(u, __builtin_amdgcn_readlane(rw, (s + u) & 63), __builtin_amdgcn_readlane(rw1, (s + u) & 63));
       }
       lds_publish(&s_step, min(s + 4, nstep));
     }
@@ -383,7 +391,7 @@ __global__ void __launch_bounds__(SB_THREADS)
     // The entries of a group are loaded while the group before it is
     // fetched, their x_old (constant) before the waits.
     StrainImport e[2] = {};
-    StrainGroup G{0, 0, -1, -1}, Gn = G;
+    StrainGroup G{0, 0, -1, -1, 0, 0}, Gn = G;
     if (wave - 1 < ngrp) {
       G = B.grp[grp0 + wave - 1];
 #pragma unroll
@@ -401,12 +409,10 @@ __global__ void __launch_bounds__(SB_THREADS)
       if (g + SB_IMPORT < ngrp) Gn = B.grp[grp0 + g + SB_IMPORT];
       else Gn.imp0 = Gn.imp1 = 0;
       uint32_t warm = 0u, warmp = 0u;
-      {  // bring the group's records (64 lines of 128 B) and pre-check bytes into L2
-        const int f = STRAIN_GROUP * g, n = min(STRAIN_GROUP, nstep - f);
-        const char* p = reinterpret_cast<const char*>(B.rec + (size_t)(step0 + f) * STRAIN_STEP_SLOTS);
-        if (128 * lane < n * STRAIN_STEP_SLOTS * (int)sizeof(StrainRec))
-          warm = *reinterpret_cast<const uint32_t*>(p + 128 * lane);
-        if (k == 0 && lane < n) warmp = B.pre[(size_t)(step0 + f + lane) * STRAIN_STEP_SLOTS];
+      {  // bring the group's records (up to 64 lines of 128 B) and pre-check bytes into L2
+        const int n = G.rec1 - G.rec0;
+        if (4 * lane < n) warm = *reinterpret_cast<const uint32_t*>(B.rec + G.rec0 + 4 * lane);
+        if (k == 0 && STRAIN_STEP_SLOTS * lane < n) warmp = B.pre[G.rec0 + STRAIN_STEP_SLOTS * lane];
       }
       // places of vertices that left more than STRAIN_AHEAD groups ago
       for (Spin sp; lds_load(&s_done) < STRAIN_GROUP * (g - STRAIN_AHEAD);) {

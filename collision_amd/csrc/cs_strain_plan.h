@@ -39,7 +39,7 @@ constexpr int STRAIN_VERT_BYTES = 56;
 constexpr int STRAIN_LDS_VERTS = 2560;  // vertices of a task's LDS window (140 KB of the 160)
 
 // one element of a step, 32 B: rest lengths of edges (0,1), (1,2), (2,0), the
-// LDS places of its vertices, its vertex count (0: unused lane)
+// LDS places of its vertices, its vertex count
 struct StrainRec {
   double L0[3];
   uint16_t place[3];
@@ -49,9 +49,10 @@ struct StrainImport {
   uint32_t v, place;
 };
 // imports of a group of steps, and the levels they wait for (-1: none): of
-// lower bands in the same sweep, of this and higher bands in the previous one
+// lower bands in the same sweep, of this and higher bands in the previous one;
+// the group's records
 struct StrainGroup {
-  int32_t imp0, imp1, need_same, need_prev;
+  int32_t imp0, imp1, need_same, need_prev, rec0, rec1;
 };
 struct StrainExport {
   uint32_t v;
@@ -60,11 +61,26 @@ struct StrainExport {
   int32_t pad;
 };
 
+// The records of all steps one after another, so that a step takes the room of
+// its elements (rows of STRAIN_STEP_SLOTS took 2 KB each, 2 GB for one string of
+// 10^6 bonds).  Read as rows: element i % STRAIN_STEP_SLOTS of step
+// i / STRAIN_STEP_SLOTS, vertex count 0 where the step has fewer elements.
+struct StrainRows {
+  std::vector<StrainRec> packed;     // (+ STRAIN_STEP_SLOTS unused ones at the end)
+  std::vector<int32_t> first{0};     // [steps + 1] first record of each step
+  size_t size() const { return (first.size() - 1) * STRAIN_STEP_SLOTS; }
+  int32_t at(size_t i) const { return first[i / STRAIN_STEP_SLOTS] + (int32_t)(i % STRAIN_STEP_SLOTS); }
+  const StrainRec& operator[](size_t i) const {
+    static const StrainRec none{};
+    return at(i) < first[i / STRAIN_STEP_SLOTS + 1] ? packed[(size_t)at(i)] : none;
+  }
+};
+
 struct StrainPlan {
   int nband = 0, n_levels = 0, cap = 0;   // cap: LDS places of the largest window
   std::vector<int32_t> step_ptr;          // [nband + 1] steps of each band
   std::vector<int32_t> step_level;        // [steps + 64]
-  std::vector<StrainRec> rec;             // [steps][STRAIN_STEP_SLOTS]
+  StrainRows rec;                         // [steps][STRAIN_STEP_SLOTS]
   std::vector<int32_t> grp_ptr;           // [nband + 1] groups of each band
   std::vector<StrainGroup> grp;           // [groups]
   std::vector<StrainImport> imp;
@@ -72,7 +88,7 @@ struct StrainPlan {
   std::vector<StrainExport> exp;          // (+ 64 unused entries at the end)
   std::vector<int32_t> lo_ptr, lo;        // lower bands a band's imports come from
   std::vector<int32_t> up_ptr, up;        // bands (of the previous sweep) likewise
-  std::vector<int32_t> slot;              // [ne] element -> index into rec, -1 rigid
+  std::vector<int64_t> slot;              // [ne] element -> index into rec, -1 rigid
   size_t steps() const { return step_ptr.empty() ? 0 : (size_t)step_ptr.back(); }
 };
 
@@ -291,7 +307,6 @@ inline bool strain_build_plan(int nv, int ne, const int* ev, const uint8_t* rigi
     const int nstep = (int)lvl_of_step.size();
     const size_t step0 = P.steps();
     // slots, and each vertex's first and last step in the band
-    P.rec.resize((step0 + nstep) * STRAIN_STEP_SLOTS);
     touched.clear();
     {
       int st = -1, fill = STRAIN_STEP_SLOTS, cur = -1;
@@ -300,8 +315,10 @@ inline bool strain_build_plan(int nv, int ne, const int* ev, const uint8_t* rigi
           ++st;
           fill = 0;
           cur = lev[e];
+          P.rec.first.push_back(P.rec.first.back());
         }
-        P.slot[e] = (int32_t)((step0 + st) * STRAIN_STEP_SLOTS + fill++);
+        P.slot[e] = (int64_t)((step0 + st) * STRAIN_STEP_SLOTS + fill++);
+        ++P.rec.first.back();
         for (int k = 0; k < np_of(e); ++k) {
           const int v = vtx(e, k);
           if (stamp[v] != b) {
@@ -325,7 +342,9 @@ inline bool strain_build_plan(int nv, int ne, const int* ev, const uint8_t* rigi
     for (int g = 0; g < ngrp; ++g) {
       if (g - STRAIN_AHEAD - 1 >= 0)
         for (int32_t p : leave[g - STRAIN_AHEAD - 1]) freep.push_back(p);
-      StrainGroup G{(int32_t)P.imp.size(), 0, -1, -1};
+      const size_t s0 = step0 + (size_t)g * STRAIN_GROUP;
+      StrainGroup G{(int32_t)P.imp.size(), 0, -1, -1, P.rec.first[s0],
+                    P.rec.first[std::min(s0 + STRAIN_GROUP, step0 + nstep)]};
       for (int32_t v : bystep[g]) {
         int p;
         if (!freep.empty()) {
@@ -351,8 +370,9 @@ inline bool strain_build_plan(int nv, int ne, const int* ev, const uint8_t* rigi
     if (used > STRAIN_LDS_VERTS) return false;
     P.cap = std::max(P.cap, used);
     // records
+    P.rec.packed.resize((size_t)P.rec.first.back());
     for (int32_t e : order) {
-      StrainRec& r = P.rec[(size_t)P.slot[e]];
+      StrainRec& r = P.rec.packed[(size_t)P.rec.at((size_t)P.slot[e])];
       r.np = (uint16_t)np_of(e);
       for (int k = 0; k < 3; ++k) {
         r.L0[k] = len0[4 * (size_t)e + k];
@@ -383,6 +403,7 @@ inline bool strain_build_plan(int nv, int ne, const int* ev, const uint8_t* rigi
     P.lo_ptr.push_back((int32_t)P.lo.size());
     P.up_ptr.push_back((int32_t)P.up.size());
   }
+  P.rec.packed.resize(P.rec.packed.size() + STRAIN_STEP_SLOTS, StrainRec{});
   P.step_level.resize(P.step_level.size() + 64, std::numeric_limits<int32_t>::max());
   P.exp.resize(P.exp.size() + 64, StrainExport{0, 0, std::numeric_limits<int32_t>::max(), 0});
   P.lo.resize(P.lo.size() + 64, 0);
