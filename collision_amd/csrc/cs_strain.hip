@@ -40,6 +40,7 @@
 #include <algorithm>
 
 #include "cs_internal.h"
+#include "cs_strain_edge.h"
 
 namespace cs {
 
@@ -107,44 +108,8 @@ struct Spin {
   }
 };
 
-// One edge of an element (reduceSuperelastOnce): is it over the strain or the
-// strain-rate limit.  The screen decides from FP32 ratios of the FP64 edge
-// vector: rounding the vector, its square, the hardware reciprocal square roots
-// and reciprocals (1 ulp) and the products are each within 2^-22 relative, so
-// the ratios are within 1e-6 of the exact ones, and a decision is taken only
-// more than 1e-4 from the limit.  Inputs near the limit, degenerate lengths
-// and anything that is not finite in FP32 run the exact test.
-constexpr float kOver = (float)CS_SUPERELAS_TOL + 1e-4f, kUnder = (float)CS_SUPERELAS_TOL - 1e-4f;
+static_assert(STRAIN_TOL == CS_SUPERELAS_TOL && STRAIN_MIN_LEN == CS_ROUND_EPS, "cs_strain_edge.h");
 
-__device__ inline float sq_f32(const double* a, const double* b) {
-  const float x = (float)(a[0] - b[0]), y = (float)(a[1] - b[1]), z = (float)(a[2] - b[2]);
-  return x * x + y * y + z * z;
-}
-// 1 / the x_old length (NaN, so that no decision is taken, near or below the
-// degenerate length)
-__device__ inline float inv_old_length(const double* o0, const double* o1) {
-  const float so = sq_f32(o0, o1);
-  return so > 1e-19f ? __builtin_amdgcn_rsqf(so) : __builtin_nanf("");
-}
-// 1 over, 0 under, -1 not certain; p: end positions o + dt a
-__device__ inline int edge_screen(const double* p0, const double* p1, float il0, float ilo) {
-  const float s = sq_f32(p0, p1);
-  const float ln = s * __builtin_amdgcn_rsqf(s);
-  const float m = fmaxf(fabsf(ln * il0 - 1.0f), fabsf(ln * ilo - 1.0f));
-  // (fmaxf drops a NaN operand: the sum does not)
-  const bool fine = ln > 2e-10f && (ln * il0 + ln * ilo) < 1e30f;
-  return fine && m > kOver ? 1 : fine && m < kUnder ? 0 : -1;
-}
-// 0 under, 1 over, 3 over and degenerate
-__device__ inline int edge_exact(double so, double sq, double len0) {
-  const double len_old = sqrt(so), len_new = sqrt(sq);  // dist3 of the same points
-  if (len_old > CS_ROUND_EPS && len_new > CS_ROUND_EPS) {
-    const double strain_rate = (len_new - len_old) / len_old;
-    const double strain = (len_new - len0) / len0;
-    return (fabs(strain) > CS_SUPERELAS_TOL || fabs(strain_rate) > CS_SUPERELAS_TOL) ? 1 : 0;
-  }
-  return 3;
-}
 __device__ inline double sq_f64(const double* a, const double* b) {
   double s = 0.0;
 #pragma unroll
@@ -198,8 +163,9 @@ __global__ void __launch_bounds__(256)
       for (int i = 0; i < 3; ++i) {
         if (i > 0 && t.z < 0) break;
         const int j = (i + 1) % 3;
-        int r = edge_screen(p[i], p[j], __builtin_amdgcn_rcpf((float)len[i]), inv_old_length(o[i], o[j]));
-        if (r < 0) r = edge_exact(sq_f64(o[i], o[j]), sq_f64(p[i], p[j]), len[i]);
+        const double so = sq_f64(o[i], o[j]), sn = sq_f64(p[i], p[j]);
+        int r = edge_screen(sn, edge_limits(so, len[i]));
+        if (r < 0) r = edge_exact(so, sn, len[i]);
         any = any || r > 0;
       }
       pre[s] = any ? 1 : 0;
@@ -290,8 +256,11 @@ __global__ void __launch_bounds__(SB_THREADS)
         const int thr = k > 0 ? 1 + (k - 1) * NL + L : 1;
         if (wrote) stamps(u);
         // (place[2] of a bond repeats place[0])
-        const StrainRec& q = r[u];
-        const bool act = lane < n[u] && (pr[u] || t[u][0] >= thr || t[u][1] >= thr || t[u][2] >= thr);
+        const StrainRec q = r[u];
+        // (no short circuit: the stamp reads would be put off behind it)
+        const bool act = (lane < n[u]) & ((pr[u] != 0) | (t[u][0] >= thr) | (t[u][1] >= thr) | (t[u][2] >= thr));
+        // the same step of the next group
+        load(u, __builtin_amdgcn_readlane(rw, (s + u) & 63), __builtin_amdgcn_readlane(rw1, (s + u) & 63));
         if (__ballot(act)) {
           if (act) {
             BandVertex* w[3] = {win + q.place[0], win + q.place[1], win + q.place[2]};
@@ -305,19 +274,17 @@ __global__ void __launch_bounds__(SB_THREADS)
               }
               end_position(o[i], a[i], dt, p[i]);
             }
-            float il0[3], ilo[3];
+            EdgeLimits lim[3];
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-              il0[i] = __builtin_amdgcn_rcpf((float)q.L0[i]);
-              ilo[i] = inv_old_length(o[i], o[(i + 1) % 3]);
-            }
+            for (int i = 0; i < 3; ++i) lim[i] = edge_limits(sq_f64(o[i], o[(i + 1) % 3]), q.L0[i]);
             uint32_t wm = 0u;
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
               const int j = (i + 1) % 3;
-              int v = edge_screen(p[i], p[j], il0[i], ilo[i]);
+              const double sn = sq_f64(p[i], p[j]);
+              int v = edge_screen(sn, lim[i]);
               if (i > 0 && q.np != 3) v = 0;
-              if (v < 0) v = edge_exact(sq_f64(o[i], o[j]), sq_f64(p[i], p[j]), q.L0[i]);
+              if (v < 0) v = edge_exact(sq_f64(o[i], o[j]), sn, q.L0[i]);
               if (v > 0) {
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
@@ -346,8 +313,6 @@ __global__ void __launch_bounds__(SB_THREADS)
           wrote = true;
           lds_publish(&s_step, min(s + u + 1, nstep));
         }
-        // the same step of the next group
-        load(u, __builtin_amdgcn_readlane(rw, (s + u) & 63), __builtin_amdgcn_readlane(rw1, (s + u) & 63));
       }
       lds_publish(&s_step, min(s + 4, nstep));
     }
