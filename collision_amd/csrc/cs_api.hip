@@ -22,6 +22,7 @@
 
 #include "../../include/collision_amd.h"
 #include "cs_internal.h"
+#include "cs_tune.h"
 
 using namespace cs;
 
@@ -77,6 +78,7 @@ struct SeedPairs {
 
 struct PassTimes {
   hipEvent_t e0, e1, e2, e3, t0, t1, n0, n1;
+  bool narrow_tuned;  // its narrow launches take S.tune_narrow
 };
 
 struct cs_solver {
@@ -118,24 +120,15 @@ struct cs_solver {
     }
   } graph_key;
   int64_t assemble_gen = 0;  // bumped by every cs_assemble / cs_load
-  // autotuner: over its first steps every tuning step runs one candidate
-  // launch shape per kernel; per-unit kernel times are averaged per candidate
-  struct Tuner {
+  struct Tuner {  // autotuner
     bool active = false;
-    int step = 0;
     int tuned = 0;  // cs_tuning.tuned
-    double t_trav[4] = {}, t_narrow[3] = {}, t_query[4] = {};
-    int n_trav[4] = {}, n_narrow[3] = {}, n_query[4] = {};
+    LaunchTuner T;
     std::string key;
   } tuner;
 };
 
 namespace {
-constexpr int kTuneTrav[4] = {4, 8, 16, 32};
-constexpr int kTuneNarrow[3] = {64, 128, 256};
-constexpr int kTuneQuery[4] = {1024, 2048, 4096, 8192};
-constexpr int kTuneSteps = 8;  // two rounds of the four-candidate lists
-
 // CS_TUNE_CACHE: one line per key, "key traverse narrow query"
 bool tune_cache_lookup(const std::string& key, int* tr, int* na, int* qu) {
   const char* path = std::getenv("CS_TUNE_CACHE");
@@ -490,6 +483,7 @@ int run_pass(cs_solver* h, int kind, int index, int pass_id, bool* any_hit) {
     NP.ds_stride = h->L.ds_stride;
     NP.ds_salt = h->L.ds_salt++;
   }
+  T.narrow_tuned = (ccd && P.learned) || !narrow_rest(NP);
   int npairs = 0, carried_hits = 0, carried_hp = 0, carried_pairs = 0;
   unsigned long long cand = 0;
   int nq = 0;
@@ -1416,7 +1410,7 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
     while (lg < 40 && (1ll << (lg + 1)) <= (long long)std::max(ne, 1)) ++lg;
     h->tuner = cs_solver::Tuner();
     h->tuner.key = arch + ":ne2^" + std::to_string(lg) + (S.nscene > 1 ? ":batch" : ":single");
-    int tr = 8, na = 128, qu = 4096;
+    int tr = TUNE_TRAV_DEFAULT, na = TUNE_NARROW_DEFAULT, qu = TUNE_QUERY_DEFAULT;
     if (tune_cache_lookup(h->tuner.key, &tr, &na, &qu)) h->tuner.tuned = 2;
     S.tune_trav = tr;
     S.tune_narrow = na;
@@ -1564,12 +1558,10 @@ int resolve_impl(cs_solver* h, cs_step_report* report, bool predict) {
   std::vector<hipEvent_t> strain_marks;
   const bool spread_stats = P.precision == 1 || P.learned;
   cs_solver::Tuner& tu = h->tuner;
-  if (P.autotune && !tu.active && tu.tuned == 0 && tu.step == 0) tu.active = true;
+  if (P.autotune && !tu.active && tu.tuned == 0 && tu.T.step() == 0) tu.active = true;
   int saved_timing = -1;
   if (tu.active) {  // this step's candidates; kernel times need the timing markers
-    S.tune_trav = kTuneTrav[tu.step % 4];
-    S.tune_narrow = kTuneNarrow[tu.step % 3];
-    S.tune_query = kTuneQuery[tu.step % 4];
+    tu.T.candidates(&S.tune_trav, &S.tune_narrow, &S.tune_query);
     if (h->P.pass_timing < 1) {
       saved_timing = h->P.pass_timing;
       h->P.pass_timing = 1;
@@ -1639,36 +1631,16 @@ int resolve_impl(cs_solver* h, cs_step_report* report, bool predict) {
     pi.ms_traverse_kernel = elapsed(T.t0, T.t1);
     pi.ms_narrow_kernel = elapsed(T.n0, T.n1);
   }
-  if (tu.active) {  // per-unit kernel times of this step's candidates
-    double trav = 0.0, query = 0.0, narrow = 0.0;
-    int64_t lanes = 0;
-    int nfull = 0, ninc = 0;
-    for (const cs_pass_info& pi : h->passes) {
-      if (pi.incremental) {
-        query += pi.ms_traverse_kernel;
-        ++ninc;
-      } else {
-        trav += pi.ms_traverse_kernel;
-        ++nfull;
-      }
-      narrow += pi.ms_narrow_kernel;
-      lanes += std::max<int64_t>(pi.tested_pairs, 0);
+  if (tu.active) {  // kernel times of this step's candidates
+    std::vector<TunePass> ran;
+    for (size_t i = 0; i < h->passes.size() && i < h->ptimes.size(); ++i) {
+      const cs_pass_info& pi = h->passes[i];
+      ran.push_back({pi.incremental != 0, h->ptimes[i].narrow_tuned, pi.ms_traverse_kernel,
+                     pi.ms_narrow_kernel, pi.tested_pairs});
     }
-    const int a = tu.step % 4, b = tu.step % 3;
-    if (nfull) { tu.t_trav[a] += trav / nfull; tu.n_trav[a]++; }
-    if (ninc) { tu.t_query[a] += query / ninc; tu.n_query[a]++; }
-    if (lanes) { tu.t_narrow[b] += narrow / (double)lanes; tu.n_narrow[b]++; }
     if (saved_timing >= 0) h->P.pass_timing = saved_timing;
-    if (++tu.step >= kTuneSteps) {  // keep the fastest of each (defaults where unmeasured)
-      auto best = [](const double* t, const int* n, int m, const int* cand, int def) {
-        int bi = -1;
-        for (int i = 0; i < m; ++i)
-          if (n[i] && (bi < 0 || t[i] / n[i] < t[bi] / n[bi])) bi = i;
-        return bi < 0 ? def : cand[bi];
-      };
-      S.tune_trav = best(tu.t_trav, tu.n_trav, 4, kTuneTrav, 8);
-      S.tune_narrow = best(tu.t_narrow, tu.n_narrow, 3, kTuneNarrow, 128);
-      S.tune_query = best(tu.t_query, tu.n_query, 4, kTuneQuery, 4096);
+    if (tu.T.add_step(ran)) {
+      tu.T.choice(&S.tune_trav, &S.tune_narrow, &S.tune_query);
       tu.active = false;
       tu.tuned = 1;
       tune_cache_store(tu.key, S.tune_trav, S.tune_narrow, S.tune_query);
@@ -2177,8 +2149,8 @@ int cs_set_tuning(cs_solver* h, const cs_tuning* in) {
       if (c[i] == v) return true;
     return false;
   };
-  if (!one_of(in->traverse_blocks_per_cu, kTuneTrav, 4) || !one_of(in->narrow_threads, kTuneNarrow, 3) ||
-      !one_of(in->query_grid, kTuneQuery, 4))
+  if (!one_of(in->traverse_blocks_per_cu, TUNE_TRAV, 4) || !one_of(in->narrow_threads, TUNE_NARROW, 3) ||
+      !one_of(in->query_grid, TUNE_QUERY, 4))
     return fail(h, CS_ERR_ARG, "launch shape outside the candidate lists");
   h->S.tune_trav = in->traverse_blocks_per_cu;
   h->S.tune_narrow = in->narrow_threads;

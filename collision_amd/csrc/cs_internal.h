@@ -401,6 +401,11 @@ void launch_grow_carry(hipStream_t st, DevState& S, double dt, int nhits_prev, i
 void launch_carry_pairs_from(hipStream_t st, DevState& S, const int2* src, int n);
 
 // narrow phase
+// the form for the re-queried pairs of a plain incremental pass, which has a
+// work-group size of its own (the others take S.tune_narrow)
+inline bool narrow_rest(const NarrowParams& P) {
+  return P.ccd && !P.lseed && P.ds_cap <= 0 && !P.screen;
+}
 void launch_narrow(hipStream_t st, DevState& S, const NarrowParams& P, const int2* pairs,
                    int npairs, const int* npairs_dev, int cap);
 // learned form: score a pair stream's CCD sub-tests and sort the pairs by

@@ -1039,16 +1039,16 @@ void launch_narrow(hipStream_t st, DevState& S, const NarrowParams& P, const int
   if (!P.ccd) {
     if (P.mixed) size(std::integral_constant<int, NK_MIXED>{});
     else size(std::integral_constant<int, NK_PROX>{});
-  } else if (P.lseed || P.ds_cap > 0) {
-    size(std::integral_constant<int, NK_EXTRA>{});
-  } else if (P.screen) {
-    size(std::integral_constant<int, NK_CCD>{});
-  } else {
+  } else if (narrow_rest(P)) {
     // One wavefront per work-group: a few hundred work-groups, spread over twice as
     // many CUs as with 128 lanes (85 launches at 1024 x 1024 2.56 -> 2.50 ms, 33 at
     // 256 x 256 0.73 -> 0.71 ms).
     T = 64;
     go(k_narrow<64, NK_REST>);
+  } else if (P.lseed || P.ds_cap > 0) {
+    size(std::integral_constant<int, NK_EXTRA>{});
+  } else {
+    size(std::integral_constant<int, NK_CCD>{});
   }
 }
 
