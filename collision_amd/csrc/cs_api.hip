@@ -123,7 +123,7 @@ struct cs_solver {
   struct Tuner {  // autotuner
     bool active = false;
     int tuned = 0;  // cs_tuning.tuned
-    LaunchTuner T;
+    LaunchTuner T{0, 0};
     std::string key;
   } tuner;
 };
@@ -1409,6 +1409,7 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
     int lg = 0;
     while (lg < 40 && (1ll << (lg + 1)) <= (long long)std::max(ne, 1)) ++lg;
     h->tuner = cs_solver::Tuner();
+    h->tuner.T = LaunchTuner(ne, S.num_cus);
     h->tuner.key = arch + ":ne2^" + std::to_string(lg) + (S.nscene > 1 ? ":batch" : ":single");
     int tr = TUNE_TRAV_DEFAULT, na = TUNE_NARROW_DEFAULT, qu = TUNE_QUERY_DEFAULT;
     if (tune_cache_lookup(h->tuner.key, &tr, &na, &qu)) h->tuner.tuned = 2;

@@ -25,6 +25,7 @@
 
 #include "cs_internal.h"
 #include "cs_pairs.h"
+#include "cs_tune.h"
 
 namespace cs {
 
@@ -460,7 +461,6 @@ __device__ inline bool pair_rejected(int4 ta, int4 tb, uint8_t fa) {
 // surface field (the lower half is the surface's id within the scene)
 __device__ inline int scene_of(const int4& t) { return t.w >> 16; }
 
-constexpr int TRAV_THREADS = 256;
 constexpr int TRAV_BUF = 8;  // pairs buffered per lane before the wavefront writes them
 
 // Full-pass self query.  Lane = one leaf's stackless walk in depth-first order
@@ -494,7 +494,6 @@ constexpr int TRAV_BUF = 8;  // pairs buffered per lane before the wavefront wri
 // rigid surface is tested.  The kept pairs are tested by k_split_seed, so
 // one walk serves both passes.
 constexpr int TRAV_STEPS = 16;    // walk steps between checks of the buffers
-constexpr int TRAV_LANES = 262144, TRAV_SUB_MAX = 6;
 constexpr int TRAV_LONG = 128;
 constexpr int TRAV_SPLIT = 64;
 
@@ -1329,7 +1328,7 @@ void launch_grow_carry(hipStream_t st, DevState& S, double dt, int nhits_prev, i
 void launch_query_dirty(hipStream_t st, DevState& S, int emit, int snap, int count, int exact) {
   if (S.ne < 2) return;
   const int npre = 2 * S.ne - 1;
-  hipLaunchKernelGGL(k_query_ranges, dim3(std::min((npre + 63) / 64, S.tune_query)), dim3(64), 0, st,
+  hipLaunchKernelGGL(k_query_ranges, dim3(query_grid(S.ne, S.tune_query)), dim3(64), 0, st,
                      S.nodes, S.nright, S.ebox, S.ev, S.eflags, S.dirty_e, S.dpre, S.dirty_epoch, S.rlist, npre,
                      emit, S.nscene > 1, snap, exact, count == CNT_PAIRS ? S.pairs : S.qpairs,
                      count == CNT_PAIRS ? S.pair_cap : S.qpair_cap, count, S.counters);
@@ -1409,11 +1408,7 @@ void launch_traverse(hipStream_t st, DevState& S, int2* out, int cap, const dbox
                      bool check) {
   const int n = S.ne;
   if (n < 2) return;
-  int lsub = 0;
-  while (lsub < TRAV_SUB_MAX && ((int64_t)n << (lsub + 1)) <= TRAV_LANES) ++lsub;
-  const int64_t need = (((int64_t)n << lsub) + TRAV_THREADS - 1) / TRAV_THREADS;
-  // one walk per lane, up to 8 x tune_trav work-groups per CU
-  const int blocks = (int)std::min<int64_t>(need, 8ll * S.num_cus * S.tune_trav);
+  const int lsub = traverse_cuts(n), blocks = traverse_grid(n, S.num_cus, S.tune_trav);
   TravItem* q0 = reinterpret_cast<TravItem*>(S.tq);
   TravItem* q1 = q0 + TRAV_QCAP;
   int* n0 = S.counters + CNT_TSPLIT;
