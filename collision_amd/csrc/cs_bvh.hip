@@ -1422,7 +1422,7 @@ void launch_traverse(hipStream_t st, DevState& S, int2* out, int cap, const dbox
   A2.qout = nullptr;
   A2.qout_n = nullptr;
   // where a share of the tree has no more nodes than a walk may take, no walk is
-  // handed over and the rounds for them are not launched (up to 4,032 elements)
+  // handed over and the rounds for them are not launched (up to 4,095 elements)
   const bool rounds = ((2 * (int64_t)n) >> lsub) + 1 > TRAV_LONG;
   if (!rounds) A.qout = nullptr;
   auto go = [&](auto main, auto split) {
