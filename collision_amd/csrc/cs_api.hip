@@ -808,14 +808,15 @@ struct LearnedWorkspace {
 
 // The banded strain-limit plan, with more bands (smaller vertex windows) as
 // long as a window does not fit; false when none does (elements in random
-// order over a large mesh: every band then meets most vertices at once).
+// order over a large mesh: every band then meets most vertices at once).  lev, nl:
+// the elements' levels, for the other schedule.
 bool strain_plan_for(int nv, int ne, const std::vector<int4>& ev, const std::vector<uint8_t>& ef,
-                     const std::vector<dvec4>& l0, int nsched, StrainPlan& plan) {
+                     const std::vector<dvec4>& l0, int nsched, StrainPlan& plan,
+                     std::vector<int>& lev, int& nl) {
   std::vector<uint8_t> rigid((size_t)ne);
   for (int e = 0; e < ne; ++e) rigid[e] = (ef[e] & EF_RIGID) ? 1 : 0;
-  std::vector<int> lev;
   const int* e4 = reinterpret_cast<const int*>(ev.data());
-  const int nl = strain_levels(nv, ne, e4, rigid.data(), lev);
+  nl = strain_levels(nv, ne, e4, rigid.data(), lev);
   for (int nb = strain_band_count(nsched, nl);; nb = std::min(2 * nb, STRAIN_MAX_BANDS)) {
     if (strain_build_plan(nv, ne, e4, rigid.data(), reinterpret_cast<const double*>(l0.data()), lev,
                           nl, nb, plan))
@@ -838,10 +839,10 @@ struct PipeSchedule {
 // level (the elements of one level share no vertex, so any order is exact there)
 int build_pipe_schedule(cs_solver* h, int nv, int ne, const std::vector<int4>& ev,
                         const std::vector<uint8_t>& ef, const std::vector<dvec4>& l0,
-                        PipeSchedule& Q) {
+                        std::vector<int>&& lev, int nl, PipeSchedule& Q) {
   std::vector<int> level;
   int nlev = 0;
-  build_strain_schedule(nv, ne, ev.data(), ef.data(), level, nlev, Q.delta);
+  build_strain_schedule(nv, ne, ev.data(), ef.data(), std::move(lev), nl, level, nlev, Q.delta);
   Q.n_levels = nlev;
   int nsched = 0;
   for (int e = 0; e < ne; ++e)
@@ -1220,11 +1221,13 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   int nsched = 0;
   for (int e = 0; e < ne; ++e) nsched += !(ef[e] & EF_RIGID);
   if (nsched > 0) {
-    if (strain_plan_for(nv, ne, ev, ef, l0, nsched, plan)) {
+    std::vector<int> lev;
+    int nl = 0;
+    if (strain_plan_for(nv, ne, ev, ef, l0, nsched, plan, lev, nl)) {
       if (plan.n_levels >= (1 << 21))
         return fail(h, CS_ERR_UNSUPPORTED, "strain schedule above 2^21 levels");
     } else {
-      const int rc = build_pipe_schedule(h, nv, ne, ev, ef, l0, pipe);
+      const int rc = build_pipe_schedule(h, nv, ne, ev, ef, l0, std::move(lev), nl, pipe);
       if (rc) return rc;
     }
   }

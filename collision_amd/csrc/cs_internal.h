@@ -456,9 +456,9 @@ hipError_t strain_limit(hipStream_t st, DevState& S, double dt, int max_sweeps,
 hipError_t strain_bands_setup(DevState& S);
 hipError_t strain_limit_bands(hipStream_t st, DevState& S, double dt, int max_sweeps,
                               std::vector<hipEvent_t>* marks);
-// cs_schedule.hip (host)
-void build_strain_schedule(int nv, int ne, const int4* ev, const uint8_t* ef,
-                           std::vector<int>& level, int& n_levels, int& delta);
+// cs_schedule.hip (host); lev, L: the elements' levels and their number (strain_levels)
+void build_strain_schedule(int nv, int ne, const int4* ev, const uint8_t* ef, std::vector<int> lev,
+                           int L, std::vector<int>& level, int& n_levels, int& delta);
 void launch_final_velocity(hipStream_t st, DevState& S);
 // cs_set_state / cs_get_state: [n][3] arrays (device or pinned host memory) to
 // and from the state; want: x, vel, avgVel, x_old

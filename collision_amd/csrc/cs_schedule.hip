@@ -14,14 +14,11 @@
 // visits lie within fewer than `delta` levels (its first visit in sweep k+1
 // then comes after its last visit in sweep k).  The schedule is built so
 // that this span is small:
-//   1. earliest levels (1 + max level of earlier elements on shared vertices);
-//   2. relaxation: a vertex's first visit is raised to at most W levels below
-//      its last visit, repeated until nothing moves (W starts at the largest
-//      vertex valence - 1 and doubles when a pass limit is hit; without
-//      convergence the earliest levels are kept);
-//   3. connected components much shorter than the schedule (strings, small
+//   1. the levels of strain_levels (cs_strain_plan.h), which the caller has: most
+//      of the time of a schedule for elements in random order;
+//   2. connected components much shorter than the schedule (strings, small
 //      pieces) are shifted as a whole to the least loaded levels;
-//   4. levels with more than STRAIN_LEVEL_CAP elements are split.
+//   3. levels with more than STRAIN_LEVEL_CAP elements are split.
 // Any schedule that keeps the element order of each vertex is exact; these
 // steps only make the sweep faster.
 #include <algorithm>
@@ -45,8 +42,8 @@ int find_root(std::vector<int>& uf, int x) {
 
 }  // namespace
 
-void build_strain_schedule(int nv, int ne, const int4* ev, const uint8_t* ef,
-                           std::vector<int>& level, int& n_levels, int& delta) {
+void build_strain_schedule(int nv, int ne, const int4* ev, const uint8_t* ef, std::vector<int> lev,
+                           int L, std::vector<int>& level, int& n_levels, int& delta) {
   level.assign((size_t)std::max(ne, 1), -1);
   n_levels = 0;
   delta = 1;
@@ -56,13 +53,7 @@ void build_strain_schedule(int nv, int ne, const int4* ev, const uint8_t* ef,
   for (int e = 0; e < ne; ++e)
     if (!(ef[e] & EF_RIGID)) ++nsched;
   if (nsched == 0) return;
-  // 1 + 2: earliest levels, relaxed so that each vertex's visits stay within W levels
-  std::vector<int> lev;
-  std::vector<uint8_t> rigid((size_t)std::max(ne, 1));
-  for (int e = 0; e < ne; ++e) rigid[e] = (ef[e] & EF_RIGID) ? 1 : 0;
-  const int L = strain_levels(nv, ne, reinterpret_cast<const int*>(ev), rigid.data(), lev);
-
-  // 3: shift short components to the least loaded levels
+  // 2: shift short components to the least loaded levels
   std::vector<int> uf((size_t)nv);
   std::iota(uf.begin(), uf.end(), 0);
   for (int e = 0; e < ne; ++e) {
@@ -132,7 +123,7 @@ void build_strain_schedule(int nv, int ne, const int4* ev, const uint8_t* ef,
       if (root[e] >= 0 && is_short(root[e])) lev[e] += shift[root[e]];
   }
 
-  // 4: split levels above the cap (element order within a level)
+  // 3: split levels above the cap (element order within a level)
   std::vector<int> cnt((size_t)L, 0);
   for (int e = 0; e < ne; ++e)
     if (root[e] >= 0) cnt[lev[e]]++;
