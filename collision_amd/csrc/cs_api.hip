@@ -1502,11 +1502,10 @@ int cs_predict(cs_solver* h) {
 
 namespace {
 
-// The launches of a resolve before its first pass (kernels
-// only, so that they can be captured in a graph): the dirty marks of the last
-// pass and the counters, the batched scenes' pass state, then
-// computeAverageVelocity with the union-find (makeSet, dcollid.cpp:1015-1031),
-// the recorded impulses and the zone marks.
+// The launches of a resolve before its first pass (kernels only, so that they
+// can be captured in a graph): the counters, the statistics and the batched
+// scenes' pass state cleared, then computeAverageVelocity with the union-find
+// (makeSet, dcollid.cpp:1015-1031), the recorded impulses and the zone marks.
 void resolve_prologue(cs_solver* h, bool stats, bool predict) {
   DevState& S = h->S;
   const cs_params& P = h->P;

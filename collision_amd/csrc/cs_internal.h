@@ -356,7 +356,8 @@ hipError_t exclusive_scan_u32(hipStream_t st, uint32_t* data, int n, uint32_t* p
 hipError_t radix_sort_u32(hipStream_t st, uint32_t* keys, uint32_t* vals, uint32_t* tmp_keys,
                           uint32_t* tmp_vals, uint32_t* hist, uint32_t* partials, int n, int bits,
                           bool* result_in_tmp);
-// iota: the values are the keys' indices (vals is only used as a buffer)
+// iota: the values are the keys' indices (vals is only used as a buffer); only
+// above RANK_SORT_MAX keys, the fewer hits of a pass are sorted by rank_hits
 hipError_t radix_sort_u64(hipStream_t st, uint64_t* keys, uint32_t* vals, uint64_t* tmp_keys,
                           uint32_t* tmp_vals, uint32_t* hist, uint32_t* partials, int n, int bits,
                           bool* result_in_tmp, bool iota = false);
@@ -482,14 +483,14 @@ __device__ inline int xcd_block(int b, int G) {
   return (x < r) ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
 }
 
-// slot in a list for the lanes with want set, one atomic per wavefront;
-// every active lane of the wavefront calls it
 // one wavefront of a kernel zeroes the counters in the mask
 static_assert(CNT_INTS <= 64, "one bit of the mask per counter");
 __device__ inline void clear_counters(uint64_t mask, int* counters) {
   if (threadIdx.x < CNT_INTS && (mask >> threadIdx.x & 1ull)) counters[threadIdx.x] = 0;
 }
 
+// slot in a list for the lanes with want set, one atomic per wavefront;
+// every active lane of the wavefront calls it
 __device__ inline int wave_append(bool want, int* counter) {
   const uint64_t m = __ballot(want);
   if (m == 0) return -1;

@@ -525,8 +525,6 @@ __device__ bool d_is_coplanar(const Sub& S, double dt, double roots[4]) {
   return roots[0] > CS_MACH_EPS || roots[1] > CS_MACH_EPS || roots[2] > CS_MACH_EPS;
 }
 
-// roots / *coplanar: isCoplanar's outcome for a CCD sub-test (roots -1 and
-// false when the certified screen decided it)
 // The forms of the narrow kernel, each compiled by itself, so that none pays for
 // the registers of another.  As one kernel all had 168 VGPRs (3 wavefronts per
 // SIMD) and 128 B of scratch per lane.  Now, at 2.6e6 pairs of a 1024 x 1024
@@ -542,6 +540,8 @@ enum NarrowKind {
   NK_REST,   // CCD without it: the re-queried pairs of incremental passes
   NK_EXTRA   // CCD, learned form or collecting samples
 };
+// roots / *coplanar: isCoplanar's outcome for a CCD sub-test (roots -1 and
+// false when the certified screen decided it)
 template <int KIND>
 __device__ bool d_subtest(const Sub& S, bool is_pt, const NarrowParams& P, Contrib& C, int* err,
                           double roots[4], bool* coplanar, int known) {
@@ -985,11 +985,11 @@ __device__ __attribute__((always_inline)) inline void narrow_lane(
   if (P.zone_mode && active && s >= first_hit) zone_merge4(Z, P.vbody, q);
 }
 
-// npairs_dev != nullptr: the pair count is read on the device (clamped to
-// cap); the grid covers the first npairs pairs of it
 // wavefronts per SIMD that the registers are cut for
 constexpr int narrow_waves(int kind) { return kind == NK_REST ? 2 : kind <= NK_MIXED ? 4 : 3; }
 
+// npairs_dev != nullptr: the pair count is read on the device, and nothing is
+// tested when it is above cap; the grid covers the first npairs pairs
 template <int THREADS, int KIND>
 __global__ void __launch_bounds__(THREADS, narrow_waves(KIND))
     k_narrow(const int2* __restrict__ pairs, int npairs, const int* __restrict__ npairs_dev,

@@ -256,7 +256,6 @@ __device__ __attribute__((always_inline)) inline void rank_keys(const K* __restr
   }
 }
 
-// vals null: each key's value is its index
 template <typename K>
 __global__ void __launch_bounds__(64 * RANK_WAVES) k_sort_rank(const K* __restrict__ keys,
                                                               const uint32_t* __restrict__ vals,
@@ -264,7 +263,7 @@ __global__ void __launch_bounds__(64 * RANK_WAVES) k_sort_rank(const K* __restri
                                                               uint32_t* __restrict__ vals_out, int n) {
   rank_keys(keys, n, [&](int r, int i, K k) {
     keys_out[r] = k;
-    vals_out[r] = vals ? vals[i] : (uint32_t)i;
+    vals_out[r] = vals[i];
   });
 }
 
@@ -296,10 +295,10 @@ static hipError_t radix_sort_impl(hipStream_t st, K* keys, uint32_t* vals, K* tm
                                   uint32_t* tmp_vals, uint32_t* hist, uint32_t* partials, int n,
                                   int bits, bool* result_in_tmp, bool iota = false) {
   *result_in_tmp = false;
-  if ((n <= 1 && !iota) || n <= 0 || bits <= 0) return hipSuccess;
+  if (n <= 1 || bits <= 0) return hipSuccess;
   if (n <= RANK_SORT_MAX) {
     hipLaunchKernelGGL(k_sort_rank<K>, dim3((n + 63) / 64), dim3(64 * RANK_WAVES), 0, st, keys,
-                       iota ? nullptr : vals, tmp_keys, tmp_vals, n);
+                       vals, tmp_keys, tmp_vals, n);
     *result_in_tmp = true;
     return hipGetLastError();
   }

@@ -10,8 +10,9 @@
 // level, so a sweep is `levels` dependent steps (4,090 on a 1024 x 1024 cloth)
 // however many compute units take part; the sweeps and bands follow each other
 // a few steps apart.  A step is one wavefront's work on LDS only (three stamp
-// reads; where an element has to be evaluated, its vertices and the edges' tests), and everything that touches memory is done by the task's
-// other wavefronts ahead of it or behind it:
+// reads; where an element has to be evaluated, its vertices and the edges'
+// tests), and everything that touches memory is done by the task's other
+// wavefronts ahead of it or behind it:
 //   wavefront 0     steps
 //   wavefronts 1,2  imports: wait for the other tasks' progress, load the
 //                   vertices of a group of steps into LDS (alternate groups)
