@@ -324,6 +324,7 @@ struct LearnedState {
   int64_t ds_alloc = 0, ds_cap = 0;
   int32_t ds_stride = 1;
   uint32_t ds_salt = 0;
+  int num_cus = 256;  // compute units of the device
   // inputs and outputs of cs_learned_infer / cs_learned_grad (kept up to WS_KEEP
   // bytes) and the pinned copy of a gradient and its loss
   float* ws = nullptr;

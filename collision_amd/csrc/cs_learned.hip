@@ -25,7 +25,7 @@ namespace cs {
 // the activations went through LDS between layers: 200,003 samples 170 us in the
 // kernel, the call 1.01 -> 0.87 ms (the rest is the host link).
 constexpr int INF_W2 = 16, INF_W3 = INF_W2 + 64, INF_OPS = INF_W3 + 8;
-constexpr int INF_GROUPS = 3, INF_CUS = 256;  // per CU, CUs
+constexpr int INF_GROUPS = 3;  // per CU
 
 // the left operand of fragment f, lane l
 __device__ inline int infer_operand(int f, int l) {
@@ -370,6 +370,9 @@ hipError_t ensure_train(LearnedState& L, int ntile) {
 
 hipError_t learned_alloc(LearnedState& L) {
   if (L.w) return hipSuccess;
+  int device = 0;
+  CS_HIP_RET(hipGetDevice(&device));
+  CS_HIP_RET(hipDeviceGetAttribute(&L.num_cus, hipDeviceAttributeMultiprocessorCount, device));
   CS_HIP_RET(lalloc(&L.w, MF_NPARAM));
   CS_HIP_RET(lalloc(&L.m, MF_NPARAM));
   CS_HIP_RET(lalloc(&L.v, MF_NPARAM));
@@ -428,7 +431,7 @@ hipError_t learned_infer(LearnedState& L, hipStream_t st, const float* dx, int64
   // the work-groups that fit the card, or as many as give every wavefront the
   // same number of rounds
   constexpr int waves = MLP_THREADS / 64;
-  const int64_t ntile = (n + 15) / 16, fit = (int64_t)INF_GROUPS * INF_CUS * waves;
+  const int64_t ntile = (n + 15) / 16, fit = (int64_t)INF_GROUPS * L.num_cus * waves;
   const int64_t rounds = (ntile + fit - 1) / fit;
   const unsigned grid = (unsigned)((ntile + rounds * waves - 1) / (rounds * waves));
   hipLaunchKernelGGL(k_mlp_infer, dim3(grid), dim3(MLP_THREADS), 0, st, dx, n, L.wb, L.w, dout);
