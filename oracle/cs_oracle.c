@@ -390,6 +390,7 @@ typedef struct {
     double *imp, *fric;
     int32_t *num;
     int err;
+    int dry;               /* only the outcome: no impulse is stored */
 } imp_ctx;
 
 static inline int c_static(const imp_ctx *C, int32_t v) { return C->fixed[v] != 0; }
@@ -410,6 +411,7 @@ static void spread_rg(imp_ctx *C, int32_t v, double impulse, const double nor[3]
 static void pt_impulse(imp_ctx *C, const int32_t p[4], double nor[3], double w[3],
                        double dist, double root) {
     (void)root;
+    if (C->dry) return;
     const orc_params *P = C->P;
     const double eps_m = P->mach_eps;
     double v_rel[3] = {0.0, 0.0, 0.0}, vn, vt;
@@ -508,6 +510,7 @@ static void pt_impulse(imp_ctx *C, const int32_t p[4], double nor[3], double w[3
 static void ee_impulse(imp_ctx *C, const int32_t p[4], double nor[3], double a, double b,
                        double dist, double root) {
     (void)root;
+    if (C->dry) return;
     const orc_params *P = C->P;
     const double eps_m = P->mach_eps;
     double v_rel[3], vn, vt, impulse = 0.0, m_impulse = 0.0;
@@ -841,7 +844,7 @@ static int32_t narrow_pair(orc_solver *s, imp_ctx *C, int32_t A, int32_t B, int 
 #define SUBTEST(idx, ispt)                                             \
     do {                                                                \
         if (subtest(s, C, (ispt), p, ccd, h)) { status = 1; mask |= 1 << (idx); } \
-        if (status && zone) create_imp_zone(s, p);                     \
+        if (status && zone && !C->dry) create_imp_zone(s, p);          \
     } while (0)
     if (ta && tb) {
         if (s->surf[A] == s->surf[B] && elem_is_rigid(s, A)) return 0;
@@ -1102,6 +1105,61 @@ static void tree_query(orc_solver *s, tree_t *t) {
     free(ist);
 }
 
+/* The same query with the leaves dealt to the processors, for the checking form
+ * (canonical order, deterministic functions).  "Not yet queried" is "later in
+ * the in-order sequence", so a leaf's walk depends on no other; the pairs are
+ * joined in sequence order, which gives tree_query's list. */
+enum { QUERY_CHUNK = 64 };
+static void tree_query_parallel(orc_solver *s, tree_t *t) {
+    int32_t ne = s->ne, nleaf = 0, isp = 0, cur = t->root;
+    int32_t *ist = (int32_t *)malloc(sizeof(int32_t) * (size_t)(t->n + 1));
+    int32_t *seq = (int32_t *)malloc(sizeof(int32_t) * (size_t)(ne ? ne : 1));
+    int32_t *rank = (int32_t *)malloc(sizeof(int32_t) * (size_t)(ne ? ne : 1));
+    while (cur >= 0 || isp) {
+        while (cur >= 0) { ist[isp++] = cur; cur = t->left[cur]; }
+        cur = ist[--isp];
+        if (t->left[cur] < 0 && t->right[cur] < 0) {
+            rank[t->leaf[cur]] = nleaf;
+            seq[nleaf++] = cur;
+        }
+        cur = t->right[cur];
+    }
+    free(ist);
+    int32_t nchunk = (nleaf + QUERY_CHUNK - 1) / QUERY_CHUNK;
+    vec_t *found = (vec_t *)calloc((size_t)(nchunk ? nchunk : 1), sizeof(vec_t));
+#pragma omp parallel
+    {
+        int32_t *qst = (int32_t *)malloc(sizeof(int32_t) * (size_t)(2 * ne + 64));
+#pragma omp for schedule(dynamic, 1)
+        for (int32_t c = 0; c < nchunk; ++c) {
+            found[c].sz = sizeof(int64_t);
+            int32_t end = (c + 1) * QUERY_CHUNK < nleaf ? (c + 1) * QUERY_CHUNK : nleaf;
+            for (int32_t q = c * QUERY_CHUNK; q < end; ++q) {
+                int32_t n = seq[q], qsp = 0, c2 = t->root;
+                const box_t *nb = &t->box[n];
+                for (;;) {
+                    while (c2 >= 0 && box_overlap(&t->box[c2], nb)) {
+                        if (t->left[c2] < 0 && t->right[c2] < 0 && rank[t->leaf[c2]] > q) {
+                            int64_t pr = ((int64_t)t->leaf[c2] << 32) | (uint32_t)t->leaf[n];
+                            vec_push(&found[c], &pr);
+                        }
+                        qst[qsp++] = c2;
+                        c2 = t->left[c2];
+                    }
+                    if (!qsp) break;
+                    c2 = t->right[qst[--qsp]];
+                }
+            }
+        }
+        free(qst);
+    }
+    for (int32_t c = 0; c < nchunk; ++c) {
+        for (int64_t i = 0; i < found[c].n; ++i) vec_push(&s->pairs, (int64_t *)found[c].p + i);
+        free(found[c].p);
+    }
+    free(found); free(rank); free(seq);
+}
+
 static int cmp_i64(const void *a, const void *b) {
     int64_t x = *(const int64_t *)a, y = *(const int64_t *)b;
     return (x > y) - (x < y);
@@ -1125,7 +1183,11 @@ static int run_pass(orc_solver *s, int kind) {
         }
     }
     s->pairs.n = 0;
-    tree_query(s, t);
+    /* the checking form uses all processors; the reference's order with libm,
+     * whose time is quoted, runs as the reference does */
+    int checking = s->P.order_mode == ORC_ORDER_CANONICAL && s->P.math_mode == ORC_MATH_DET;
+    if (checking) tree_query_parallel(s, t);
+    else tree_query(s, t);
     int64_t *pp = (int64_t *)s->pairs.p;
     int64_t np = s->pairs.n;
     if (s->P.order_mode == ORC_ORDER_CANONICAL) {
@@ -1137,14 +1199,33 @@ static int run_pass(orc_solver *s, int kind) {
         qsort(pp, (size_t)np, sizeof(int64_t), cmp_i64);
     }
     imp_ctx C = {&s->P, s->fixed, s->nbody ? s->vbody : NULL, s->bmass, s->rg_imp, s->rg_num,
-                 s->av, s->x_old, s->imp, s->fric, s->num, 0};
+                 s->av, s->x_old, s->imp, s->fric, s->num, 0, 0};
     orc_pass_info *pi = &s->cur;
     memset(pi, 0, sizeof(*pi));
     pi->kind = kind;
     pi->candidates = np;
     int any = 0;
+    /* A pair's outcome depends on the state of the pass alone (impulses are only
+     * added up), so the pairs without a hit are found first, in any order; the
+     * others then run in the canonical order as if this had not been done. */
+    uint8_t *none = NULL;  /* 1: no hit, 2: no hit and sub-tests ran */
+    if (checking) {
+        none = (uint8_t *)malloc((size_t)(np ? np : 1));
+#pragma omp parallel for schedule(dynamic, 64)
+        for (int64_t i = 0; i < np; ++i) {
+            imp_ctx D = C;
+            D.dry = 1;
+            int ran = 0;
+            int32_t mask = narrow_pair(s, &D, (int32_t)(pp[i] & 0xffffffff), (int32_t)(pp[i] >> 32), ccd, &ran);
+            none[i] = (mask || D.err) ? 0 : 1 + ran;
+        }
+    }
     for (int64_t i = 0; i < np; ++i) {
         int32_t A, B;
+        if (none && none[i]) {
+            pi->narrow_pairs += none[i] - 1;
+            continue;
+        }
         if (s->P.order_mode == ORC_ORDER_CANONICAL) {
             B = (int32_t)(pp[i] >> 32);              /* lo = query leaf */
             A = (int32_t)(pp[i] & 0xffffffff);       /* hi */
@@ -1166,6 +1247,7 @@ static int run_pass(orc_solver *s, int kind) {
             }
         }
     }
+    free(none);
     if (C.err) s->err = C.err;
     return any;
 }
@@ -1614,7 +1696,7 @@ int orc_last_impulses(orc_solver *s, double *imp, int32_t *num) {
 int32_t orc_debug_pair(orc_solver *s, int32_t A, int32_t B, int32_t ccd, int32_t zone_mode) {
     if (!s || !s->x || A < 0 || B < 0 || A >= s->ne || B >= s->ne) return -1;
     imp_ctx C = {&s->P, s->fixed, s->nbody ? s->vbody : NULL, s->bmass, s->rg_imp, s->rg_num,
-                 s->av, s->x_old, s->imp, s->fric, s->num, 0};
+                 s->av, s->x_old, s->imp, s->fric, s->num, 0, 0};
     int saved = s->zone_mode, ran = 0;
     s->zone_mode = zone_mode;
     int32_t mask = narrow_pair(s, &C, A, B, ccd, &ran);
@@ -1645,7 +1727,7 @@ static int unit_subtest(const orc_params *p, const double *c, const double *x_ol
     memset(counts, 0, 4 * sizeof(int32_t));
     uint8_t fx[4] = {0, 0, 0, 0};
     if (is_fixed) memcpy(fx, is_fixed, 4);
-    imp_ctx C = {p, fx, NULL, NULL, NULL, NULL, avg_vel, x_old, imp, fric, counts, 0};
+    imp_ctx C = {p, fx, NULL, NULL, NULL, NULL, avg_vel, x_old, imp, fric, counts, 0, 0};
     int32_t ids[4] = {0, 1, 2, 3};
     int hit = pt ? point_to_tri(&C, ids, (const double(*)[3])c, h, 0.0)
                  : edge_to_edge(&C, ids, (const double(*)[3])c, h, 0.0);
