@@ -807,8 +807,8 @@ struct LearnedWorkspace {
 };
 
 // The banded strain-limit plan, with more bands (smaller vertex windows) as
-// long as a window does not fit; false when none does (elements in random
-// order over a large mesh: every band then meets most vertices at once).  lev, nl:
+// long as a window does not fit; false when none does or the one that does is
+// not worth it (elements in random order: every band meets most vertices).  lev, nl:
 // the elements' levels, for the other schedule.
 bool strain_plan_for(int nv, int ne, const std::vector<int4>& ev, const std::vector<uint8_t>& ef,
                      const std::vector<dvec4>& l0, int nsched, StrainPlan& plan,
@@ -819,8 +819,10 @@ bool strain_plan_for(int nv, int ne, const std::vector<int4>& ev, const std::vec
   nl = strain_levels(nv, ne, e4, rigid.data(), lev);
   for (int nb = strain_band_count(nsched, nl);; nb = std::min(2 * nb, STRAIN_MAX_BANDS)) {
     if (strain_build_plan(nv, ne, e4, rigid.data(), reinterpret_cast<const double*>(l0.data()), lev,
-                          nl, nb, plan))
-      return true;
+                          nl, nb, plan)) {
+      if (strain_plan_pays(plan)) return true;
+      break;
+    }
     if (nb >= STRAIN_MAX_BANDS || nb >= nsched) break;
   }
   plan = StrainPlan();
@@ -1215,7 +1217,8 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
     if (!used[v])
       return fail(h, CS_ERR_ARG, "every vertex must belong to a triangle or bond");
   // strain limiting: the banded plan, or the level schedule of the one-work-group
-  // sweep where no number of bands has vertex windows that fit LDS
+  // sweep where no number of bands has vertex windows that fit LDS or the bands
+  // would run one after another
   StrainPlan plan;
   PipeSchedule pipe;
   int nsched = 0;

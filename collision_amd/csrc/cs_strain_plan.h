@@ -78,6 +78,7 @@ struct StrainRows {
 
 struct StrainPlan {
   int nband = 0, n_levels = 0, cap = 0;   // cap: LDS places of the largest window
+  int64_t nvert = 0;                      // vertices of the elements planned
   std::vector<int32_t> step_ptr;          // [nband + 1] steps of each band
   std::vector<int32_t> step_level;        // [steps + 64]
   StrainRows rec;                         // [steps][STRAIN_STEP_SLOTS]
@@ -176,6 +177,30 @@ inline int strain_band_count(int64_t nsched, int n_levels) {
   int n = (int)std::min<int64_t>(std::max<int64_t>(b, 1), STRAIN_MAX_BANDS);
   if (n > 8) n = (n + 7) & ~7;  // a band's tasks then tend to share an XCD
   return n;
+}
+
+// Whether the banded sweeps are the better ones of a plan that fits, or all sweeps
+// in one work-group (k_strain_pipe).  Where many vertices are met by many bands, a
+// band begins when the ones below it are nearly over: the bands of all sweeps run
+// one after another, and their steps last as long as their imports.  An order
+// with locality imports a vertex 1.0 to 2.2 times a sweep (rows, columns, radial,
+// Morton; tiles of 16), elements in random order 2.6 times (24 x 24) and more.
+// Kernel ms, banded / one work-group, with many / few edges over the limit:
+//   imports  mesh                                 many          few
+//   1.0      64 x 64 by rows                      0.41 / 1.54   0.27 / 0.85
+//   2.1      256 x 256, shuffled tiles of 16      1.45 / 4.63   1.27 / 1.79
+//   2.1      32 x 32, shuffled within 1,024       0.31 / 0.35   0.28 / 0.17
+//   2.2      512 x 512, shuffled tiles of 16      11.8 / 15.3   11.7 / 2.4
+//   2.9      128 x 128, shuffled tiles of 4       4.8 / 1.2     4.8 / 0.28
+//   3.7      128 x 128, shuffled within 4,096     1.42 / 1.02   1.38 / 0.28
+//   5.7      160 x 160 in random order            11.2 / 1.4    11.2 / 0.31
+// (One string of 30,000 bonds: 24 / 97 and 7.5 / 4.4; a closed one 110 / 362 and
+// 65 / 50: there the idle steps of the bands cost more than skipped levels.)
+// A sweep of few steps cannot cost much in bands, and a mesh with every edge over the
+// limit gains: 24 x 24 in random order (44 steps) 0.34 / 0.22 and 0.32 / 0.14, but
+// the whole step of one with every edge over it 0.59 / 1.00 ms.
+inline bool strain_plan_pays(const StrainPlan& P) {
+  return 10 * (int64_t)P.imp.size() <= 24 * P.nvert || P.steps() <= 64;
 }
 
 // Microseconds after which a wait of a task means that the plan is broken.  A
@@ -280,6 +305,7 @@ inline bool strain_build_plan(int nv, int ne, const int* ev, const uint8_t* rigi
         vlast[vtx(sched[i], k)] = lev[sched[i]];
         vband[vtx(sched[i], k)] = b;
       }
+  for (int v = 0; v < nv; ++v) P.nvert += vband[v] >= 0;
   std::vector<int32_t> pband((size_t)nv, -1), plevel((size_t)nv, -1);  // previous band's last visit
   std::vector<int32_t> stamp((size_t)nv, -1), fstep((size_t)nv), lstep((size_t)nv), place((size_t)nv);
   std::vector<int32_t> order, cnt((size_t)n_levels + 1), touched;
