@@ -205,20 +205,18 @@ __global__ void __launch_bounds__(SB_THREADS)
   int* stat = B.stat;
   if (wave == 0) {
     // --- the steps.  Records (static) are loaded one group ahead into
-    // registers.  The lanes past the step's last element hold that one's record
-    // (so that their stamp reads meet it in LDS and not in other banks) and take
-    // no part.
+    // registers.  The lanes past the step's last element hold the records of the
+    // steps after it, or the unused ones at the end, and take no part.  (Holding them
+    // to the last record is slower: 96 x 96 drape 324 -> 335 us a launch.)
     static_assert(STRAIN_GROUP == 4, "unrolled by hand");
     const int32_t* row_ptr = B.row_ptr + step0;
     StrainRec r[4];
     int pr[4], n[4];
-    // step u's record and pre-check byte: records [row, end), none past the last step
-    // (one past it is read then)
+    // step u's records and pre-check bytes: [row, end), none past the last step
     auto load = [&](int u, int row, int end) {
       n[u] = end - row;
-      const unsigned i = min(lane, max(end - row - 1, 0));
-      r[u] = (B.rec + row)[i];
-      pr[u] = k == 0 ? (B.pre + row)[i] : 0;
+      r[u] = (B.rec + row)[lane];
+      pr[u] = k == 0 ? (B.pre + row)[lane] : 0;
     };
 #pragma unroll
     for (int u = 0; u < 4; ++u) load(u, row_ptr[min(u, nstep)], row_ptr[min(u + 1, nstep)]);
