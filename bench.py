@@ -44,14 +44,15 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense BF16
 MLP_FWD_FLOP = 2 * (24 * 128 + 128 * 128 + 128 * 2)                    # 39,424
 MLP_TRAIN_FLOP = MLP_FWD_FLOP + 2 * (2 * 128 * 2 + 2 * 128 * 128 + 128 * 24)  # + backward
 ROOFLINE_NOTES = {
-    "strain": "one work-group runs about 2,900 dependent level iterations per step (the exact "
-              "Gauss-Seidel order; a second work-group on its XCD reads the next levels' records into "
-              "L2); bound by that chain's latency, not by HBM: it moves about 4.7e8 B "
-              "per launch (profiles/traffic_strain.json; mostly the prefetching work-group streaming the "
-              "records once) against the 1.6e8 B of reading every vertex and element once",
-    "traverse": "per-lane stackless walks, bound by dependent L2 misses; walks longer than 512 steps "
+    "strain": "one work-group per (sweep, band of the element order), about 4,090 dependent steps in "
+              "each sweep (the exact Gauss-Seidel order); bound by that chain's latency, not by HBM: it "
+              "moves about 3.4e9 B per launch (profiles/traffic_strain.json; the vertices that cross "
+              "bands and sweeps, through the coherence point) against the 1.6e8 B of reading every "
+              "vertex and element once",
+    "traverse": "per-lane stackless walks, bound by dependent L2 misses; walks longer than 128 steps "
                 "are continued over 64 sub-ranges by k_traverse_split (its time is included)",
-    "narrow": "gather of each sub-test's four vertices; FP64 VALU co-bound",
+    "narrow": "FP64 VALU; in incremental passes the chain of one sub-test (the pair's vertices are "
+              "gathered once, through LDS)",
 }
 FORMS = {"plain": {}, "mixed": {"precision": 1}, "learned": {"learned": 1},
          "learned_mixed": {"learned": 1, "precision": 1}}

@@ -21,7 +21,7 @@
 // Kernel time per time step, against all sweeps in one work-group (k_strain_pipe,
 // whose level iterations each scanned ten rows of marks, loaded 256 B records
 // and crossed two barriers): 64 x 64 cloth, every edge over the limit, 1.76 ->
-// 0.39 ms; 256 x 256 17.0 -> 1.2 ms (1.3e6 evaluations, 0.96 us a step, of which
+// 0.39 ms; 256 x 256 17.0 -> 1.15 ms (1.3e6 evaluations, 0.95 us a step, of which
 // 0.76 us evaluation); 1024 x 1024 cloth with 2,000 strings, few edges over the
 // limit, 8.2 -> 2.7 ms (0.17-0.37 us a step); 64 scenes 1.5 -> 0.52 ms.  The
 // pre-check replaces a packing and a check kernel (0.58 -> below 0.06 ms at 1024^2).

@@ -158,7 +158,9 @@ typedef struct cs_step_report {
     int32_t strain_edges;    /* edges over the limit in the last sweep */
     int32_t degenerate_edges;
     int32_t strain_levels;   /* schedule levels the strain sweeps went through (sum over
-                                the sweeps run; 0 when no edge was over the limit) */
+                                the sweeps run; 0 when no edge was over the limit; meshes
+                                without locality in their element order: level steps
+                                of the sweeps in flight together) */
     int64_t candidates;      /* sum over passes; -1 when a pass reports -1 */
     int64_t narrow_pairs;    /* sum over passes; -1 when a pass reports -1 */
     int64_t hit_pairs, hit_subtests;
