@@ -1229,7 +1229,8 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
     if (strain_plan_for(nv, ne, ev, ef, l0, nsched, plan, lev, nl)) {
       if (plan.n_levels >= (1 << 21))
         return fail(h, CS_ERR_UNSUPPORTED, "strain schedule above 2^21 levels");
-    } else {
+    }
+    if (plan.nband == 0 || strain_is_chain(nsched, nl)) {
       const int rc = build_pipe_schedule(h, nv, ne, ev, ef, l0, std::move(lev), nl, pipe);
       if (rc) return rc;
     }
@@ -1310,9 +1311,9 @@ int cs_assemble(cs_solver* h, const cs_mesh_view* m) {
   HIPCHK(h, dalloc(&S.zkey64, nv)); HIPCHK(h, dalloc(&S.zkey64_tmp, nv));
   HIPCHK(h, dalloc(&S.zval, nv)); HIPCHK(h, dalloc(&S.zval_tmp, nv));
   S.n_sched = nsched;
-  if (plan.nband > 0) {
-    HIPCHK(h, upload_plan(S, plan));
-  } else if (nsched > 0) {
+  if (plan.nband > 0) HIPCHK(h, upload_plan(S, plan));
+  if (pipe.n_levels > 0) {
+    S.bands.chain = plan.nband > 0;
     S.n_levels = pipe.n_levels;
     S.strain_delta = pipe.delta;
     HIPCHK(h, upload(&S.lvl_ptr, pipe.lptr));
@@ -1618,7 +1619,14 @@ int resolve_impl(cs_solver* h, cs_step_report* report, bool predict) {
   mark(h, &t_strain0);
   if (status == CS_OK || status == CS_WARN_ZONE_CAP) {
     launch_final_position(h->st, S, P.dom_lo, P.dom_hi, P.dt, P.friction);
-    HIPCHK(h, strain_limit(h->st, S, P.dt, P.max_strain_sweeps,
+    bool few = false;
+    if (S.bands.chain && P.max_strain_sweeps > 0) {
+      launch_strain_count(h->st, S, P.dt);
+      HIPCHK(h, hipGetLastError());
+      if ((rc = read_counters(h))) return rc;
+      few = strain_few(h->h_counters[CNT_STRAIN_OVER], S.n_sched, strain_in_flight(S) == 1);
+    }
+    HIPCHK(h, strain_limit(h->st, S, P.dt, P.max_strain_sweeps, few,
                            P.pass_timing >= 1 ? &strain_marks : nullptr));
     launch_final_velocity(h->st, S);
     launch_final_bodies(h->st, S, P.dt);  // updateFinalForRG

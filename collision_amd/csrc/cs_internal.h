@@ -55,6 +55,7 @@ enum {
   CNT_SNAP = 28,         // 28..31: pair/hit counts carried into the current pass
   CNT_PCAND64 = 32,      // 32, 33: static-box overlaps found by the swept-box traversal
   CNT_PPAIRS = 34,       // pairs of that traversal whose static boxes overlap
+  CNT_STRAIN_OVER = 37,  // chains: elements over the limit before the sweeps
   CNT_STRAIN_PROG = 35,  // strain sweep: level iteration reached (-1: done), read by its prefetcher
   CNT_INTS = 40
 };
@@ -144,6 +145,7 @@ constexpr int SB_STAT_INTS = 32;
 struct StrainBands {
   int nband = 0, n_levels = 0, cap = 0;
   int64_t steps = 0;        // of one sweep, all bands together
+  bool chain = false;       // the fields of k_strain_pipe are there too: either may sweep
   // device clock ticks after which a wait gives up, and the most that count
   // between two looks at the clock
   long long wait_ticks = 0, look_ticks = 0;
@@ -452,12 +454,17 @@ void launch_final_position(hipStream_t st, DevState& S, const double lo[3], cons
                            double dt, double mu);
 // marks != nullptr: a pair of events around every k_strain_pipe launch is
 // appended (the caller reads and destroys them)
-hipError_t strain_limit(hipStream_t st, DevState& S, double dt, int max_sweeps,
+// few: a chain with few elements over the limit (strain_few)
+hipError_t strain_limit(hipStream_t st, DevState& S, double dt, int max_sweeps, bool few,
                         std::vector<hipEvent_t>* marks);
 // cs_strain.hip: the same by bands (S.bands.nband > 0)
 hipError_t strain_bands_setup(DevState& S);
 hipError_t strain_limit_bands(hipStream_t st, DevState& S, double dt, int max_sweeps,
                               std::vector<hipEvent_t>* marks);
+// the elements over the limit, into CNT_STRAIN_OVER
+void launch_strain_count(hipStream_t st, DevState& S, double dt);
+// sweeps of k_strain_pipe in flight
+int strain_in_flight(const DevState& S);
 // cs_schedule.hip (host); lev, L: the elements' levels and their number (strain_levels)
 void build_strain_schedule(int nv, int ne, const int4* ev, const uint8_t* ef, std::vector<int> lev,
                            int L, std::vector<int>& level, int& n_levels, int& delta);

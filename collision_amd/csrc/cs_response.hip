@@ -896,6 +896,7 @@ constexpr int SP_KMAX = 10;            // sweeps in flight
 constexpr int SP_LP_MAX = 8192;        // levels whose slot offsets are kept in LDS
 constexpr int SP_PRE_LEVELS = 65536;   // levels whose pre-check bits are kept in LDS
 static_assert(STRAIN_LEVEL_CAP % 4 == 0 && STRAIN_LEVEL_CAP <= 1024, "work entry layout");
+static_assert(STRAIN_SKIP_LEVELS == SP_PRE_LEVELS, "levels that can be skipped");
 
 __device__ inline bool bit_get(const uint32_t* b, int i) { return (b[i >> 5] >> (i & 31)) & 1u; }
 __device__ inline void bit_set(uint32_t* b, int i) { atomicOr(&b[i >> 5], 1u << (i & 31)); }
@@ -1282,13 +1283,15 @@ __global__ void __launch_bounds__(SP_THREADS)
   }
 }
 
-hipError_t strain_limit(hipStream_t st, DevState& S, double dt, int max_sweeps,
+// marks pending at one time cover K * delta - 1 levels
+int strain_in_flight(const DevState& S) { return std::max(1, SP_RING / std::max(1, S.strain_delta)); }
+
+hipError_t strain_limit(hipStream_t st, DevState& S, double dt, int max_sweeps, bool few,
                         std::vector<hipEvent_t>* marks) {
   const int n = S.n_sched;
   if (S.ne == 0 || n == 0 || max_sweeps <= 0) return hipSuccess;
-  if (S.bands.nband > 0) return strain_limit_bands(st, S, dt, max_sweeps, marks);
-  // sweeps in flight: marks pending at one time cover K * delta - 1 levels
-  const int kfit = std::max(1, SP_RING / std::max(1, S.strain_delta));
+  if (S.bands.nband > 0 && !few) return strain_limit_bands(st, S, dt, max_sweeps, marks);
+  const int kfit = strain_in_flight(S);
   for (int k0 = 0; k0 < max_sweeps;) {
     const int K = std::min({SP_KMAX, kfit, max_sweeps - k0});
     hipLaunchKernelGGL(k_strain_pack, dim3((n + 255) / 256), dim3(256), 0, st, S.sslot, S.x_old,

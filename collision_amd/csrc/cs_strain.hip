@@ -130,14 +130,14 @@ __device__ inline void end_position(const double* o, const double* a, double dt,
 // Pre-check with the velocities at the start of the launch, in element order
 // (neighbouring elements share the gathered vertices): the byte of every
 // element's slot, and the any-edge flag.  Also resets the tasks' progress and
-// statistics.
+// statistics.  count: the elements over the limit are counted (CNT_STRAIN_OVER).
 __global__ void __launch_bounds__(256)
     k_strain_precheck(const int4* __restrict__ ev, const dvec4* __restrict__ len0,
                       const int32_t* __restrict__ slot, const dvec4* __restrict__ x_old,
                       const dvec4* __restrict__ av, double dt, int ne, uint8_t* __restrict__ pre,
                       int* __restrict__ prog, int ntask, int nband,
                       const int32_t* __restrict__ step_ptr, const int32_t* __restrict__ step_level,
-                      int* __restrict__ stat, int* __restrict__ counters) {
+                      int* __restrict__ stat, int* __restrict__ counters, int count) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   // (a task has nothing to do below its band's first level)
   for (int i = e; i < ntask; i += gridDim.x * blockDim.x)
@@ -172,8 +172,20 @@ __global__ void __launch_bounds__(256)
       pre[s] = any ? 1 : 0;
     }
   }
-  if (__any(any) && (threadIdx.x & 63) == 0) atomicOr(&counters[CNT_STRAIN_FLAG], 1);
+  const uint64_t over = __ballot(any);
+  if (over && (threadIdx.x & 63) == 0) {
+    atomicOr(&counters[CNT_STRAIN_FLAG], 1);
+    if (count) atomicAdd(&counters[CNT_STRAIN_OVER], __popcll(over));
+  }
 }
+
+static void launch_precheck(hipStream_t st, DevState& S, double dt, int count) {
+  const StrainBands& B = S.bands;
+  hipLaunchKernelGGL(k_strain_precheck, dim3((S.ne + 255) / 256), dim3(256), 0, st, S.ev, S.len0,
+                     B.slot, S.x_old, S.av, dt, S.ne, B.pre, B.prog, SB_MAX_SWEEPS * B.nband,
+                     B.nband, B.step_ptr, B.step_level, B.stat, S.counters, count);
+}
+void launch_strain_count(hipStream_t st, DevState& S, double dt) { launch_precheck(st, S, dt, 1); }
 
 __global__ void __launch_bounds__(SB_THREADS)
     k_strain_bands(StrainBands B, const dvec4* __restrict__ x_old, dvec4* av, double dt, int K,
@@ -520,9 +532,7 @@ hipError_t strain_limit_bands(hipStream_t st, DevState& S, double dt, int max_sw
   const StrainBands& B = S.bands;
   for (int k0 = 0; k0 < max_sweeps;) {
     const int K = std::min(SB_MAX_SWEEPS, max_sweeps - k0);
-    hipLaunchKernelGGL(k_strain_precheck, dim3((S.ne + 255) / 256), dim3(256), 0, st, S.ev, S.len0,
-                       B.slot, S.x_old, S.av, dt, S.ne, B.pre, B.prog, SB_MAX_SWEEPS * B.nband,
-                       B.nband, B.step_ptr, B.step_level, B.stat, S.counters);
+    launch_precheck(st, S, dt, 0);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (marks && hipEventCreate(&e0) == hipSuccess && hipEventCreate(&e1) == hipSuccess)
       (void)hipEventRecord(e0, st);

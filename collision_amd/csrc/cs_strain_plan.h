@@ -194,13 +194,34 @@ inline int strain_band_count(int64_t nsched, int n_levels) {
 //   2.9      128 x 128, shuffled tiles of 4       4.8 / 1.2     4.8 / 0.28
 //   3.7      128 x 128, shuffled within 4,096     1.42 / 1.02   1.38 / 0.28
 //   5.7      160 x 160 in random order            11.2 / 1.4    11.2 / 0.31
-// (One string of 30,000 bonds: 24 / 97 and 7.5 / 4.4; a closed one 110 / 362 and
-// 65 / 50: there the idle steps of the bands cost more than skipped levels.)
 // A sweep of few steps cannot cost much in bands, and a mesh with every edge over the
 // limit gains: 24 x 24 in random order (44 steps) 0.34 / 0.22 and 0.32 / 0.14, but
 // the whole step of one with every edge over it 0.59 / 1.00 ms.
 inline bool strain_plan_pays(const StrainPlan& P) {
   return 10 * (int64_t)P.imp.size() <= 24 * P.nvert || P.steps() <= 64;
+}
+
+// Chains: long schedules with few elements on a level (single strings, strips).
+// The bands' steps are made whether or not an element is evaluated, 0.25 us each,
+// while the one-work-group sweep goes to the levels with something to do, at some 4 us
+// an iteration.  With most bonds over the limit the bands are four times faster, with
+// two of 30,000 eight times slower; so a chain is laid out for both, and the number of
+// elements over the limit before the sweeps decides at every step (one host wait more,
+// 10 us).  Whole step in us, one work-group / bands, by moved points (one puts one
+// or two bonds over the limit):
+//   open string of 1,000     5: 188 / 401       50: 777 / 443
+//   open, 30,000             2: 403 / 6,520     150: 1,580 / 6,690   1,500: 13,100 / 8,000
+//   closed, 1,000            2: 1,040 / 2,210   50: 4,590 / 2,340
+//   closed, 30,000           2: 27,100 / 59,900 150: 101,000 / 59,600
+// The sweeps of a closed string follow each other one by one (one in flight), so an
+// element costs more there.  Up to 512 levels the difference is below the wait; above
+// 65,536 the one-work-group sweep cannot skip.
+constexpr int STRAIN_CHAIN_LEVELS = 512, STRAIN_SKIP_LEVELS = 65536;
+inline bool strain_is_chain(int64_t nsched, int n_levels) {
+  return n_levels > STRAIN_CHAIN_LEVELS && n_levels <= STRAIN_SKIP_LEVELS && nsched <= 8ll * n_levels;
+}
+inline bool strain_few(int64_t over, int64_t nsched, bool one_in_flight) {
+  return over > 0 && over * (one_in_flight ? 256 : 64) < nsched;
 }
 
 // Microseconds after which a wait of a task means that the plan is broken.  A
